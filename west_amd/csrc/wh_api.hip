@@ -8,6 +8,7 @@
 
 #include "../../include/west_hip.h"
 #include "wh_context.h"
+#include "wh_fft_rect.h"
 #include "wh_fft_tpl.h"
 #include "wh_fft_reg.h"
 #include "wh_gemm.h"
@@ -1047,7 +1048,16 @@ int wh_set_potential(const double* vrs) {
   WH_REQUIRE(c.have_grid, "wh_set_grid first");
   if (c.d_vrs) WH_HIP(hipFree(c.d_vrs));
   WH_HIP(hipMalloc(&c.d_vrs, sizeof(double) * c.nnr));
-  WH_HIP(hipMemcpy(c.d_vrs, vrs, sizeof(double) * c.nnr, hipMemcpyDefault));
+  if (c.plan.transposed_grid()) {   // the plane kernels of this grid read [a3][a1][a2]
+    // staged in the perturbations' buffer
+    double* in = c.w_dvr.as<double>(c.nnr);
+    WH_HIP(hipMemcpy(in, vrs, sizeof(double) * c.nnr, hipMemcpyDefault));
+    wait_for_caller(c);   // a device source's copy is ordered on the null stream only
+    rect_transpose_grid(c.nr1, c.nr2, c.nr3, in, c.d_vrs, c.stream);
+    WH_HIP(hipStreamSynchronize(c.stream));
+  } else {
+    WH_HIP(hipMemcpy(c.d_vrs, vrs, sizeof(double) * c.nnr, hipMemcpyDefault));
+  }
   c.have_pot = true;
   c.mixed_valid = false;
   return 0;

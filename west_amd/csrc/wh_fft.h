@@ -60,9 +60,24 @@ constexpr int kZregCols = 128;
 struct TplKernels;
 struct TplKernels32;
 
+// Run-time shape of the plane kernels of wh_fft_rect.hip
+struct RectPlan {
+  bool ok = false;
+  int r10 = 0, r11 = 0, r20 = 0, r21 = 0;   // n1 = r10 r11, n2 = r20 r21
+  int nt = 256;    // threads per workgroup (256 or 512)
+  int pz = 1;      // planes per workgroup
+  int nj = 1;      // a1 lines per chunk
+  int nrc = 1;     // rows per chunk of the a2 passes
+  int rs2 = 0;     // row stride (odd)
+  int xs = 0;      // a1 line stride (odd)
+  float inv_n2 = 0.f;
+};
+
 struct StickPlan {
   StickPlanDev dev{};
-  const TplKernels* tpl = nullptr;   // size-specialised kernels for this grid, if compiled
+  const TplKernels* tpl = nullptr;   // size-specialised plane kernels (n1 = n2 compiled), if any
+  const TplKernels* tplz = nullptr;  // size-specialised z kernels (n3 compiled), if any
+  RectPlan rect;                     // two-pass plane kernels for the grids without tpl
   const TplKernels32* tpl32 = nullptr;   // FP32 operator kernels for this grid, if compiled
   // workgroups per CU the size-specialised plane kernel's LDS is sized for
   // (FP64 / FP32 operator); 0 until timed on the first large launch
@@ -75,6 +90,8 @@ struct StickPlan {
   void build(int nr1, int nr2, int nr3, int npw, const int* nl_1based, const int* nlm_1based);
   void release();
   long sticks_elems() const { return static_cast<long>(dev.n3) * dev.nct; }
+  // real-space arrays of the plane kernels are [a3][a1][a2] (else [a3][a2][a1])
+  bool transposed_grid() const { return !tpl && rect.ok; }
 };
 
 // Variant of the plane kernel for a launch of nitems items: a fixed choice

@@ -18,6 +18,7 @@
 #include <mutex>
 
 #include "wh_fft.h"
+#include "wh_fft_rect.h"
 #include "wh_fft_reg.h"
 #include "wh_fft_q4.h"
 #include "wh_fft_tpl.h"
@@ -673,8 +674,13 @@ void StickPlan::build(int nr1, int nr2, int nr3, int npw, const int* nl, const i
   pick_maxe(static_cast<long>(2 * kCPW) * nr3);
   // kernels specialised on the grid size, unless WH_FFT_GENERIC is set
   const char* gen = std::getenv("WH_FFT_GENERIC");
-  tpl = (gen && gen[0] == '1') ? nullptr : tpl_kernels_f64(dev);
+  const bool generic = gen && gen[0] == '1';
+  tpl = generic ? nullptr : tpl_kernels_f64(dev);
+  tplz = generic ? nullptr : tpl_z_kernels_f64(dev);
   tpl32 = tpl_kernels_f32(dev);
+  // (a grid of the FP32 operator keeps the layout that its kernels read)
+  rect = RectPlan{};
+  if (!tpl && !tpl32) rect_plan(dev, rect);
   // plane-kernel variant: WH_PLANE_OCC (1..9) fixes it, else timed on the first large launch
   const char* occ_env = std::getenv("WH_PLANE_OCC");
   const int occ = (occ_env && occ_env[0] >= '1' && occ_env[0] <= '9') ? occ_env[0] - '0' : 0;
@@ -686,8 +692,8 @@ void launch_zinv(const StickPlan& p, const FftItem* d_items, int nitems, const z
                  const z64* psiB, long ldB, z64* sticks, int mode, hipStream_t s) {
   if (nitems <= 0) return;
   const StickPlanDev& P = p.dev;
-  if (p.tpl) {
-    p.tpl->zinv(P, d_items, nitems, psiA, ldA, psiB, ldB, sticks, mode, s);
+  if (p.tplz) {
+    p.tplz->zinv(P, d_items, nitems, psiA, ldA, psiB, ldB, sticks, mode, s);
     WH_HIP(hipGetLastError());
     return;
   }
@@ -746,6 +752,7 @@ void launch_plane_vloc(const StickPlan& p, const FftItem* d_items, int nitems, c
     WH_HIP(hipGetLastError());
     return;
   }
+  if (p.rect.ok) return rect_plane_vloc(P, p.rect, d_items, nitems, sin, sout, vpot, ldpot, scale, s);
   const int njc = plane_njc(P);
   const int maxe = pick_maxe(std::max<long>(static_cast<long>(P.nrows) * P.n2, static_cast<long>(njc) * P.n1));
   const size_t smem = plane_smem_bytes(P, njc, false);
@@ -763,6 +770,7 @@ void launch_plane_to_real(const StickPlan& p, const FftItem* d_items, int nitems
     WH_HIP(hipGetLastError());
     return;
   }
+  if (p.rect.ok) return rect_plane_to_real(P, p.rect, d_items, nitems, sin, out, ldout, s);
   const int njc = plane_njc(P);
   const int maxe = pick_maxe(std::max<long>(static_cast<long>(P.nrows) * P.n2, static_cast<long>(njc) * P.n1));
   const size_t smem = plane_smem_bytes(P, njc, false);
@@ -772,7 +780,7 @@ void launch_plane_to_real(const StickPlan& p, const FftItem* d_items, int nitems
 }
 
 long plane_density_scratch(const StickPlan& p) {
-  return (p.tpl && p.tpl->density_scratch > 0) ? p.tpl->density_scratch : 0;
+  return (p.tpl && p.tpl->density_scratch > 0) ? p.tpl->density_scratch * p.dev.n3 : 0;
 }
 
 void launch_plane_density(const StickPlan& p, int npert, int nband, const z64* sin, const double* occ,
@@ -784,6 +792,7 @@ void launch_plane_density(const StickPlan& p, int npert, int nband, const z64* s
     WH_HIP(hipGetLastError());
     return;
   }
+  if (p.rect.ok) return rect_plane_density(P, p.rect, npert, nband, sin, occ, sout, s);
   const int njc = plane_njc(P);
   const int maxe = pick_maxe(std::max<long>(static_cast<long>(P.nrows) * P.n2, static_cast<long>(njc) * P.n1));
   const size_t smem = plane_smem_bytes(P, njc, true);
@@ -797,8 +806,8 @@ void launch_zfwd(const StickPlan& p, const FftItem* d_items, int nitems, const z
                  long ldin, z64* out, long ldout, const ZfwdArgs& args, hipStream_t s) {
   if (nitems <= 0) return;
   const StickPlanDev& P = p.dev;
-  if (p.tpl) {
-    p.tpl->zfwd(P, d_items, nitems, sticks, in, ldin, out, ldout, args, s);
+  if (p.tplz) {
+    p.tplz->zfwd(P, d_items, nitems, sticks, in, ldin, out, ldout, args, s);
     WH_HIP(hipGetLastError());
     return;
   }

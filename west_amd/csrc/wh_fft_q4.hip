@@ -108,10 +108,10 @@ __global__ __launch_bounds__(NTQ) __attribute__((amdgpu_waves_per_eu(WPE))) void
   const int r0 = IMX - P.imax;
   const int nct = P.nct;
   const int z0 = blockIdx.x * PZ;
-  const int nz = min(PZ, N - z0);
+  const int nz = min(PZ, P.n3 - z0);
   const FftItem item = items[blockIdx.y];
   if (item.a < 0) return;   // inactive item (uniform per workgroup)
-  const long sl = static_cast<long>(N) * nct;
+  const long sl = static_cast<long>(P.n3) * nct;
   const int tid = threadIdx.x;
   const int l = tid & 3;
   const int quad = tid >> 2;
@@ -264,7 +264,7 @@ void launch_q4(const StickPlanDev& P, const FftItem* it, int n, const z64* si, z
       set = true;
     }
   }
-  k_plane_vloc_q4<N, IMX, PZ, NTQ, WPE><<<dim3(ceil_div(N, PZ), n), NTQ, sm, s>>>(P, it, si, so, v, ldv, scale);
+  k_plane_vloc_q4<N, IMX, PZ, NTQ, WPE><<<dim3(ceil_div(P.n3, PZ), n), NTQ, sm, s>>>(P, it, si, so, v, ldv, scale);
 }
 
 // variants (sphere bound, planes per workgroup, threads): 0: (18, 3, 768),
@@ -278,7 +278,7 @@ bool q4_tight(const StickPlanDev& P) { return P.imax <= 16 && P.jext <= 16; }
 }  // namespace
 
 int plane_q4_variants(const StickPlanDev& P) {
-  if (P.n1 != P.n2 || P.n1 != P.n3) return 0;
+  if (P.n1 != P.n2) return 0;
   if (P.n1 != 72 && P.n1 != 60 && P.n1 != 100) return 0;
   // the a1 and a2 transforms take |i| and |j| beyond N/4 as known zeros
   const int imx = (P.n1 + 3) / 4;

@@ -7,8 +7,8 @@
 namespace wh {
 
 // Number of register-line plane variants for this plan in FP32 (fp32) or
-// FP64 (0: the grid is not cubic of a compiled size -- FP64 lines stop at 64
-// points -- or its sphere is too wide for them).
+// FP64 (0: n1 = n2 is not a compiled size -- FP64 lines stop at 64 points; in FP32
+// the grid is not cubic -- or its sphere is too wide for them).
 int plane_reg_variants(const StickPlanDev& P, bool fp32);
 
 // Variant v (0 <= v < plane_reg_variants(P, true)) of the FP32 plane step

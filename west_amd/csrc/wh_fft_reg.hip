@@ -62,10 +62,10 @@ __global__ __launch_bounds__((nt_reg<N, PZ>())) __attribute__((amdgpu_waves_per_
   const int r0 = IMX - P.imax;   // first row of the sphere
   const int nct = P.nct;
   const int z0 = blockIdx.x * PZ;
-  const int nz = min(PZ, N - z0);
+  const int nz = min(PZ, P.n3 - z0);
   const FftItem item = items[blockIdx.y];
   if (item.a < 0) return;   // inactive item (uniform per workgroup)
-  const long sl = static_cast<long>(N) * nct;
+  const long sl = static_cast<long>(P.n3) * nct;
   const int tid = threadIdx.x;
 
   // sticks of planes z0 .. z0 + nz - 1 (contiguous) into zeroed rows
@@ -190,7 +190,7 @@ void launch_pz(const StickPlanDev& P, const FftItem* it, int n, const cplx<T>* s
                double scale, hipStream_t s) {
   const size_t sm = reg_smem(P, PZ, sizeof(cplx<T>));
   allow_smem_reg(k_plane_vloc_reg<T, N, PT, PZ>, sm);
-  k_plane_vloc_reg<T, N, PT, PZ><<<dim3(ceil_div(N, PZ), n), nt_reg<N, PZ>(), sm, s>>>(P, it, si, so, v, ldv, scale);
+  k_plane_vloc_reg<T, N, PT, PZ><<<dim3(ceil_div(P.n3, PZ), n), nt_reg<N, PZ>(), sm, s>>>(P, it, si, so, v, ldv, scale);
 }
 
 template <typename T, int N, typename PT>
@@ -502,7 +502,7 @@ void zfwd_reg(const StickPlanDev& P, const FftItem* items, int n, const z32* sti
 }
 
 int plane_reg_variants(const StickPlanDev& P, bool fp32) {
-  if (P.n1 != P.n2 || P.n1 != P.n3 || !compiled(P.n1, fp32)) return 0;
+  if (P.n1 != P.n2 || (fp32 && P.n1 != P.n3) || !compiled(P.n1, fp32)) return 0;
   // the a1 and a2 transforms take |i| and |j| beyond N/4 as known zeros
   if (P.imax > (P.n1 + 3) / 4 || P.jext > (P.n2 + 3) / 4) return 0;
   const size_t elem = fp32 ? sizeof(z32) : sizeof(z64);

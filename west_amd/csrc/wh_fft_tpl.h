@@ -1,4 +1,4 @@
-// Compile-time-size FFT kernels for cubic grids (declarations).
+// Compile-time-size FFT kernels (declarations).
 #pragma once
 
 #include "wh_fft.h"
@@ -14,9 +14,9 @@ struct TplKernels {
                hipStream_t);
   void (*to_real)(const StickPlanDev&, const FftItem*, int, const void*, double*, long, hipStream_t);
   // density(P, npert, nband, sticks in, occ, sticks out, scratch, stream): scratch holds
-  // density_scratch reals per perturbation (may be null when that is 0)
+  // density_scratch n3 reals per perturbation (may be null when that is 0)
   void (*density)(const StickPlanDev&, int, int, const void*, const double*, void*, void*, hipStream_t);
-  long density_scratch;   // 0: none needed; -1: this grid has no density kernel
+  long density_scratch;   // per plane; 0: none needed; -1: this grid has no density kernel
   int max_occ;
 };
 
@@ -30,9 +30,11 @@ struct TplKernels32 {
   int max_occ;
 };
 
-// kernels specialised on N = nr1 = nr2 = nr3, or null when the grid is not
-// one of the compiled sizes (the runtime-size kernels are used then)
+// FP64: plane kernels specialised on N = nr1 = nr2 (any nr3) and z kernels on
+// N = nr3, or null when that length is not one of the compiled sizes (the
+// runtime-size kernels are used then); FP32: cubic grids only
 const TplKernels* tpl_kernels_f64(const StickPlanDev& P);
+const TplKernels* tpl_z_kernels_f64(const StickPlanDev& P);
 const TplKernels32* tpl_kernels_f32(const StickPlanDev& P);
 
 }  // namespace wh

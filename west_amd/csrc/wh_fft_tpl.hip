@@ -1,7 +1,8 @@
-// Gamma-point FFT kernels with compile-time line length (cubic grids).
+// Gamma-point FFT kernels with compile-time line length.
 //
 // Same algorithm and data layout as the runtime-size kernels of wh_fft.hip
-// (stick layout, zinv -> plane -> zfwd), specialised on N = nr1 = nr2 = nr3:
+// (stick layout, zinv -> plane -> zfwd), specialised on
+// N = nr1 = nr2 (plane kernels, any nr3) and N = nr3 (z kernels):
 //  * each 1D transform is a Stockham sequence of large radices chosen at
 //    compile time (N = 72 = 9 x 8: two LDS passes instead of four), with
 //    composite radices 6, 8, 9, 10, 12 done in registers as two-level
@@ -442,7 +443,7 @@ __global__ __launch_bounds__(NTP) __attribute__((amdgpu_waves_per_eu(2 * OCC))) 
   const int it = blockIdx.y;
   const FftItem item = items[it];
   if (item.a < 0) return;   // inactive item (uniform per workgroup)
-  const long sl = static_cast<long>(N) * P.nct;
+  const long sl = static_cast<long>(P.n3) * P.nct;
   const int imax = P.imax;
   load_tw<T, N>(S.tw, P.tw1);
   plane_fill<T, N>(P, S, sin + static_cast<long>(item.a) * sl + static_cast<long>(z) * P.nct);
@@ -494,7 +495,7 @@ __global__ __launch_bounds__(NTP) void k_plane_to_real_t(StickPlanDev P, const F
   const int it = blockIdx.y;
   const FftItem item = items[it];
   if (item.a < 0) return;   // inactive item (uniform per workgroup)
-  const long sl = static_cast<long>(N) * P.nct;
+  const long sl = static_cast<long>(P.n3) * P.nct;
   const int imax = P.imax;
   load_tw<T, N>(S.tw, P.tw1);
   plane_fill<T, N>(P, S, sin + static_cast<long>(it) * sl + static_cast<long>(z) * P.nct);
@@ -525,7 +526,7 @@ __global__ __launch_bounds__(NTP) void k_plane_density_t(StickPlanDev P, int nba
   T* acc = reinterpret_cast<T*>(S.x + JC * N);
   const int z = blockIdx.x;
   const int p = blockIdx.y;
-  const long sl = static_cast<long>(N) * P.nct;
+  const long sl = static_cast<long>(P.n3) * P.nct;
   const int imax = P.imax;
   load_tw<T, N>(S.tw, P.tw1);
   for (int t = threadIdx.x; t < N * N; t += NTP) acc[t] = T(0);
@@ -604,10 +605,10 @@ __global__ __launch_bounds__(NTP) void k_plane_density_big_t(StickPlanDev P, int
   T* acc = reinterpret_cast<T*>(S.x + JC * N);
   const int z = blockIdx.x;
   const int p = blockIdx.y;
-  const long sl = static_cast<long>(N) * P.nct;
+  const long sl = static_cast<long>(P.n3) * P.nct;
   const int imax = P.imax;
   load_tw<T, N>(S.tw, P.tw1);
-  T* park = scratch + (static_cast<long>(p) * N + z) * N * H;   // [j][x < H]
+  T* park = scratch + (static_cast<long>(p) * P.n3 + z) * N * H;   // [j][x < H]
   cplx<T>* pl = S.pl;
   for (int h = 0; h < 2; ++h) {
     for (int t = threadIdx.x; t < N * H; t += NTP) acc[t] = T(0);
@@ -689,7 +690,7 @@ void vloc_occ(const StickPlanDev& P, const FftItem* it, int n, const void* si, v
   constexpr size_t sm = vloc_smem<T, N, OCC>();
   static_assert(sm <= 160u * 1024u, "plane kernel exceeds LDS");
   allow_smem(k_plane_vloc_t<T, N, PT, OCC>, sm);
-  k_plane_vloc_t<T, N, PT, OCC><<<dim3(N, n), NTP, sm, s>>>(P, it, static_cast<const cplx<T>*>(si),
+  k_plane_vloc_t<T, N, PT, OCC><<<dim3(P.n3, n), NTP, sm, s>>>(P, it, static_cast<const cplx<T>*>(si),
                                                             static_cast<cplx<T>*>(so), v, ldv, scale);
 }
 
@@ -730,14 +731,14 @@ struct Launch {
                       hipStream_t s) {
     const size_t sm = plane_smem<T, N>(false);
     allow_smem(k_plane_to_real_t<T, N>, sm);
-    k_plane_to_real_t<T, N><<<dim3(N, n), NTP, sm, s>>>(P, it, static_cast<const cplx<T>*>(si), out, ldout);
+    k_plane_to_real_t<T, N><<<dim3(P.n3, n), NTP, sm, s>>>(P, it, static_cast<const cplx<T>*>(si), out, ldout);
   }
   static void density(const StickPlanDev& P, int np, int nb, const void* si, const double* occ, void* so,
                       void* scratch, hipStream_t s) {
     if constexpr (density_fits_lds<T, N>()) {
       const size_t sm = plane_smem<T, N>(true);
       allow_smem(k_plane_density_t<T, N>, sm);
-      k_plane_density_t<T, N><<<dim3(N, np), NTP, sm, s>>>(P, nb, static_cast<const cplx<T>*>(si), occ,
+      k_plane_density_t<T, N><<<dim3(P.n3, np), NTP, sm, s>>>(P, nb, static_cast<const cplx<T>*>(si), occ,
                                                           static_cast<cplx<T>*>(so));
       return;
     }
@@ -746,7 +747,7 @@ struct Launch {
       constexpr size_t smb = big_density_smem<T, N>();
       static_assert(smb <= 160u * 1024u, "big density kernel exceeds LDS");
       allow_smem(k_plane_density_big_t<T, N>, smb);
-      k_plane_density_big_t<T, N><<<dim3(N, np), NTP, smb, s>>>(P, nb, static_cast<const cplx<T>*>(si), occ,
+      k_plane_density_big_t<T, N><<<dim3(P.n3, np), NTP, smb, s>>>(P, nb, static_cast<const cplx<T>*>(si), occ,
                                                                static_cast<cplx<T>*>(so), static_cast<T*>(scratch));
     } else {
       WH_REQUIRE(false, "response-density plane does not fit in LDS for this grid");
@@ -773,14 +774,14 @@ struct Launch32 {
   }
 };
 
-// scratch reals per perturbation the density launcher needs (0: the plane fits in LDS;
+// scratch reals per perturbation and plane the density launcher needs (0: the plane fits in LDS;
 // -1: no kernel for this size)
 template <typename T, int N>
 long density_scratch() {
   if constexpr (density_fits_lds<T, N>()) {
     return 0;
   } else if constexpr (N % 2 == 0 && xh_chunk<T, N>() >= 1) {
-    return static_cast<long>(N) * N * (N / 2);
+    return static_cast<long>(N) * (N / 2);
   } else {
     return -1;
   }
@@ -864,9 +865,11 @@ const TplKernels32* tpl_kernels_f32(const StickPlanDev& P) {
 }
 
 const TplKernels* tpl_kernels_f64(const StickPlanDev& P) {
-  if (P.n1 != P.n2 || P.n2 != P.n3) return nullptr;
+  if (P.n1 != P.n2) return nullptr;
   if (P.nrows > P.n1 / 2 + 2) return nullptr;
   return table_for<double>(P.n1);
 }
+
+const TplKernels* tpl_z_kernels_f64(const StickPlanDev& P) { return table_for<double>(P.n3); }
 
 }  // namespace wh
