@@ -1,0 +1,98 @@
+"""The q-point path on grids beyond the LDS (stick transforms, one CG over the
+columns of every k point) against the oracle: the operator and the CG at each
+k point, chi0(q) with all k points in one solve and one after another, and a
+grid whose planes take the two-radix kernels or the compiled ones."""
+import numpy as np
+import pytest
+
+from west_amd.kpoint import make_h2_crystal, make_k_ground_state
+
+pytestmark = pytest.mark.gpu
+
+
+def _rel(a, b):
+    return float(np.abs(a - b).max() / np.abs(b).max())
+
+
+def _smooth(n, npwx, m, g2, seed):
+    rng = np.random.default_rng(seed)
+    a = np.zeros((m, npwx), complex)
+    a[:, :n] = (rng.normal(size=(m, n)) + 1j * rng.normal(size=(m, n))) / (1.0 + g2[None, :n])
+    return a
+
+
+# (30, 25, 27): n1 != n2; (27, 20, 20): an odd length; (25, 25, 30) n1 = n2 not
+# compiled; (30, 30, 18): n1 = n2 compiled
+CASES = {"n30x25x27": ((9.0, 7.8, 8.4), (2, 1, 1)), "n27x20x20": ((8.4, 5.9, 5.9), (3, 1, 1)),
+         "n25x25x30": ((7.8, 7.8, 9.0), (1, 2, 1)), "n30x30x18": ((9.0, 9.0, 5.3), (1, 1, 2))}
+
+
+@pytest.fixture(scope="module", params=list(CASES), ids=list(CASES))
+def ksys(gpu, request):
+    cell, nk = CASES[request.param]
+    print(f"case {request.param}: ground state", flush=True)
+    at = np.diag(cell) + np.array([[0, 0.1, 0.2], [0, 0, 0.1], [0, 0, 0]])
+    kgs = make_k_ground_state(make_h2_crystal(25.0, cell=at), nk, nbnd=4)
+    assert "n" + "x".join(str(n) for n in kgs.nr) == request.param
+    h = gpu.system_create()
+    gpu.system_select(h)
+    gpu.set_k_ground_state(kgs)
+    yield kgs
+    gpu.system_select(0)
+    gpu.system_destroy(h)
+
+
+# tolerances as in test_gpu_kpoint.py: FP64 operator 1e-12, converged solves 1e-9
+def test_operator_at_k(gpu, ksys):
+    from oracle import kpoint as K
+    for ik in range(ksys.nks):
+        v = K.KView(ksys, ik)
+        for m in (1, 5):
+            psi = _smooth(v.basis.npw, ksys.npwx, m, v.basis.g2kin, 10 + ik)
+            e = np.linspace(-0.6, 0.1, m)
+            gpu.set_current_k(ik + 1)
+            out = gpu.apply_sternheimerop_to_m_wfcs(ksys.nbndval, psi, e, ksys.alpha_pv)
+            assert _rel(out, K.apply_sternheimerop_k(v, psi, e, ksys.alpha_pv)) < 1e-12
+
+
+def test_linsolve_at_k(gpu, ksys):
+    from oracle import kpoint as K
+    from oracle.linsolve import linsolve_sternheimer_m_wfcts
+    v = K.KView(ksys, ksys.nks - 1)
+    m, nb = 3, ksys.nbndval
+    b = _smooth(v.basis.npw, ksys.npwx, m, v.basis.g2kin, 3)
+    e = np.full(m, float(v.et[:nb].min()) - 0.3)
+    ep = K.set_eprec_k(v, v.evc[:1]).repeat(m)
+    x0 = K.precondition_k(v, b, ep)
+    xr, br = x0.copy(), b.copy()
+    linsolve_sternheimer_m_wfcts(v, nb, br, xr, e, ep, 1e-22, 250, None)
+    gpu.set_current_k(ksys.nks)
+    x = x0.copy()
+    assert gpu.linsolve_sternheimer_m_wfcts(nb, m, b.copy(), x, e, ep, 1e-22) == 0
+    assert _rel(x, xr) < 1e-9
+
+
+@pytest.mark.parametrize("kbatch", ["1", "0"])
+def test_dfpt_at_q(gpu, ksys, kbatch, monkeypatch):
+    from oracle import kpoint as K
+    monkeypatch.setenv("WH_KBATCH", kbatch)
+    for iq in range(len(ksys.qpts)):
+        qb = ksys.qpts[iq].basis
+        dv = _smooth(qb.npw, ksys.npwqx, 3, qb.g2kin, 40 + iq)
+        for tr2, tol in ((-1.0, 1e-12), (1e-22, 1e-9)):
+            out, ierr = gpu.dfpt(3, dv, tr2, iq=iq + 1, return_ierr=True)
+            assert not ierr.any()
+            assert _rel(out, K.dfpt_q(ksys, iq, dv, tr2)) < tol
+
+
+def test_iteration_limit_counts_unconverged(gpu, ksys):
+    """n_dfpt_maxiter = 2 leaves every column unconverged: nks nbndval a perturbation."""
+    try:
+        gpu.set_k_ground_state(ksys, n_dfpt_maxiter=2)
+        qb = ksys.qpts[0].basis
+        dv = _smooth(qb.npw, ksys.npwqx, 2, qb.g2kin, 7)
+        with pytest.warns(UserWarning):
+            _, ierr = gpu.dfpt(2, dv, 1e-22, iq=1, return_ierr=True)
+        assert list(ierr) == [ksys.nks * ksys.nbndval] * 2
+    finally:
+        gpu.set_k_ground_state(ksys)

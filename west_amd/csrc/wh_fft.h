@@ -88,6 +88,10 @@ struct StickPlan {
   std::vector<int> perm;           // stick position -> caller index (0-based)
   std::vector<void*> allocations;
   void build(int nr1, int nr2, int nr3, int npw, const int* nl_1based, const int* nlm_1based);
+  // Plane part only, for complex functions with the given columns (i, j): no
+  // mirror columns and no points (k points: wh_kfft_sticks.hip's z kernels
+  // bring their own).  False where the grid has neither tpl nor rect kernels.
+  bool build_columns(int nr1, int nr2, int nr3, const std::vector<int>& ci, const std::vector<int>& cj);
   void release();
   long sticks_elems() const { return static_cast<long>(dev.n3) * dev.nct; }
   // real-space arrays of the plane kernels are [a3][a1][a2] (else [a3][a2][a1])
@@ -231,6 +235,26 @@ void cg_iter_lds(int n1, int n2, int n3, int npw, long ld, const int* nl, const 
                  int nq2, const double* q2, const double* qs, int cap, const int* l2i, const int* nc,
                  const double* beta, const double* eu, const double* ep, z64* h, z64* hold, z64* x, z64* g, z64* bc,
                  z64* tc, double* rho, hipStream_t s, const KlKpoint* ktab = nullptr, int cols_per_k = 1);
+
+// Local term at k points through sticks (wh_kfft_sticks.hip): the columns are
+// those of a StickPlan::build_columns plan that holds every k sphere, the
+// points of k point k lie in column order (col_off: n columns + 1).  Band
+// column b belongs to k point (l2i ? l2i[b] : b) / cols_per_k of the table (0
+// where cols_per_k is 0).
+struct KStick {
+  int npw;
+  const int* col_off;
+  const int* pt_col;
+  const int* pt_k;
+  const double* g2;   // |k+G|^2, stick order
+};
+bool kz_available(int n3);
+// columns c0 .. c0 + n - 1 (below *d_nc, may be null) of x to sticks[0 .. n)
+void launch_kzinv(const StickPlan& p, const KStick* tab, const int* l2i, int cols_per_k, int c0, int n,
+                  const int* d_nc, const z64* x, long ld, z64* sticks, hipStream_t s);
+// t = sphere part of the sticks' forward transform + (g2 - e[b]) x, zero beyond npw
+void launch_kzfwd(const StickPlan& p, const KStick* tab, const int* l2i, int cols_per_k, int c0, int n,
+                  const int* d_nc, const z64* sticks, const z64* x, const double* e, z64* t, long ld, hipStream_t s);
 
 // kernel launchers (double precision)
 void launch_zinv(const StickPlan& p, const FftItem* d_items, int nitems, const z64* psi, long ldpsi,

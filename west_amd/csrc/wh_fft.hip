@@ -688,6 +688,40 @@ void StickPlan::build(int nr1, int nr2, int nr3, int npw, const int* nl, const i
   vloc32_occ = occ;
 }
 
+bool StickPlan::build_columns(int nr1, int nr2, int nr3, const std::vector<int>& ci, const std::vector<int>& cj) {
+  release();
+  const int n = static_cast<int>(ci.size());
+  WH_REQUIRE(n > 0 && ci.size() == cj.size(), "a stick plan needs columns");
+  StickPlanDev& d = dev;
+  d = StickPlanDev{};
+  for (int c = 0; c < n; ++c) {
+    d.imax = std::max(d.imax, std::abs(ci[c]));
+    d.jext = std::max(d.jext, std::abs(cj[c]));
+  }
+  d.nrows = 2 * d.imax + 1;
+  if (d.nrows > nr1 || 2 * d.jext + 1 > nr2) return false;
+  d.n1 = nr1; d.n2 = nr2; d.n3 = nr3;
+  d.ncs = d.nct = n;
+  col_i = ci;
+  col_j = cj;
+  col_pos.assign(n, 0);
+  for (int c = 0; c < n; ++c) col_pos[c] = (ci[c] + d.imax) * nr2 + ((cj[c] % nr2 + nr2) % nr2);
+  d.ax1 = make_axis(nr1);
+  d.ax2 = make_axis(nr2);
+  d.ax3 = make_axis(nr3);
+  d.col_pos = upload(col_pos, allocations);
+  d.tw1 = upload_twiddles(nr1, allocations);
+  d.tw2 = upload_twiddles(nr2, allocations);
+  d.tw3 = upload_twiddles(nr3, allocations);
+  tpl = tpl_kernels_f64(dev);
+  tplz = nullptr;
+  tpl32 = nullptr;
+  rect = RectPlan{};
+  if (!tpl) rect_plan(dev, rect);
+  vloc_occ = 0;
+  return tpl || rect.ok;
+}
+
 void launch_zinv(const StickPlan& p, const FftItem* d_items, int nitems, const z64* psiA, long ldA,
                  const z64* psiB, long ldB, z64* sticks, int mode, hipStream_t s) {
   if (nitems <= 0) return;

@@ -16,6 +16,23 @@ void dgemm(bool transa, int M, int N, int K, double alpha, const double* A, long
 void dgemm_bra(int M, int N, int K, double alpha, const double* A, long lda, const double* B, long ldb, double g0,
                const double* scale, double* C, long ldc, hipStream_t s, const int* d_n = nullptr);
 
+// Products whose columns fall into ng consecutive groups with a left operand
+// each (device arrays: A[g]; columns starts[g] .. starts[g+1] - 1 of group g;
+// tstart[g] = the tiles of kGroupTile columns before group g, tstart[ng] = all).
+struct DgemmGroups {
+  const double* const* A = nullptr;
+  const int* starts = nullptr;
+  const int* tstart = nullptr;
+  int ng = 0;
+};
+constexpr int kGroupTile = 64;
+// C(i, j) = scale_i (A_g^T B)(i, j), K split as in dgemm_bra; N bounds the columns
+void dgemm_bra_groups(const DgemmGroups& G, int M, int N, int K, long lda, const double* B, long ldb,
+                      const double* scale, double* C, long ldc, hipStream_t s, const int* d_n);
+// C = A_g B + beta C
+void dgemm_ket_groups(const DgemmGroups& G, int M, int N, int K, long lda, const double* B, long ldb, double beta,
+                      double* C, long ldc, hipStream_t s);
+
 // C(i, j) = scale_i * (C(i, j) - g0 * A[i*lda] * B[j*ldb])   (scale may be null)
 void g0_fix_scale(int M, int N, double g0, const double* A, long lda, const double* B, long ldb,
                   const double* scale, double* C, long ldc, hipStream_t s);

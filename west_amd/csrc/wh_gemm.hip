@@ -103,13 +103,19 @@ __host__ __device__ inline int xcd_blocks(int tiles) { return (tiles + kXcds - 1
 // WN: 16-column MFMA blocks per wavefront along N, i.e. tiles of
 // BM x (32 WN) (WN = 4: 128 x 128; narrower tiles give more workgroups to
 // products with few columns).
-template <bool TA, int WN>
+// GRP: the columns fall into groups with a left operand of their own (device
+// tables G); a tile lies within one group.
+template <bool TA, int WN, bool GRP = false>
 __global__ __launch_bounds__(NT, 2) void k_dgemm(int M, int N, int K, int kchunk, double alpha,
                                               const double* __restrict__ A, long lda, const double* __restrict__ B,
                                               long ldb, double beta, double* __restrict__ C, long ldc, long pstride,
-                                              int gx, int gy, int gz, const int* __restrict__ d_n) {
+                                              int gx, int gy, int gz, const int* __restrict__ d_n,
+                                              DgemmGroups G) {
   constexpr int TN = 32 * WN;
-  if (d_n) {
+  if (GRP) {
+    gy = G.tstart[G.ng];
+    if (gy == 0) return;   // no active column
+  } else if (d_n) {
     // columns the device left active: the tiles of the active columns are
     // renumbered over the whole grid, so they still spread over all XCDs
     N = min(N, *d_n);
@@ -129,7 +135,19 @@ __global__ __launch_bounds__(NT, 2) void k_dgemm(int M, int N, int K, int kchunk
   const int W = static_cast<int>(blockIdx.x % kXcds) * (xcd_blocks(tiles) / kXcds) + static_cast<int>(blockIdx.x / kXcds);
   if (W >= tiles) return;   // uniform per workgroup
   const int m0 = (W % gx) * BM;
-  const int n0 = ((W / gx) % gy) * TN;
+  int n0 = ((W / gx) % gy) * TN;
+  if (GRP) {
+    const int by = (W / gx) % gy;
+    int lo = 0, hi = G.ng;   // the last group that starts at or before this tile
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) / 2;
+      if (G.tstart[mid] <= by) lo = mid;
+      else hi = mid;
+    }
+    A = G.A[lo];
+    n0 = G.starts[lo] + (by - G.tstart[lo]) * TN;
+    N = G.starts[lo + 1];
+  }
   if (n0 >= N) return;      // uniform per workgroup
   const int kz = W / (gx * gy);
   const int kbeg = kz * kchunk;
@@ -337,7 +355,8 @@ __global__ void k_reduce_g0(int M, int N, int nsplit, const double* P, long pstr
   const long o = static_cast<long>(j) * ldc + i;
   double acc = 0.0;
   for (int z = 0; z < nsplit; ++z) acc += P[static_cast<long>(z) * pstride + o];
-  double v = alpha * acc - g0 * A[static_cast<long>(i) * lda] * B[static_cast<long>(j) * ldb];
+  double v = alpha * acc;
+  if (g0 != 0.0) v -= g0 * A[static_cast<long>(i) * lda] * B[static_cast<long>(j) * ldb];
   if (s) v *= s[i];
   C[o] = v;
 }
@@ -391,7 +410,7 @@ static void launch_tiles(int M, int N, int K, int kchunk, int gz, double alpha, 
                          const int* d_n) {
   const int gx = ceil_div(M, BM), gy = ceil_div(N, 32 * WN);
   k_dgemm<TA, WN><<<xcd_blocks(gx * gy * gz), NT, 0, s>>>(M, N, K, kchunk, alpha, A, lda, B, ldb, beta, C, ldc,
-                                                          pstride, gx, gy, gz, d_n);
+                                                          pstride, gx, gy, gz, d_n, DgemmGroups{});
   WH_HIP(hipGetLastError());
 }
 
@@ -580,6 +599,43 @@ void dgemm_bra(int M, int N, int K, double alpha, const double* A, long lda, con
   lk.unlock();
   // recomputed with the chosen variant, so the result does not depend on the timing order
   run(pick);
+}
+
+// ---- grouped products (one left operand per group of columns) -------------
+// 64-column tiles: a group (one k point's active columns) has a few tens to
+// a few hundred columns.
+static_assert(kGroupTile == 64, "the grouped products run k_dgemm's WN = 2 tiles");
+
+template <bool TA>
+static void launch_groups(const DgemmGroups& G, int M, int N, int K, int kchunk, int gz, double alpha, long lda,
+                          const double* B, long ldb, double beta, double* C, long ldc, long pstride, hipStream_t s) {
+  const int gx = ceil_div(M, BM), gy = ceil_div(N, kGroupTile) + G.ng;
+  k_dgemm<TA, 2, true><<<xcd_blocks(gx * gy * gz), NT, 0, s>>>(M, N, K, kchunk, alpha, nullptr, lda, B, ldb, beta, C,
+                                                               ldc, pstride, gx, gy, gz, nullptr, G);
+  WH_HIP(hipGetLastError());
+}
+
+void dgemm_bra_groups(const DgemmGroups& G, int M, int N, int K, long lda, const double* B, long ldb,
+                      const double* scale, double* C, long ldc, hipStream_t s, const int* d_n) {
+  if (M <= 0 || N <= 0) return;
+  // as bra_split, for the fewest tiles N columns can make
+  const int tiles = ceil_div(M, BM) * ceil_div(N, kGroupTile);
+  int split = std::max(1, std::min({64, ceil_div(512, tiles), K / (16 * BK)}));
+  const int kchunk = ceil_div(ceil_div(std::max(K, 1), split), BK) * BK;
+  split = ceil_div(std::max(K, 1), kchunk);
+  const long pstride = static_cast<long>(ldc) * N;
+  double* P = partials().get(static_cast<size_t>(split) * pstride, s);
+  launch_groups<true>(G, M, N, K, kchunk, split, 1.0, lda, B, ldb, 0.0, P, ldc, pstride, s);
+  const long n = static_cast<long>(M) * N;
+  k_reduce_g0<<<ceil_div(n, 256), 256, 0, s>>>(M, N, split, P, pstride, 1.0, 0.0, nullptr, 0, nullptr, 0, scale, C,
+                                               ldc, d_n);
+  WH_HIP(hipGetLastError());
+}
+
+void dgemm_ket_groups(const DgemmGroups& G, int M, int N, int K, long lda, const double* B, long ldb, double beta,
+                      double* C, long ldc, hipStream_t s) {
+  if (M <= 0 || N <= 0) return;
+  launch_groups<false>(G, M, N, K, std::max(K, 1), 1, 1.0, lda, B, ldb, beta, C, ldc, 0, s);
 }
 
 // ---- products for callers that neither allocate nor time -------------------

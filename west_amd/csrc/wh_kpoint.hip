@@ -9,10 +9,17 @@
 // (davidson_diago_k) with the complex branch of do_mgs (909-1117) and
 // do_randomize_q (1186-1250).
 //
-// Layout: vectors keep the caller's order (rows of npwx or npwqx complex).
-// Away from Gamma a wave function has no Hermitian partner, so there is no
-// two-band packing and no half sphere: each band is one complex transform on
-// the full FFT grid (GridFft, three batched passes of LDS line transforms).
+// Layout: rows of npwx or npwqx complex.  Away from Gamma a wave function has
+// no Hermitian partner, so there is no two-band packing and no half sphere.
+// Grids that fit the LDS keep the caller's order and transform each band in
+// one workgroup (wh_kfft_lds.hip).  On larger grids the k-point vectors are in
+// stick order (columns of constant (i, j), k ascending) and the operator runs
+// through sticks: z transforms of the columns that hold points
+// (wh_kfft_sticks.hip) around the Gamma path's plane kernels, which take one
+// complex function per item.  One column set holds every k sphere, so a
+// launch takes the columns of several k points.  The transforms of dfpt's
+// grids, and of grids without such kernels, are full-grid ones (GridFft,
+// three batched passes of LDS line transforms).
 // The complex projections run on the FP64 matrix-core GEMMs of the Gamma path
 // through the real view of the arrays: with Q2 = [evc, i evc, vkb, i vkb]
 // (2 npwx x 2 nq reals), Q2^T f = [Re; Im] of Q^H f and Q2 [Re X; Im X] = Q X,
@@ -27,11 +34,13 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <map>
 #include <vector>
 
 #include "../../include/west_hip.h"
 #include "wh_context.h"
 #include "wh_fft.h"
+#include "wh_fft_rect.h"
 #include "wh_gemm.h"
 #include "wh_vec.h"
 
@@ -46,6 +55,10 @@ struct KPointDev {
   std::vector<double> eprec;  // nbndval: 1.35 sum |evc|^2 |k+G|^2 (Tools/set_eprec.f90:40-56)
   double* d_et = nullptr;     // the same two on the device
   double* d_eprec = nullptr;
+  // stick order (KPath::sticks_want): caller index of each stick position, and
+  // the columns (i, j) with the points' column and k
+  int* perm = nullptr;
+  std::vector<int> col_i, col_j, pt_col, pt_k;
   bool set = false;
 };
 
@@ -84,6 +97,16 @@ struct KPath {
   hipEvent_t cg_ev[4] = {nullptr, nullptr, nullptr, nullptr};   // lagged reads of the CG loop
   KlKpoint* ktab = nullptr;   // device: each k point's sphere and projectors (batched CG)
   double* sck = nullptr;      // device: 2 w_k / (Omega N_r) per k point (densities at q)
+  // stick transforms (grids beyond the LDS): k-point vectors are in stick order
+  bool sticks_want = false;   // the grid has the z kernels
+  bool sticks_built = false;  // the plan below holds every registered k sphere
+  bool sticks_ok = false;     // ... and the grid has plane kernels for it
+  StickPlan plan;             // union of the k spheres' columns
+  KStick* stab = nullptr;     // device, per k point
+  const double** qptr = nullptr;   // device, per k point: q2
+  double* vrs_plane = nullptr;     // vrs in the plane kernels' layout
+  std::vector<void*> stick_allocs;
+  DevBuf w_sa, w_sb, w_ident, w_grp;
   DevBuf w_dk;                // densities per (k point, perturbation) before the sum over k
 };
 
@@ -97,6 +120,9 @@ void free_kpath(KPath* k) {
   if (!k) return;
   for (void* p : k->allocs) (void)hipFree(p);
   k->fft.release();
+  k->plan.release();
+  for (void* p : k->stick_allocs) (void)hipFree(p);
+  for (DevBuf* b : {&k->w_sa, &k->w_sb, &k->w_ident, &k->w_grp}) b->release();
   for (DevBuf* b : {&k->g_a, &k->g_b, &k->g_c, &k->g_aux, &k->w_x, &k->w_t, &k->w_g, &k->w_h, &k->w_hold, &k->w_bc,
                     &k->w_tc, &k->w_c2, &k->w_l2i, &k->w_rho, &k->w_rhoold, &k->w_conv, &k->w_nonconv, &k->w_beta,
                     &k->w_eu, &k->w_ecol, &k->w_epcol, &k->w_dv, &k->w_dn, &k->w_in, &k->w_out, &k->w_in2})
@@ -245,11 +271,15 @@ __global__ void k_scale_rows(int m, int n, long ld, const double* __restrict__ w
 
 // pf = f / max(1, g2kin / eprec[col])  (precondition_m_wfcts.f90:35-51)
 __global__ void k_precond(int m, int npw, long ld, const double* __restrict__ g2, const double* __restrict__ ep,
-                          const z64* __restrict__ f, z64* __restrict__ pf) {
+                          const z64* __restrict__ f, z64* __restrict__ pf, const KlKpoint* __restrict__ tab, int cols) {
   const long n = static_cast<long>(m) * ld;
   for (long t = blockIdx.x * static_cast<long>(NT) + threadIdx.x; t < n; t += static_cast<long>(gridDim.x) * NT) {
     const int b = static_cast<int>(t / ld);
     const int ig = static_cast<int>(t - static_cast<long>(b) * ld);
+    if (tab) {
+      npw = tab[b / cols].npw;
+      g2 = tab[b / cols].g2;
+    }
     pf[t] = ig < npw ? cscale(f[t], 1.0 / fmax(1.0, g2[ig] / ep[b])) : mk(0.0, 0.0);
   }
 }
@@ -261,13 +291,19 @@ __global__ void k_precond(int m, int npw, long ld, const double* __restrict__ g2
 // cg_select on the device; nc null: all launched columns).
 
 // h = g / max(1, g2kin/eprec) on the listed columns, rho[band] = Re <h|g> (150-160, 183-205)
+// (tab: columns [k cols, (k + 1) cols) belong to k point k; null: npw and g2 for all)
 __global__ __launch_bounds__(NT) void k_cg_prec_rho(const int* __restrict__ l2i, const int* __restrict__ nc,
                                                     int npw, long ld, const double* __restrict__ g2,
                                                     const double* __restrict__ ep, const z64* __restrict__ g,
-                                                    z64* __restrict__ h, double* __restrict__ rho) {
+                                                    z64* __restrict__ h, double* __restrict__ rho,
+                                                    const KlKpoint* __restrict__ tab, int cols) {
   __shared__ double red[NT / 64];
   if (nc && static_cast<int>(blockIdx.x) >= *nc) return;   // whole workgroup
   const int col = l2i[blockIdx.x];
+  if (tab) {
+    npw = tab[col / cols].npw;
+    g2 = tab[col / cols].g2;
+  }
   const z64* gc = g + col * ld;
   z64* hc = h + col * ld;
   const double e = ep[col];
@@ -309,11 +345,16 @@ __global__ __launch_bounds__(NT) void k_cg_step(const int* __restrict__ l2i, con
                                                 const double* __restrict__ ep, z64* __restrict__ x,
                                                 z64* __restrict__ g, z64* __restrict__ h,
                                                 const z64* __restrict__ tc, z64* __restrict__ hold,
-                                                double* __restrict__ rho) {
+                                                double* __restrict__ rho, const KlKpoint* __restrict__ tab,
+                                                int cols) {
   __shared__ double red[NT / 64];
   const int lb = blockIdx.x;
   if (lb >= *nc) return;   // whole workgroup
   const int col = l2i[lb];
+  if (tab) {
+    npw = tab[col / cols].npw;
+    g2 = tab[col / cols].g2;
+  }
   z64* xc = x + col * ld;
   z64* gc = g + col * ld;
   z64* hc = h + col * ld;
@@ -366,6 +407,57 @@ __global__ void k_band_cols(int cols, int nb, const double* __restrict__ et, con
   if (j < cols) {
     ec[j] = et[j % nb];
     epc[j] = ep[j % nb];
+  }
+}
+
+// the same for the columns of every k point (perturbation-major inside each)
+__global__ void k_band_cols_all(int m, int cols, int nb, const KlKpoint* __restrict__ tab,
+                                const KlQpoint* __restrict__ qtab, double* __restrict__ ec, double* __restrict__ epc) {
+  const int j = blockIdx.x * NT + threadIdx.x;
+  if (j >= m) return;
+  const int k = j / cols;
+  const int v = (j - k * cols) % nb;
+  ec[j] = tab[qtab[k].ikq].et[v];
+  epc[j] = tab[k].eprec[v];
+}
+
+// plane items of n columns in chunks: slot q % chunk while q < *nc (nc null: all)
+__global__ void k_ident_cols(FftItem* items, int n, int chunk, const int* __restrict__ nc) {
+  const int q = blockIdx.x * NT + threadIdx.x;
+  if (q >= n) return;
+  FftItem it;
+  it.a = (!nc || q < *nc) ? q % chunk : -1;
+  it.b = -1;
+  it.pot = -1;
+  it.pad = 0;
+  items[q] = it;
+}
+
+// Where each k point's columns lie among the *nc active ones (l2i ascending;
+// null: all m columns) and the column tiles of width tn before them
+__global__ __launch_bounds__(NT) void k_group_starts(int ng, int cols, int m, const int* __restrict__ l2i,
+                                                     const int* __restrict__ nc, int tn, int* __restrict__ starts,
+                                                     int* __restrict__ tstart) {
+  const int n = nc ? *nc : m;
+  for (int g = threadIdx.x; g <= ng; g += NT) {
+    int lo = 0, hi = n;
+    const int key = g * cols;
+    while (lo < hi) {
+      const int mid = (lo + hi) / 2;
+      if ((l2i ? l2i[mid] : mid) < key) lo = mid + 1;
+      else hi = mid;
+    }
+    starts[g] = lo;
+  }
+  __threadfence_block();
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int t = 0;
+    for (int g = 0; g < ng; ++g) {
+      tstart[g] = t;
+      t += (starts[g + 1] - starts[g] + tn - 1) / tn;
+    }
+    tstart[ng] = t;
   }
 }
 
@@ -478,6 +570,127 @@ static bool klds_enabled() {
   return on;
 }
 
+// WH_KSTICKS=0: the full-grid transforms also where the grid has stick kernels
+// (read when the k grid is registered)
+static bool ksticks_enabled() {
+  const char* ev = std::getenv("WH_KSTICKS");
+  return !(ev && ev[0] == '0');
+}
+
+// The stick plan of the registered k points: the union of their columns, so
+// that one plane launch takes items of any of them.  Built at the first use
+// after a registration.
+static bool sticks_ready(KPath& K) {
+  if (!K.sticks_want) return false;
+  if (K.sticks_built) return K.sticks_ok;
+  Context& c = ctx();
+  WH_HIP(hipStreamSynchronize(c.stream));
+  for (void* p : K.stick_allocs) (void)hipFree(p);
+  K.stick_allocs.clear();
+  K.stab = nullptr;
+  K.sticks_ok = false;
+  std::map<std::pair<int, int>, int> at;
+  for (const KPointDev& P : K.k)
+    for (size_t q = 0; q < P.col_i.size(); ++q) at[{P.col_i[q], P.col_j[q]}] = 0;
+  std::vector<int> ci, cj;
+  for (auto& e : at) {
+    e.second = static_cast<int>(ci.size());
+    ci.push_back(e.first.first);
+    cj.push_back(e.first.second);
+  }
+  K.sticks_built = true;
+  if (ci.empty() || !K.plan.build_columns(K.fft.n1, K.fft.n2, K.fft.n3, ci, cj)) return false;
+  auto up = [&](const auto& h) {
+    using V = typename std::decay_t<decltype(h)>::value_type;
+    V* d = nullptr;
+    WH_HIP(hipMalloc(&d, sizeof(V) * std::max<size_t>(h.size(), 1)));
+    K.stick_allocs.push_back(d);
+    if (!h.empty()) WH_HIP(hipMemcpy(d, h.data(), sizeof(V) * h.size(), hipMemcpyHostToDevice));
+    return d;
+  };
+  std::vector<KStick> tab(K.nks, KStick{0, nullptr, nullptr, nullptr, nullptr});
+  std::vector<const double*> qp(K.nks, nullptr);
+  for (int ik = 0; ik < K.nks; ++ik) {
+    const KPointDev& P = K.k[ik];
+    if (!P.set) continue;
+    std::vector<int> off(ci.size() + 1, 0), pc(P.npw);
+    for (int s = 0; s < P.npw; ++s) {
+      pc[s] = at[{P.col_i[P.pt_col[s]], P.col_j[P.pt_col[s]]}];
+      ++off[pc[s] + 1];
+    }
+    for (size_t q = 1; q < off.size(); ++q) off[q] += off[q - 1];
+    tab[ik] = KStick{P.npw, up(off), up(pc), up(P.pt_k), P.g2kin};
+    qp[ik] = reinterpret_cast<const double*>(P.q2);
+  }
+  K.stab = up(tab);
+  K.qptr = up(qp);
+  K.vrs_plane = K.vrs;
+  if (K.plan.transposed_grid()) {
+    double* v = nullptr;
+    WH_HIP(hipMalloc(&v, sizeof(double) * K.fft.nnr()));
+    K.stick_allocs.push_back(v);
+    rect_transpose_grid(K.fft.n1, K.fft.n2, K.fft.n3, K.vrs, v, c.stream);
+    K.vrs_plane = v;
+  }
+  K.sticks_ok = true;
+  return true;
+}
+
+// t = F^-1 V F x + (|k+G|^2 - e) x through sticks for m columns (cols_per_k,
+// l2i: as in KStick; 0: all of k point ik)
+static void vloc_sticks(KPath& K, int ik, int cols_per_k, const int* l2i, const z64* x, z64* t, const double* d_e,
+                        int m, const int* d_nc) {
+  Context& c = ctx();
+  hipStream_t s = c.stream;
+  const long ld = K.npwx;
+  const long sl = K.plan.sticks_elems();
+  const long fit = static_cast<long>(K.grid_budget) / (2 * sl * static_cast<long>(sizeof(z64)));
+  const int chunk = static_cast<int>(std::max<long>(1, std::min<long>({fit, 65535L, m})));
+  FftItem* items = K.w_ident.as<FftItem>(m);
+  k_ident_cols<<<ceil_div(m, NT), NT, 0, s>>>(items, m, chunk, d_nc);
+  WH_HIP(hipGetLastError());
+  z64* sa = K.w_sa.as<z64>(static_cast<size_t>(chunk) * sl);
+  z64* sb = K.w_sb.as<z64>(static_cast<size_t>(chunk) * sl);
+  const KStick* tab = cols_per_k > 0 ? K.stab : K.stab + ik;
+  const double scale = 1.0 / static_cast<double>(K.fft.nnr());
+  for (int c0 = 0; c0 < m; c0 += chunk) {
+    const int n = std::min(chunk, m - c0);
+    WH_TIMED("kzinv", launch_kzinv(K.plan, tab, l2i, cols_per_k, c0, n, d_nc, x, ld, sa, s));
+    WH_TIMED("plane_vloc", launch_plane_vloc(K.plan, items + c0, n, sa, sb, K.vrs_plane, 0, scale, s));
+    WH_TIMED("kzfwd", launch_kzfwd(K.plan, tab, l2i, cols_per_k, c0, n, d_nc, sb, x, d_e, t, ld, s));
+  }
+}
+
+// The columns of every k point at once: bra and ket products whose left
+// operand is the column's k point's (rows beyond npw are zero in the
+// projectors and the vectors, so all k points share the length 2 npwx)
+static DgemmGroups k_groups(KPath& K, int cols, int m, const int* l2i, const int* d_nc) {
+  Context& c = ctx();
+  int* st = K.w_grp.as<int>(2 * (static_cast<size_t>(K.nks) + 1));
+  k_group_starts<<<1, NT, 0, c.stream>>>(K.nks, cols, m, l2i, d_nc, kGroupTile, st, st + K.nks + 1);
+  WH_HIP(hipGetLastError());
+  return DgemmGroups{K.qptr, st, st + K.nks + 1, K.nks};
+}
+
+static void stern_all(KPath& K, int cols, const z64* x, z64* t, const double* d_e, int m, const int* l2i,
+                      const int* d_nc) {
+  Context& c = ctx();
+  hipStream_t s = c.stream;
+  const long ld = K.npwx;
+  vloc_sticks(K, 0, cols, l2i, x, t, d_e, m, d_nc);
+  const int nq = K.nbndval + K.nkb;
+  if (nq > 0) {
+    set_qscale2(K, K.alpha_pv);
+    const DgemmGroups G = k_groups(K, cols, m, l2i, d_nc);
+    double* c2 = K.w_c2.as<double>(static_cast<size_t>(2) * nq * m);
+    WH_TIMED("gemm_bra", dgemm_bra_groups(G, 2 * nq, m, 2 * static_cast<int>(ld), 2 * ld,
+                                          reinterpret_cast<const double*>(x), 2 * ld, K.qscale2, c2, 2 * nq, s, d_nc));
+    WH_TIMED("gemm_ket", dgemm_ket_groups(G, 2 * static_cast<int>(ld), m, 2 * nq, 2 * ld, c2, 2 * nq, 1.0,
+                                          reinterpret_cast<double*>(t), 2 * ld, s));
+  }
+  if (!d_nc) c.nstern += m;
+}
+
 // d_nc (device int, may be null): only the first min(m, *d_nc) columns are
 // used (a CG launch sized for a capacity); the caller counts the applications.
 static void stern_k(KPath& K, int ik, const z64* x, z64* t, const double* d_e, int m, double alpha,
@@ -493,7 +706,9 @@ static void stern_k(KPath& K, int ik, const z64* x, z64* t, const double* d_e, i
   if (lds)
     WH_TIMED("kvloc_lds", kvloc_lds(K.fft.n1, K.fft.n2, K.fft.n3, m, P.npw, ld, P.nl, x, K.vrs, P.g2kin, d_e, t, s,
                                     d_nc));
-  for (int c0 = 0; c0 < (lds ? 0 : m); c0 += gc) {
+  const bool sticks = !lds && !c.l_kinetic_only && m > 0 && sticks_ready(K);
+  if (sticks) vloc_sticks(K, ik, 0, nullptr, x, t, d_e, m, d_nc);
+  for (int c0 = 0; c0 < (lds || sticks ? 0 : m); c0 += gc) {
     const int mc = std::min(gc, m - c0);
     const z64* xc = x + c0 * ld;
     z64* tc = t + c0 * ld;
@@ -539,6 +754,20 @@ static void minus_pc_k(KPath& K, int ik, z64* f, int m) {
                              reinterpret_cast<double*>(f), 2 * ld, c.stream));
 }
 
+// the same for the columns of every k point
+static void minus_pc_all(KPath& K, int cols, z64* f, int m) {
+  Context& c = ctx();
+  const long ld = K.npwx;
+  const int nb = K.nbndval;
+  const DgemmGroups G = k_groups(K, cols, m, nullptr, nullptr);
+  double* c2 = K.w_c2.as<double>(static_cast<size_t>(2) * nb * m);
+  WH_TIMED("gemm_bra", dgemm_bra_groups(G, 2 * nb, m, 2 * static_cast<int>(ld), 2 * ld,
+                                        reinterpret_cast<const double*>(f), 2 * ld, nullptr, c2, 2 * nb, c.stream,
+                                        nullptr));
+  WH_TIMED("gemm_ket", dgemm_ket_groups(G, 2 * static_cast<int>(ld), m, 2 * nb, 2 * ld, c2, 2 * nb, -1.0,
+                                        reinterpret_cast<double*>(f), 2 * ld, c.stream));
+}
+
 // PCG for (H_k - e_i + alpha_pv P_v) x_i = b_i, i < m; b is destroyed.
 // Columns are perturbation-major, `group` bands per perturbation (call count).
 // The loop (linsolve_sternheimer_m_wfcts.f90:146-330) runs on the device:
@@ -556,7 +785,7 @@ static void minus_pc_k(KPath& K, int ik, z64* f, int m) {
 // launched to cg_k_count.
 // nkb = 1: the cols columns belong to k point ik.  nkb = nks: columns
 // [k cols, (k + 1) cols) belong to k point k, all in one solve (the fused
-// iteration only, kbatch_ok).
+// iteration, kbatch_ok, or the stick operator, kbatch_cols).
 static int linsolve_k(KPath& K, int ik, int nkb, int cols, z64* b, z64* x, const double* d_e, const double* d_ep,
                       double tr2, int group, int nper, int* rec, int* nonconv) {
   Context& c = ctx();
@@ -589,18 +818,21 @@ static int linsolve_k(KPath& K, int ik, int nkb, int cols, z64* b, z64* x, const
   const int nq2 = 2 * (K.nbndval + K.nkb);
   const bool fused = klds_enabled() && !c.l_kinetic_only &&
                      cg_iter_lds_available(K.fft.n1, K.fft.n2, K.fft.n3, nq2);
-  WH_REQUIRE(fused || nkb == 1, "linsolve_k: several k points need the fused iteration");
+  WH_REQUIRE(fused || nkb == 1 || (!c.l_kinetic_only && sticks_ready(K)),
+             "linsolve_k: several k points need the fused iteration or the stick operator");
+  const KlKpoint* tab = nkb > 1 ? K.ktab : nullptr;
   if (fused) set_qscale2(K, K.alpha_pv);
   // step 1 (127-138): g = A x - b, and h = M^-1 g, rho of every band
-  if (nkb > 1) {   // every k point's columns in one launch
+  if (nkb > 1 && fused) {   // every k point's columns in one launch
     WH_TIMED("cg_iter_lds", cg_first_lds(K.fft.n1, K.fft.n2, K.fft.n3, ld, K.vrs, nq2, K.qscale2, m, d_e, d_ep, x,
                                          b, g, h, d_rhob, K.ktab, cols, s));
     c.nstern += m;
   } else {
     iota(d_l2i, m, s);
-    stern_k(K, ik, x, g, d_e, m, K.alpha_pv);
+    if (nkb > 1) stern_all(K, cols, x, g, d_e, m, nullptr, nullptr);
+    else stern_k(K, ik, x, g, d_e, m, K.alpha_pv);
     k_sub<<<blocks(static_cast<long>(vec)), NT, 0, s>>>(static_cast<long>(vec), b, g);
-    k_cg_prec_rho<<<m, NT, 0, s>>>(d_l2i, nullptr, P.npw, ld, P.g2kin, d_ep, g, h, d_rhob);
+    k_cg_prec_rho<<<m, NT, 0, s>>>(d_l2i, nullptr, P.npw, ld, P.g2kin, d_ep, g, h, d_rhob, tab, cols);
     WH_HIP(hipGetLastError());
   }
   count_calls(m, nullptr, group);
@@ -625,8 +857,9 @@ static int linsolve_k(KPath& K, int ik, int nkb, int cols, z64* b, z64* x, const
     } else {
       k_cg_dir<<<blocks(static_cast<long>(cap) * ld), NT, 0, s>>>(cap, d_nc, d_l2i, ld, d_beta, d_e, h, hold, bc,
                                                                   d_eu);
-      stern_k(K, ik, bc, tc, d_eu, cap, K.alpha_pv, d_nc);
-      k_cg_step<<<cap, NT, 0, s>>>(d_l2i, d_nc, P.npw, ld, P.g2kin, d_ep, x, g, h, tc, hold, d_rhob);
+      if (nkb > 1) stern_all(K, cols, bc, tc, d_eu, cap, d_l2i, d_nc);
+      else stern_k(K, ik, bc, tc, d_eu, cap, K.alpha_pv, d_nc);
+      k_cg_step<<<cap, NT, 0, s>>>(d_l2i, d_nc, P.npw, ld, P.g2kin, d_ep, x, g, h, tc, hold, d_rhob, tab, cols);
       WH_HIP(hipGetLastError());
     }
     WH_HIP(hipMemcpyAsync(rec + 2 * it, d_rec, 2 * sizeof(int), hipMemcpyDeviceToHost, s));
@@ -670,6 +903,24 @@ static bool kbatch_ok(const KPath& K, int m) {
          bytes <= static_cast<long>(K.grid_budget);
 }
 
+// On grids beyond the LDS: perturbations per solve over every k point through
+// the stick operator, 0 for the k points one after another.  Counted against
+// the grid budget as above.
+static int kbatch_cols(KPath& K, int m) {
+  const char* ev = std::getenv("WH_KBATCH");
+  if (ev && ev[0] == '0') return 0;
+  const Context& c = ctx();
+  if (c.l_kinetic_only || K.nks < 2 || K.nbndval < 1 || !sticks_ready(K)) return 0;
+  const long nnr = K.fft.nnr(), z = static_cast<long>(sizeof(z64));
+  const long fixed = z * nnr * (static_cast<long>(K.nks) * K.nbndval + m);
+  const long per = z * (7L * K.nks * K.nbndval * K.npwx + static_cast<long>(K.nbndval + 1) * nnr);
+  const long room = static_cast<long>(K.grid_budget) - fixed;
+  if (room < per) return 0;
+  const long fit = std::min<long>({room / per, m, (1L << 24) / (static_cast<long>(K.nks) * K.nbndval)});
+  // equal chunks
+  return fit < 1 ? 0 : ceil_div(m, ceil_div(m, fit));
+}
+
 // dng (npwqx, m) = chi0(q) dvg for q point iq (0-based)  (dfpt_module.f90:163-505)
 static int dfpt_q(KPath& K, int iq, int m, const z64* dvg, z64* dng, double tr2, std::vector<int>* ierr_pert) {
   Context& c = ctx();
@@ -685,7 +936,9 @@ static int dfpt_q(KPath& K, int iq, int m, const z64* dvg, z64* dng, double tr2,
   if (ierr_pert) ierr_pert->assign(m, 0);
   if (m == 0 || nb == 0) return 0;
   // perturbations per chunk: their band columns' grids within the budget
-  const int mp = std::max(1, std::min(m, grid_cols(K) / std::max(nb, 1)));
+  const bool lds_all = tr2 >= 0.0 && kbatch_ok(K, m);
+  const int mall = tr2 >= 0.0 && !lds_all ? kbatch_cols(K, m) : 0;
+  const int mp = mall > 0 ? mall : std::max(1, std::min(m, grid_cols(K) / std::max(nb, 1)));
   // per solve: its CG records (pinned) and iterations launched, read at the end
   const int nsolve = K.nks * ((m + mp - 1) / mp);
   const size_t rec_len = 2 * (static_cast<size_t>(c.n_dfpt_maxiter) + 1);
@@ -699,25 +952,20 @@ static int dfpt_q(KPath& K, int iq, int m, const z64* dvg, z64* dng, double tr2,
   k_scatter<<<blocks(static_cast<long>(m) * Q.npwq), NT, 0, s>>>(m, Q.npwq, Q.nl, dvg, ldq, aux, nnr);
   WH_TIMED("kfft", launch_grid_fft(K.fft, aux, m, +1, s));
   // states at k - q in real space with the phase exp(-i g0.r) (288, 295)
-  auto states_kmq = [&](int ik) {
+  auto states_kmq = [&](int ik, z64* psik) {
     const KPointDev& PQ = K.k[Q.ikq[ik]];
-    z64* psik = K.g_b.as<z64>(static_cast<size_t>(nb) * nnr);
     zero_grids(psik, nb * nnr, s);
     k_scatter<<<blocks(static_cast<long>(nb) * PQ.npw), NT, 0, s>>>(nb, PQ.npw, PQ.nl, PQ.q2, ld, psik, nnr);
     WH_TIMED("kfft", launch_grid_fft(K.fft, psik, nb, +1, s));
     k_phase<<<blocks(nb * nnr), NT, 0, s>>>(nb, K.fft.n1, K.fft.n2, K.fft.n3, Q.g0[3 * ik], Q.g0[3 * ik + 1],
                                            Q.g0[3 * ik + 2], psik);
     WH_HIP(hipGetLastError());
-    return psik;
   };
-  // perturbations p0 .. p0 + mc - 1 at k point ik: per column e at k - q
-  // (222) and eprec from the states at k (211); dvpsi = -P_c fwfft(psi_{k-q}
-  // phase dv) on the k sphere (295-302, 346) and dpsi = M^-1 dvpsi (348)
-  auto rhs = [&](int ik, int p0, int mc, const z64* psik, z64* dvpsi, z64* dpsi, double* d_e, double* d_ep) {
+  // perturbations p0 .. p0 + mc - 1 at k point ik: fwfft(psi_{k-q} phase dv)
+  // on the k sphere (295-302)
+  auto rhs_grid = [&](int ik, int p0, int mc, const z64* psik, z64* dvpsi) {
     const KPointDev& P = K.k[ik];
-    const KPointDev& PQ = K.k[Q.ikq[ik]];
     const int cols = mc * nb;
-    k_band_cols<<<blocks(cols), NT, 0, s>>>(cols, nb, PQ.d_et, P.d_eprec, d_e, d_ep);
     z64* R = K.g_a.as<z64>(static_cast<size_t>(cols) * nnr);
     k_rhs<<<blocks(static_cast<long>(cols) * nnr), NT, 0, s>>>(nb, mc, nnr, psik, aux + p0 * nnr, R);
     WH_TIMED("kfft", launch_grid_fft(K.fft, R, cols, -1, s));
@@ -725,8 +973,18 @@ static int dfpt_q(KPath& K, int iq, int m, const z64* dvg, z64* dng, double tr2,
                                                                  1.0 / static_cast<double>(nnr), nullptr, nullptr,
                                                                  nullptr, 0, dvpsi);
     WH_HIP(hipGetLastError());
+  };
+  // per column e at k - q (222) and eprec from the states at k (211); dvpsi =
+  // -P_c of those (346) and dpsi = M^-1 dvpsi (348)
+  auto rhs = [&](int ik, int p0, int mc, const z64* psik, z64* dvpsi, z64* dpsi, double* d_e, double* d_ep) {
+    const KPointDev& P = K.k[ik];
+    const KPointDev& PQ = K.k[Q.ikq[ik]];
+    const int cols = mc * nb;
+    k_band_cols<<<blocks(cols), NT, 0, s>>>(cols, nb, PQ.d_et, P.d_eprec, d_e, d_ep);
+    rhs_grid(ik, p0, mc, psik, dvpsi);
     minus_pc_k(K, ik, dvpsi, cols);
-    k_precond<<<blocks(static_cast<long>(cols) * ld), NT, 0, s>>>(cols, P.npw, ld, P.g2kin, d_ep, dvpsi, dpsi);
+    k_precond<<<blocks(static_cast<long>(cols) * ld), NT, 0, s>>>(cols, P.npw, ld, P.g2kin, d_ep, dvpsi, dpsi,
+                                                                  nullptr, 1);
     WH_HIP(hipGetLastError());
   };
   // response density sum_v conj(psi_{k-q} phase) dpsi (433-441) and
@@ -746,7 +1004,33 @@ static int dfpt_q(KPath& K, int iq, int m, const z64* dvg, z64* dng, double tr2,
                                                                    nullptr, nullptr, 1, dng + p0 * ldq);
     WH_HIP(hipGetLastError());
   };
-  if (tr2 >= 0.0 && mp == m && kbatch_ok(K, m)) {
+  if (mall > 0) {
+    // grids beyond the LDS: the right-hand sides k point by k point, one CG
+    // over the columns of every k point, then the densities
+    z64* psik = K.g_b.as<z64>(static_cast<size_t>(K.nks) * nb * nnr);
+    const size_t all = static_cast<size_t>(K.nks) * mp * nb;
+    z64* dvpsi = K.w_dv.as<z64>(all * ld);
+    z64* dpsi = K.w_x.as<z64>(all * ld);
+    double* d_e = K.w_ecol.as<double>(all);
+    double* d_ep = K.w_epcol.as<double>(all);
+    for (int ik = 0; ik < K.nks; ++ik) states_kmq(ik, psik + static_cast<size_t>(ik) * nb * nnr);
+    for (int p0 = 0; p0 < m; p0 += mp) {
+      const int mc = std::min(mp, m - p0);
+      const int cols = mc * nb;
+      const int mk_ = K.nks * cols;
+      k_band_cols_all<<<blocks(mk_), NT, 0, s>>>(mk_, cols, nb, K.ktab, Q.d_kq, d_e, d_ep);
+      for (int ik = 0; ik < K.nks; ++ik)
+        rhs_grid(ik, p0, mc, psik + static_cast<size_t>(ik) * nb * nnr, dvpsi + static_cast<size_t>(ik) * cols * ld);
+      minus_pc_all(K, cols, dvpsi, mk_);
+      k_precond<<<blocks(static_cast<long>(mk_) * ld), NT, 0, s>>>(mk_, 0, ld, nullptr, d_ep, dvpsi, dpsi, K.ktab,
+                                                                   cols);
+      WH_HIP(hipGetLastError());
+      int* rec = recs + rec_len * launched.size();
+      launched.push_back(linsolve_k(K, 0, K.nks, cols, dvpsi, dpsi, d_e, d_ep, tr2, nb, mc, rec, d_nonconv + p0));
+      for (int ik = 0; ik < K.nks; ++ik)
+        density(ik, p0, mc, psik + static_cast<size_t>(ik) * nb * nnr, dpsi + static_cast<size_t>(ik) * cols * ld);
+    }
+  } else if (lds_all && mp == m) {
     // every k point at once (350-361): the states at k - q and the
     // right-hand sides of all k points on LDS grids, -P_c and M^-1 per k
     // point, one CG whose iterations take every k point's columns, then the
@@ -774,7 +1058,8 @@ static int dfpt_q(KPath& K, int iq, int m, const z64* dvg, z64* dng, double tr2,
                                       K.sck, dk, dng, s));
   } else {
     for (int ik = 0; ik < K.nks; ++ik) {
-      const z64* psik = states_kmq(ik);
+      z64* psik = K.g_b.as<z64>(static_cast<size_t>(nb) * nnr);
+      states_kmq(ik, psik);
       for (int p0 = 0; p0 < m; p0 += mp) {
         const int mc = std::min(mp, m - p0);
         const int cols = mc * nb;
@@ -832,6 +1117,19 @@ static void finish() {
   if (c.prof.on) c.prof.flush();
 }
 
+// k-point rows between the caller's order and stick order (zero beyond npw)
+static z64* to_stick_order(KPath& K, const KPointDev& P, const z64* in, int m, z64* out) {
+  hipStream_t s = ctx().stream;
+  const long ld = K.npwx;
+  if (P.npw < ld) zero_grids(out, m * ld, s);
+  gather_sticks(m, P.npw, P.perm, in, ld, out, ld, nullptr, s);
+  return out;
+}
+static z64* to_caller_order(KPath& K, const KPointDev& P, const z64* in, int m, z64* out) {
+  scatter_caller(m, P.npw, K.npwx, P.perm, in, K.npwx, out, K.npwx, ctx().stream);
+  return out;
+}
+
 int kpath_apply_sternheimerop(int nbndval, const double* psi, double* hpsi, const double* e, const double* alpha,
                               int m) {
   Context& c = ctx();
@@ -847,8 +1145,11 @@ int kpath_apply_sternheimerop(int nbndval, const double* psi, double* hpsi, cons
   const z64* pin = dev_in(reinterpret_cast<const z64*>(psi), cin, K.w_in);
   const double* pe = dev_in(e, m, K.w_ecol);
   z64* t = K.w_t.as<z64>(cin);
+  const KPointDev& P = K.k[ik];
+  if (P.perm) pin = to_stick_order(K, P, pin, m, K.w_x.as<z64>(cin));
   stern_k(K, ik, pin, t, pe, m, a[0]);
   ++c.nstern_calls;
+  if (P.perm) t = to_caller_order(K, P, t, m, K.w_x.as<z64>(cin));
   WH_HIP(hipMemcpyAsync(hpsi, t, sizeof(z64) * cin, hipMemcpyDefault, c.stream));
   finish();
   return 0;
@@ -868,8 +1169,12 @@ int kpath_linsolve(int nbndval, int m, double* b, double* x, const double* e, co
   const size_t cin = static_cast<size_t>(m) * K.npwx;
   z64* db = K.w_dv.as<z64>(cin);
   z64* dx = K.w_x.as<z64>(cin);
-  WH_HIP(hipMemcpyAsync(db, b, sizeof(z64) * cin, hipMemcpyDefault, s));
-  WH_HIP(hipMemcpyAsync(dx, x, sizeof(z64) * cin, hipMemcpyDefault, s));
+  const KPointDev& P = K.k[ik];
+  z64* stage = P.perm ? K.w_in.as<z64>(cin) : nullptr;
+  WH_HIP(hipMemcpyAsync(P.perm ? stage : db, b, sizeof(z64) * cin, hipMemcpyDefault, s));
+  if (P.perm) to_stick_order(K, P, stage, m, db);
+  WH_HIP(hipMemcpyAsync(P.perm ? stage : dx, x, sizeof(z64) * cin, hipMemcpyDefault, s));
+  if (P.perm) to_stick_order(K, P, stage, m, dx);
   double* de = K.w_ecol.as<double>(m);
   double* dep = K.w_epcol.as<double>(m);
   WH_HIP(hipMemcpyAsync(de, e, sizeof(double) * m, hipMemcpyDefault, s));
@@ -882,6 +1187,7 @@ int kpath_linsolve(int nbndval, int m, double* b, double* x, const double* e, co
   WH_HIP(hipMemcpyAsync(&nc, d_nonconv, sizeof(int), hipMemcpyDeviceToHost, s));
   WH_HIP(hipStreamSynchronize(s));
   cg_k_count(rec, last);
+  if (P.perm) dx = to_caller_order(K, P, dx, m, stage);
   WH_HIP(hipMemcpyAsync(x, dx, sizeof(z64) * cin, hipMemcpyDefault, s));
   finish();
   if (ierr) *ierr = nc;
@@ -1029,6 +1335,9 @@ int wh_set_kgrid(int nr1, int nr2, int nr3, double omega, const double* vrs, int
     std::vector<double> v(nnr);
     WH_HIP(hipMemcpy(v.data(), vrs, sizeof(double) * nnr, hipMemcpyDefault));
     K->vrs = upload(*K, v.data(), v.size());
+    // stick order beyond the LDS grids (an axis of three or more radices has no z kernel)
+    K->sticks_want = ksticks_enabled() && kz_available(nr3) &&
+                     !(klds_enabled() && kvloc_lds_available(nr1, nr2, nr3));
     K->k.resize(nks);
     K->q.resize(nqs);
   } catch (...) {
@@ -1052,8 +1361,10 @@ int wh_set_kpoint(int ik, int npw, const int* nl, const double* g2kin, const dou
   WH_HIP(hipStreamSynchronize(ctx().stream));
   KPointDev& P = K.k[ik - 1];
   for (void* p : {static_cast<void*>(P.nl), static_cast<void*>(P.g2kin), static_cast<void*>(P.q2),
-                  static_cast<void*>(P.d_et), static_cast<void*>(P.d_eprec)})
+                  static_cast<void*>(P.d_et), static_cast<void*>(P.d_eprec), static_cast<void*>(P.perm)})
     release(K, p);
+  P.perm = nullptr;
+  K.sticks_built = false;
   const long nnr = K.fft.nnr();
   std::vector<int> hnl(npw);
   std::vector<double> hg2(npw);
@@ -1066,6 +1377,45 @@ int wh_set_kpoint(int ik, int npw, const int* nl, const double* g2kin, const dou
   const int nb = K.nbndval;
   const int nq = nb + K.nkb;
   const size_t ld = K.npwx;
+  std::vector<int> perm(npw);
+  for (int ig = 0; ig < npw; ++ig) perm[ig] = ig;
+  P.col_i.clear();
+  P.col_j.clear();
+  if (K.sticks_want) {
+    const int n1 = K.fft.n1, n2 = K.fft.n2, n3 = K.fft.n3;
+    auto center = [](int v, int n) { return v > n / 2 ? v - n : v; };
+    std::vector<int> mi(npw), mj(npw), mk3(npw);
+    for (int ig = 0; ig < npw; ++ig) {
+      mi[ig] = center(hnl[ig] % n1, n1);
+      mj[ig] = center((hnl[ig] / n1) % n2, n2);
+      mk3[ig] = center(hnl[ig] / (n1 * n2), n3);
+    }
+    std::sort(perm.begin(), perm.end(), [&](int a, int b) {
+      if (mi[a] != mi[b]) return mi[a] < mi[b];
+      if (mj[a] != mj[b]) return mj[a] < mj[b];
+      return mk3[a] < mk3[b];
+    });
+    P.pt_col.assign(npw, 0);
+    P.pt_k.assign(npw, 0);
+    for (int q = 0; q < npw; ++q) {
+      const int g = perm[q];
+      if (q == 0 || mi[g] != P.col_i.back() || mj[g] != P.col_j.back()) {
+        P.col_i.push_back(mi[g]);
+        P.col_j.push_back(mj[g]);
+      }
+      P.pt_col[q] = static_cast<int>(P.col_i.size()) - 1;
+      P.pt_k[q] = mk3[g];
+    }
+    std::vector<int> nl2(npw);
+    std::vector<double> g22(npw);
+    for (int q = 0; q < npw; ++q) {
+      nl2[q] = hnl[perm[q]];
+      g22[q] = hg2[perm[q]];
+    }
+    hnl.swap(nl2);
+    hg2.swap(g22);
+    P.perm = upload(K, perm.data(), perm.size());
+  }
   std::vector<z64> q2(ld * 2 * std::max(nq, 1), mk(0.0, 0.0));
   P.et.assign(nb, 0.0);
   P.eprec.assign(nb, 0.0);
@@ -1076,7 +1426,7 @@ int wh_set_kpoint(int ik, int npw, const int* nl, const double* g2kin, const dou
     for (int v = 0; v < nb; ++v) {
       double ep = 0.0;
       for (int ig = 0; ig < npw; ++ig) {
-        const z64 a = h[v * ld + ig];
+        const z64 a = h[v * ld + perm[ig]];
         q2[v * ld + ig] = a;
         q2[(nb + v) * ld + ig] = mk(-a.y, a.x);
         ep += (a.x * a.x + a.y * a.y) * hg2[ig];
@@ -1089,7 +1439,7 @@ int wh_set_kpoint(int ik, int npw, const int* nl, const double* g2kin, const dou
     WH_HIP(hipMemcpy(h.data(), vkb, sizeof(z64) * h.size(), hipMemcpyDefault));
     for (int j = 0; j < K.nkb; ++j)
       for (int ig = 0; ig < npw; ++ig) {
-        const z64 a = h[j * ld + ig];
+        const z64 a = h[j * ld + perm[ig]];
         q2[(2 * nb + j) * ld + ig] = a;
         q2[(2 * nb + K.nkb + j) * ld + ig] = mk(-a.y, a.x);
       }
