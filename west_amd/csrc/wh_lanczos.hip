@@ -6,9 +6,9 @@
 // All NRHS chains run together: each Lanczos step is one application of H to
 // the NRHS current vectors (the Sternheimer operator's FFT and projector
 // kernels with e = 0 and alpha = 0), one deflation P_c = 1 - sum_v |psi_v><psi_v|
-// as a bra and a ket product, then per-column kernels for the three-term
-// recurrence, the modified Gram-Schmidt sweep over the earlier vectors and
-// the norm.  alpha, beta and the basis stay on the device until the end.
+// as a bra and a ket product, then one launch for the three-term recurrence,
+// the modified Gram-Schmidt sweep over the earlier vectors, the norm and the
+// next vector.  alpha, beta and the basis stay on the device until the end.
 #include <algorithm>
 
 #include "../../include/west_hip.h"
@@ -65,56 +65,200 @@ __global__ void k_lan_scale(int npw, const z64* r, const double* beta, z64* q, l
   q[static_cast<long>(ip) * ld + g] = mk<double>(v.x * inv, v.y * inv);
 }
 
-// r -= beta_prev q_prev (il > 1);  alpha = <q|r>;  r -= alpha q   (solve...ortho.f90:145-221)
-__global__ __launch_bounds__(NT) void k_lan_alpha(int npw, int gstart, z64* r, const z64* q, const z64* qprev,
-                                                  const double* beta_prev, double* alpha_out, long ld) {
-  __shared__ double red[NT / 64];
-  const int ip = blockIdx.x;
-  const long o = static_cast<long>(ip) * ld;
-  z64* ri = r + o;
-  const z64* qi = q + o;
-  double s = 0.0;
-  if (qprev) {
-    const double bp = beta_prev[ip];
-    const z64* pi = qprev + o;
-    for (int g = threadIdx.x; g < npw; g += NT) {
-      z64 v = ri[g];
-      v.x -= pi[g].x * bp;
-      v.y -= pi[g].y * bp;
-      ri[g] = v;
-      s += qi[g].x * v.x + qi[g].y * v.y;
+// The vector part of one Lanczos step, one workgroup per chain
+// (solve...ortho.f90:145-339): r -= beta_prev q_prev (il > 0); alpha = <q|r>,
+// r -= alpha q; the modified Gram-Schmidt sweep r -= <q_a|r> q_a over q_1 ..
+// q_{il-2}, one vector at a time; beta = |r|; and the next q = r / beta.
+//
+// The sweep is a serial chain of dot products and reads every earlier vector
+// of the chain once: 128 chains x 30 steps on 9,139 plane waves read 7.6 GB,
+// 1.7 ms at this card's copy rate.  r therefore stays in registers (NE
+// elements a thread) with the current vector beside it, and the next vector's
+// first PF elements are loaded while the dot product is reduced.  The whole
+// call on that case: one launch per vector with r in memory 27.2 ms (13.0 of
+// it in those), <18, 4> 14.4, <18, 8> 15.1 and <18, 18> 17.6 (registers spill),
+// each vector read twice instead of held 14.5, 1,024 threads 15.0 to 18.6.
+// Spheres beyond 18,432 points keep r in memory (k_lan_step_mem).
+constexpr int LNT = 512;
+
+struct LanArgs {
+  int npw, gstart, il;
+  z64* r;
+  const z64* q;            // the basis: block j at q + j blk
+  long blk, ld;
+  z64* qnext;              // null at the last step
+  const double* beta_prev;
+  double *alpha, *beta, *beta_s;
+};
+
+// red: two sets of one slot per wave, used in turn (one barrier per sum)
+__device__ __forceinline__ double lan_sum(double v, double (*red)[LNT / 64], int turn) {
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  if ((threadIdx.x & 63) == 0) red[turn & 1][threadIdx.x >> 6] = v;
+  __syncthreads();
+  double t = 0.0;
+#pragma unroll
+  for (int k = 0; k < LNT / 64; ++k) t += red[turn & 1][k];
+  return t;
+}
+
+// PF elements of the next vector are loaded ahead (0: each vector is read
+// twice, for the dot product and for the update, U elements at a time)
+template <int NE, int PF>
+__global__ __launch_bounds__(LNT) void k_lan_step(LanArgs A) {
+  __shared__ double red[2][LNT / 64];
+  constexpr int U = 6;
+  static_assert(PF <= NE && (PF > 0 || NE % U == 0), "vector split");
+  const int tid = threadIdx.x;
+  const long o = static_cast<long>(blockIdx.x) * A.ld;
+  const int npw = A.npw;
+  // Gamma weight of the thread's first element: G = 0 counts once, the others twice
+  const double w0 = (tid == 0 && A.gstart == 2) ? 0.5 : 1.0;
+  const z64* q = A.q + o;
+  const int nv = A.il;   // q_il (alpha), then q_0 .. q_{il-2}: max(1, il) vectors
+  auto vec = [&](int k) { return q + (k == 0 ? A.il : k - 1) * A.blk; };
+  // element tid + u LNT, 0 beyond npw: buffer loads bound by npw, one offset
+  // register for all of a thread's elements
+  auto at = [&](const z64* p, int u) {
+    const __amdgpu_buffer_rsrc_t rs =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<z64*>(p), 0, npw * static_cast<int>(sizeof(z64)), 0x00020000);
+    typedef unsigned int v4u __attribute__((ext_vector_type(4)));
+    const v4u w = __builtin_amdgcn_raw_buffer_load_b128(rs, tid * static_cast<int>(sizeof(z64)),
+                                                        u * LNT * static_cast<int>(sizeof(z64)), 0);
+    z64 v;
+    __builtin_memcpy(&v, &w, sizeof v);
+    return v;
+  };
+  z64 r[NE];
+#pragma unroll
+  for (int u = 0; u < NE; ++u) r[u] = at(A.r + o, u);
+  if (A.il > 0) {
+    const double bp = A.beta_prev[blockIdx.x];
+    const z64* p = q + (A.il - 1) * A.blk;
+#pragma unroll
+    for (int u = 0; u < NE; ++u) r[u] = r[u] - cscale(at(p, u), bp);
+  }
+  auto term = [&](z64 a, int u) {
+    const double x = a.x * r[u].x;
+    return (u == 0 ? w0 * x : x) + a.y * r[u].y;
+  };
+  if constexpr (PF > 0) {
+    z64 c[NE], n[PF];
+#pragma unroll
+    for (int u = 0; u < NE; ++u) c[u] = at(vec(0), u);
+    for (int k = 0; k == 0 || k < nv; ++k) {
+      const bool more = k + 1 < nv;
+      const z64* pn = vec(k + 1);
+      if (more) {
+#pragma unroll
+        for (int u = 0; u < PF; ++u) n[u] = at(pn, u);
+      }
+      double s = 0.0;
+#pragma unroll
+      for (int u = 0; u < NE; ++u) s += term(c[u], u);
+      const double t = 2.0 * lan_sum(s, red, k);
+      if (k == 0 && tid == 0) A.alpha[blockIdx.x] = t;
+#pragma unroll
+      for (int u = 0; u < NE; ++u) r[u] = r[u] - cscale(c[u], t);
+      if (more) {
+#pragma unroll
+        for (int u = 0; u < NE; ++u) c[u] = u < PF ? n[u < PF ? u : 0] : at(pn, u);
+      }
     }
   } else {
-    for (int g = threadIdx.x; g < npw; g += NT) s += qi[g].x * ri[g].x + qi[g].y * ri[g].y;
+    for (int k = 0; k == 0 || k < nv; ++k) {
+      const z64* p = vec(k);
+      double s = 0.0;
+#pragma unroll
+      for (int u0 = 0; u0 < NE; u0 += U) {
+        z64 c[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) c[u] = at(p, u0 + u);
+#pragma unroll
+        for (int u = 0; u < U; ++u) s += term(c[u], u0 + u);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      const double t = 2.0 * lan_sum(s, red, k);
+      if (k == 0 && tid == 0) A.alpha[blockIdx.x] = t;
+#pragma unroll
+      for (int u0 = 0; u0 < NE; u0 += U) {
+        z64 c[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) c[u] = at(p, u0 + u);
+#pragma unroll
+        for (int u = 0; u < U; ++u) r[u0 + u] = r[u0 + u] - cscale(c[u], t);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
   }
-  s = block_sum_l(s, red);
-  // element 0 was written by thread 0 itself
-  const double a = 2.0 * s - (gstart == 2 ? qi[0].x * ri[0].x : 0.0);
-  __syncthreads();
-  if (threadIdx.x == 0) alpha_out[ip] = a;
-  for (int g = threadIdx.x; g < npw; g += NT) {
-    z64 v = ri[g];
-    v.x -= qi[g].x * a;
-    v.y -= qi[g].y * a;
-    ri[g] = v;
+  double s = 0.0;
+#pragma unroll
+  for (int u = 0; u < NE; ++u) s += term(r[u], u);
+  const double b = sqrt(2.0 * lan_sum(s, red, nv > 0 ? nv : 1));
+  if (tid == 0) {
+    A.beta[blockIdx.x] = b;
+    A.beta_s[blockIdx.x] = b;
+  }
+  if (A.qnext) {
+    const double inv = 1.0 / b;
+    z64* qn = A.qnext + o;
+#pragma unroll
+    for (int u = 0; u < NE; ++u) {
+      const int g = tid + u * LNT;
+      if (g < npw) qn[g] = cscale(r[u], inv);
+    }
   }
 }
 
-// one modified Gram-Schmidt step: t = <q_a|r>; r -= t q_a   (solve...ortho.f90:225-287)
-__global__ __launch_bounds__(NT) void k_lan_mgs(int npw, int gstart, z64* r, const z64* qa, long ld) {
-  __shared__ double red[NT / 64];
-  const int ip = blockIdx.x;
-  const long o = static_cast<long>(ip) * ld;
-  z64* ri = r + o;
-  const z64* ai = qa + o;
-  const double t = gamma_dot(ai, ri, npw, gstart, red);
-  __syncthreads();
-  for (int g = threadIdx.x; g < npw; g += NT) {
-    z64 v = ri[g];
-    v.x -= ai[g].x * t;
-    v.y -= ai[g].y * t;
-    ri[g] = v;
+// the same with r in memory
+__global__ __launch_bounds__(LNT) void k_lan_step_mem(LanArgs A) {
+  __shared__ double red[2][LNT / 64];
+  const int tid = threadIdx.x;
+  const long o = static_cast<long>(blockIdx.x) * A.ld;
+  const int npw = A.npw;
+  z64* r = A.r + o;
+  const z64* q = A.q + o;
+  const double bp = A.il > 0 ? A.beta_prev[blockIdx.x] : 0.0;
+  const int nv = A.il;
+  for (int k = 0; k == 0 || k < nv; ++k) {
+    const z64* c = q + (k == 0 ? A.il : k - 1) * A.blk;
+    const z64* p = k == 0 && A.il > 0 ? q + (A.il - 1) * A.blk : nullptr;
+    double s = 0.0;
+    for (int g = tid; g < npw; g += LNT) {
+      z64 v = r[g];
+      if (p) {
+        v = v - cscale(p[g], bp);
+        r[g] = v;
+      }
+      const double x = c[g].x * v.x;
+      s += (g == 0 && A.gstart == 2 ? 0.5 * x : x) + c[g].y * v.y;
+    }
+    const double t = 2.0 * lan_sum(s, red, k);
+    if (k == 0 && tid == 0) A.alpha[blockIdx.x] = t;
+    for (int g = tid; g < npw; g += LNT) r[g] = r[g] - cscale(c[g], t);
   }
+  double s = 0.0;
+  for (int g = tid; g < npw; g += LNT) {
+    const double x = r[g].x * r[g].x;
+    s += (g == 0 && A.gstart == 2 ? 0.5 * x : x) + r[g].y * r[g].y;
+  }
+  const double b = sqrt(2.0 * lan_sum(s, red, nv > 0 ? nv : 1));
+  if (tid == 0) {
+    A.beta[blockIdx.x] = b;
+    A.beta_s[blockIdx.x] = b;
+  }
+  if (A.qnext)
+    for (int g = tid; g < npw; g += LNT) A.qnext[o + g] = cscale(r[g], 1.0 / b);
+}
+
+void lan_step(int nrhs, const LanArgs& a, hipStream_t s) {
+  const int ne = ceil_div(a.npw, LNT);
+  if (ne <= 4) k_lan_step<4, 4><<<nrhs, LNT, 0, s>>>(a);
+  else if (ne <= 9) k_lan_step<9, 9><<<nrhs, LNT, 0, s>>>(a);
+  else if (ne <= 18) k_lan_step<18, 4><<<nrhs, LNT, 0, s>>>(a);
+  else if (ne <= 36) k_lan_step<36, 0><<<nrhs, LNT, 0, s>>>(a);
+  else k_lan_step_mem<<<nrhs, LNT, 0, s>>>(a);
+  WH_HIP(hipGetLastError());
 }
 
 }  // namespace
@@ -168,10 +312,10 @@ extern "C" int wh_solve_deflated_lanczos_w_full_ortho(int nbnd_to_deflate, int n
     // r -> q & beta (76-112)
     k_lan_norm<<<nrhs, NT, 0, s>>>(npw, c.gstart, R, ld, d_beta, d_bnorm);
     WH_HIP(hipGetLastError());
+    k_lan_scale<<<dim3(ceil_div(npw, NT), nrhs), NT, 0, s>>>(npw, R, d_beta, Q, ld);
+    WH_HIP(hipGetLastError());
     for (int il = 0; il < nlsteps; ++il) {
       z64* qi = Q + static_cast<size_t>(il) * blk;
-      k_lan_scale<<<dim3(ceil_div(npw, NT), nrhs), NT, 0, s>>>(npw, R, d_beta, qi, ld);
-      WH_HIP(hipGetLastError());
       // r = H q  (h_psi_: the operator with e = 0, alpha = 0), then r = P_c r (144-145)
       stern_apply(qi, R, d_e0, nrhs, 0.0);
       if (nbnd_to_deflate > 0) {
@@ -179,16 +323,12 @@ extern "C" int wh_solve_deflated_lanczos_w_full_ortho(int nbnd_to_deflate, int n
         WH_TIMED("gemm_ket", dgemm(false, static_cast<int>(k2), nrhs, nbnd_to_deflate, -1.0, q, k2, cm,
                                    nbnd_to_deflate, 1.0, reinterpret_cast<double*>(R), k2, s));
       }
-      k_lan_alpha<<<nrhs, NT, 0, s>>>(npw, c.gstart, R, qi, il > 0 ? qi - blk : nullptr, d_beta,
-                                     d_alpha + static_cast<size_t>(il) * nrhs, ld);
-      WH_HIP(hipGetLastError());
-      // full re-orthogonalisation against q_1 .. q_{il-2} (225-287), one vector at a time
-      for (int ia = 0; ia + 1 < il; ++ia) {
-        k_lan_mgs<<<nrhs, NT, 0, s>>>(npw, c.gstart, R, Q + static_cast<size_t>(ia) * blk, ld);
-        WH_HIP(hipGetLastError());
-      }
-      k_lan_norm<<<nrhs, NT, 0, s>>>(npw, c.gstart, R, ld, d_beta, d_beta_s + static_cast<size_t>(il) * nrhs);
-      WH_HIP(hipGetLastError());
+      const size_t row = static_cast<size_t>(il) * nrhs;
+      WH_TIMED("lanczos_step", lan_step(nrhs,
+                                        LanArgs{npw, c.gstart, il, R, Q, static_cast<long>(blk), ld,
+                                                il + 1 < nlsteps ? qi + blk : nullptr, d_beta, d_alpha + row, d_beta,
+                                                d_beta_s + row},
+                                        s));
     }
     // outputs in the reference's layouts: alpha_s(NLSTEPS, NRHS), beta_s(NLSTEPS-1, NRHS),
     // q_s(npwx, NRHS, NLSTEPS), bnorm(NRHS)
