@@ -1,5 +1,5 @@
-"""The q-point path on grids beyond the LDS (stick transforms, one CG over the
-columns of every k point) against the oracle: the operator and the CG at each
+"""The q-point path on grids beyond the LDS (stick transforms or the fused
+iteration, one CG over the columns of every k point) against the oracle: the operator and the CG at each
 k point, chi0(q) with all k points in one solve and one after another, and a
 grid whose planes take the two-radix kernels or the compiled ones."""
 import numpy as np
@@ -22,8 +22,10 @@ def _smooth(n, npwx, m, g2, seed):
 
 
 # (30, 25, 27): n1 != n2; (27, 20, 20): an odd length; (25, 25, 30) n1 = n2 not
-# compiled; (30, 30, 18): n1 = n2 compiled
+# compiled; (30, 30, 18): n1 = n2 compiled; (24, 24, 20): the fused CG
+# iteration, whose rows fit the LDS where the whole grid does not
 CASES = {"n30x25x27": ((9.0, 7.8, 8.4), (2, 1, 1)), "n27x20x20": ((8.4, 5.9, 5.9), (3, 1, 1)),
+         "n24x24x20": ((7.2, 7.2, 5.9), (2, 1, 1)),
          "n25x25x30": ((7.8, 7.8, 9.0), (1, 2, 1)), "n30x30x18": ((9.0, 9.0, 5.3), (1, 1, 2))}
 
 

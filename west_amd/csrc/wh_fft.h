@@ -90,7 +90,8 @@ struct StickPlan {
   void build(int nr1, int nr2, int nr3, int npw, const int* nl_1based, const int* nlm_1based);
   // Plane part only, for complex functions with the given columns (i, j): no
   // mirror columns and no points (k points: wh_kfft_sticks.hip's z kernels
-  // bring their own).  False where the grid has neither tpl nor rect kernels.
+  // bring their own).  False where the grid has neither tpl nor rect kernels;
+  // dev.nct is 0 where the columns do not fit the grid.
   bool build_columns(int nr1, int nr2, int nr3, const std::vector<int>& ci, const std::vector<int>& cj);
   void release();
   long sticks_elems() const { return static_cast<long>(dev.n3) * dev.nct; }
@@ -185,12 +186,6 @@ void launch_grid_fft(const GridFft& g, z64* data, int batch, int dir, hipStream_
 bool kvloc_lds_available(int n1, int n2, int n3);
 void kvloc_lds(int n1, int n2, int n3, int m, int npw, long ld, const int* nl, const z64* x, const double* vrs,
                const double* g2, const double* e, z64* t, hipStream_t s, const int* d_m = nullptr);
-// One CG iteration of the k-point Sternheimer solve per listed column (lb <
-// *nc of cap launched; band l2i[lb]) in one workgroup with the grid in LDS:
-// direction h = -h + beta hold (bc = h), t = (H_k - eu + projectors) h with
-// the local term in LDS and the projector block q2 (real view, 2 ld rows,
-// nq2 <= 32 columns, row scales qs), the CG step on x, g, hold, and the next
-// preconditioned residual h and rho[band] (wh_kfft_lds.hip)
 // Columns of several k points in one launch: ktab (device, may be null) holds
 // each k point's sphere and projectors, and band column col belongs to k point
 // col / cols_per_k (ktab null: npw, nl, g2 and q2 for every column).
@@ -202,7 +197,34 @@ struct KlKpoint {
   const double* et;      // nbndval energies
   const double* eprec;   // nbndval preconditioner energies
 };
-bool cg_iter_lds_available(int n1, int n2, int n3, int nq2);
+// One CG iteration of the k-point Sternheimer solve per listed column (lb <
+// *nc of the launched ones; band l2i[lb]) in one workgroup (wh_kfft_lds.hip):
+// direction h = -h + beta hold (bc = h), t = (H_k - eu + projectors) h with
+// the local term in LDS and the projector block q2 (real view, 2 ld rows,
+// nq2 <= 32 columns, row scales qs), the CG step on x, g, hold, and the next
+// preconditioned residual h and rho[band]
+struct KlCgArgs {
+  long ld;
+  const double* vrs;   // [a3][a1][a2]
+  int nq2;
+  const double* q2;
+  const double* qs;
+  const int* l2i;
+  const int* nc;
+  const double* beta;
+  const double* eu;
+  const double* ep;
+  z64* h;
+  z64* hold;
+  z64* x;
+  z64* g;
+  z64* bc;
+  z64* tc;
+  double* rho;
+  const KlKpoint* ktab;
+  int cols_per_k;
+  const z64* b;   // FIRST: the right-hand sides
+};
 // The grids of dfpt at q on LDS grids for every k point in one launch each
 // (kvloc_lds_available grids; qtab: per k point its k - q index and g0):
 // states_kmq_lds: psik[k][v] = F^-1[evc_v at k - q] exp(-i g0.r) (nks nb grids);
@@ -220,22 +242,11 @@ void states_kmq_lds(int n1, int n2, int n3, int nks, int nb, long ld, const KlKp
 // dfpt_module.f90:346) and x = f / max(1, |k+G|^2 / ep) (348)
 void pc_precond_all(int nks, int nb, int m, long ld, const KlKpoint* ktab, const KlQpoint* qtab, z64* f, z64* x,
                     double* e, double* ep, hipStream_t s);
-// The CG's first step for m = nks cols columns of cg_iter_lds's kind
-// (linsolve_sternheimer_m_wfcts.f90:127-205): g = (H_k - e + alpha P_v) x - b
-// with the local term in LDS, h = g / max(1, |k+G|^2 / eprec), rho[col] = Re <h|g>
-void cg_first_lds(int n1, int n2, int n3, long ld, const double* vrs, int nq2, const double* qs, int m,
-                  const double* e, const double* ep, const z64* x, const z64* b, z64* g, z64* h, double* rho,
-                  const KlKpoint* ktab, int cols_per_k, hipStream_t s);
 void rhs_lds(int n1, int n2, int n3, int nks, int nb, int m, long ld, const KlKpoint* ktab, const z64* psik,
              const z64* aux, z64* out, hipStream_t s);
 void density_lds(int n1, int n2, int n3, int nks, int nb, int m, long ld, const KlKpoint* ktab, const z64* psik,
                  const z64* dpsi, z64* dsc, int npwq, long ldq, const int* nlq, const double* sck, z64* dk, z64* dng,
                  hipStream_t s);
-void cg_iter_lds(int n1, int n2, int n3, int npw, long ld, const int* nl, const double* vrs, const double* g2,
-                 int nq2, const double* q2, const double* qs, int cap, const int* l2i, const int* nc,
-                 const double* beta, const double* eu, const double* ep, z64* h, z64* hold, z64* x, z64* g, z64* bc,
-                 z64* tc, double* rho, hipStream_t s, const KlKpoint* ktab = nullptr, int cols_per_k = 1);
-
 // Local term at k points through sticks (wh_kfft_sticks.hip): the columns are
 // those of a StickPlan::build_columns plan that holds every k sphere, the
 // points of k point k lie in column order (col_off: n columns + 1).  Band
@@ -255,6 +266,14 @@ void launch_kzinv(const StickPlan& p, const KStick* tab, const int* l2i, int col
 // t = sphere part of the sticks' forward transform + (g2 - e[b]) x, zero beyond npw
 void launch_kzfwd(const StickPlan& p, const KStick* tab, const int* l2i, int cols_per_k, int c0, int n,
                   const int* d_nc, const z64* sticks, const z64* x, const double* e, z64* t, long ld, hipStream_t s);
+
+// The fused CG iteration (wh_kfft_lds.hip): workgroups a CU holds for a
+// StickPlan::build_columns plan (0: no kernel for the grid, or more than 32
+// projector rows), and one iteration (first: the CG's first step, g = A x - b,
+// h and rho for every column) of m launched columns; stab as in KStick (the
+// column's k point's entry where a.ktab is null)
+int cg_iter_wgs(const StickPlan& p, int nq2);
+void cg_iter_rows(const StickPlan& p, const KStick* stab, bool first, int m, const KlCgArgs& a, hipStream_t s);
 
 // kernel launchers (double precision)
 void launch_zinv(const StickPlan& p, const FftItem* d_items, int nitems, const z64* psi, long ldpsi,

@@ -699,6 +699,9 @@ bool StickPlan::build_columns(int nr1, int nr2, int nr3, const std::vector<int>&
     d.jext = std::max(d.jext, std::abs(cj[c]));
   }
   d.nrows = 2 * d.imax + 1;
+  tpl = tplz = nullptr;
+  tpl32 = nullptr;
+  rect = RectPlan{};
   if (d.nrows > nr1 || 2 * d.jext + 1 > nr2) return false;
   d.n1 = nr1; d.n2 = nr2; d.n3 = nr3;
   d.ncs = d.nct = n;
@@ -714,9 +717,6 @@ bool StickPlan::build_columns(int nr1, int nr2, int nr3, const std::vector<int>&
   d.tw2 = upload_twiddles(nr2, allocations);
   d.tw3 = upload_twiddles(nr3, allocations);
   tpl = tpl_kernels_f64(dev);
-  tplz = nullptr;
-  tpl32 = nullptr;
-  rect = RectPlan{};
   if (!tpl) rect_plan(dev, rect);
   vloc_occ = 0;
   return tpl || rect.ok;

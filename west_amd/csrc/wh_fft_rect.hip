@@ -22,35 +22,16 @@
 #include <map>
 #include <mutex>
 
-#include "wh_fft_pass2.h"
 #include "wh_fft_rect.h"
+#include "wh_fft_rect_dev.h"
 
 namespace wh {
 
 namespace {
 
-struct RectLds {
-  z64* tw1;
-  z64* tw2;
-  z64* pl;   // [pz][nrows][rs2]
-  z64* wa;   // a1 lines [nj][xs]
-  double* acc;   // density: [n1][n2]
-};
-
-template <int NT>
-__device__ __forceinline__ RectLds rect_lds(const StickPlanDev& P, const RectPlan& Q, int pz) {
+__device__ __forceinline__ z64* rect_base() {
   extern __shared__ char smem_raw[];
-  RectLds S;
-  S.tw1 = reinterpret_cast<z64*>(smem_raw);
-  S.tw2 = S.tw1 + P.n1;
-  S.pl = S.tw2 + P.n2;
-  S.wa = S.pl + pz * P.nrows * Q.rs2;
-  S.acc = reinterpret_cast<double*>(S.wa + Q.nj * Q.xs);
-  const z64* t1 = reinterpret_cast<const z64*>(P.tw1);
-  const z64* t2 = reinterpret_cast<const z64*>(P.tw2);
-  for (int t = threadIdx.x; t < P.n1; t += NT) S.tw1[t] = t1[t];
-  for (int t = threadIdx.x; t < P.n2; t += NT) S.tw2[t] = t2[t];
-  return S;
+  return reinterpret_cast<z64*>(smem_raw);
 }
 
 // nz planes of sticks into zeroed rows
@@ -69,29 +50,6 @@ __device__ __forceinline__ void rect_fill(const StickPlanDev& P, const RectPlan&
   __syncthreads();
 }
 
-// a2 transforms of the rows in place, Q.nrc rows at a time
-template <int NT, int DIR>
-__device__ __forceinline__ void rect_rows(const StickPlanDev& P, const RectPlan& Q, const RectLds& S, int nrow_all) {
-  const int rs = Q.rs2;
-  for (int q0 = 0; q0 < nrow_all; q0 += Q.nrc) {
-    const int nl = min(Q.nrc, nrow_all - q0);
-    z64* rows = S.pl + q0 * rs;
-    auto ld = [=](int l, int x) { return rows[l * rs + x]; };
-    auto st = [=](int l, int x, z64 v) { rows[l * rs + x] = v; };
-    pass2<NT, DIR, PASS_FIRST, true>(nl, Q.r20, Q.r21, S.tw2, ld, no_mid, st);
-    __syncthreads();
-    pass2<NT, DIR, PASS_LAST, false>(nl, Q.r21, Q.r20, S.tw2, ld, no_mid, st);
-  }
-  __syncthreads();
-}
-
-// row of the sphere holding a1-frequency x, or -1
-__device__ __forceinline__ int rect_row(int x, int n1, int imax) {
-  if (x <= imax) return x + imax;
-  if (x >= n1 - imax) return x - n1 + imax;
-  return -1;
-}
-
 // sticks -> (V(r) * .) -> sticks
 template <int NT>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_rect_vloc(
@@ -102,44 +60,14 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
   const int z0 = blockIdx.x * Q.pz;
   const int nz = min(Q.pz, P.n3 - z0);
   const long sl = static_cast<long>(P.n3) * P.nct;
-  const RectLds S = rect_lds<NT>(P, Q, Q.pz);
+  const RectLds S = rect_lds<NT>(P, Q, Q.pz, rect_base());
   rect_fill<NT>(P, Q, S, sin + static_cast<long>(item.a) * sl + static_cast<long>(z0) * P.nct, nz);
-  rect_rows<NT, +1>(P, Q, S, nz * P.nrows);
-  const int n1 = P.n1, n2 = P.n2, imax = P.imax, rs = Q.rs2, xs = Q.xs, pe = P.nrows * rs;
-  const float inv_n2 = Q.inv_n2;
-  z64 *wa = S.wa, *pl = S.pl;
   const double* V = vpot + (item.pot >= 0 ? static_cast<long>(item.pot) * ldpot : 0L) +
-                    static_cast<long>(z0) * n1 * n2;
-  // a1 lines (plane p, second-axis position y): Q.nj at a time
-  for (int l0 = 0; l0 < nz * n2; l0 += Q.nj) {
-    const int nl = min(Q.nj, nz * n2 - l0);
-    auto col = [=](int l) {
-      const int p = fdiv(l0 + l, inv_n2);
-      return pl + p * pe + (l0 + l - p * n2);
-    };
-    auto in_wa = [=](int l, int x) { return wa[l * xs + x]; };
-    auto to_wa = [=](int l, int x, z64 v) { wa[l * xs + x] = v; };
-    pass2<NT, +1, PASS_FIRST, false>(nl, Q.r10, Q.r11, S.tw1,
-                                 [=](int l, int x) {
-                                   const int r = rect_row(x, n1, imax);
-                                   return r >= 0 ? col(l)[r * rs] : mk(0.0, 0.0);
-                                 },
-                                 no_mid, to_wa);
-    __syncthreads();
-    pass2<NT, +1, PASS_TURN, true>(nl, Q.r11, Q.r10, S.tw1, in_wa,
-                               [=](int l, int x, z64 v) {
-                                 const int p = fdiv(l0 + l, inv_n2);
-                                 return cscale(v, V[(p * n1 + x) * n2 + (l0 + l - p * n2)] * scale);
-                               },
-                               to_wa);
-    __syncthreads();
-    pass2<NT, -1, PASS_LAST, false>(nl, Q.r10, Q.r11, S.tw1, in_wa, no_mid, [=](int l, int x, z64 v) {
-      const int r = rect_row(x, n1, imax);
-      if (r >= 0) col(l)[r * rs] = v;
-    });
-    __syncthreads();
-  }
-  rect_rows<NT, -1>(P, Q, S, nz * P.nrows);
+                    static_cast<long>(z0) * P.n1 * P.n2;
+  rect_local<NT>(P, Q, S, nz, V, scale);
+  const int n2 = P.n2, rs = Q.rs2, pe = P.nrows * rs;
+  const float inv_n2 = Q.inv_n2;
+  const z64* pl = S.pl;
   z64* dst = sout + static_cast<long>(blockIdx.y) * sl + static_cast<long>(z0) * P.nct;
   for (int p = 0; p < nz; ++p)
     for (int c = threadIdx.x; c < P.nct; c += NT) {
@@ -177,7 +105,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
   const FftItem item = items[blockIdx.y];
   if (item.a < 0) return;   // inactive item (uniform per workgroup)
   const long sl = static_cast<long>(P.n3) * P.nct;
-  const RectLds S = rect_lds<NT>(P, Q, 1);
+  const RectLds S = rect_lds<NT>(P, Q, 1, rect_base());
   rect_fill<NT>(P, Q, S, sin + static_cast<long>(blockIdx.y) * sl + static_cast<long>(z) * P.nct, 1);
   rect_rows<NT, +1>(P, Q, S, P.nrows);
   const long o = static_cast<long>(z) * P.n1 * P.n2;
@@ -198,7 +126,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4))) void k_
   const int z = blockIdx.x;
   const int pp = blockIdx.y;
   const long sl = static_cast<long>(P.n3) * P.nct;
-  const RectLds S = rect_lds<NT>(P, Q, 1);
+  const RectLds S = rect_lds<NT>(P, Q, 1, rect_base());
   const int n1 = P.n1, n2 = P.n2, imax = P.imax, rs = Q.rs2, xs = Q.xs;
   double* acc = S.acc;
   for (int t = threadIdx.x; t < n1 * n2; t += NT) acc[t] = 0.0;

@@ -6,7 +6,8 @@
 //   k_gather, which make six launches and six HBM round trips of the grid);
 // * one CG iteration of the Sternheimer solve per column (direction, the
 //   operator with its projectors, CG step, next preconditioned residual), and
-//   its first step, over the columns of one k point or of every k point;
+//   its first step, over the columns of one k point or of every k point (this
+//   one with the rows of the sphere in LDS, not the whole grid);
 // * the states at k - q, the right-hand sides and the response densities of
 //   dfpt at q for every k point, and -P_c with M^-1 on the right-hand sides.
 // Each 1D pass gives one line to one thread, transformed in registers with a
@@ -35,8 +36,17 @@ constexpr bool kl_size(int n) {
 #undef WH_KL_CASE
 }
 
+// the value, hidden from the optimiser: the products with each element index of
+// every compiled length would otherwise be formed ahead of the line loops and
+// spill hundreds of scalar registers
+__device__ __forceinline__ int kl_opaque(int v) {
+  asm volatile("" : "+s"(v));
+  return v;
+}
+
 template <int NL, int DIR>
 __device__ __forceinline__ void kl_line(z64* p, int stride) {
+  stride = kl_opaque(stride);
   z64 v[NL];
 #pragma unroll
   for (int i = 0; i < NL; ++i) v[i] = p[i * stride];
@@ -48,6 +58,7 @@ __device__ __forceinline__ void kl_line(z64* p, int stride) {
 // inverse, times V(r) (vr: the line's potential, stride vs), forward
 template <int NL>
 __device__ __forceinline__ void kl_line_vloc(z64* p, int stride, const double* vr, long vs) {
+  stride = kl_opaque(stride);
   z64 v[NL];
 #pragma unroll
   for (int i = 0; i < NL; ++i) v[i] = p[i * stride];
@@ -60,7 +71,7 @@ __device__ __forceinline__ void kl_line_vloc(z64* p, int stride, const double* v
 }
 
 template <int DIR>
-__device__ void kl_pass(int n, z64* p, int stride) {
+__device__ __forceinline__ void kl_pass(int n, z64* p, int stride) {
   switch (n) {
 #define WH_KL_CASE(NN)          \
   case NN:                      \
@@ -173,7 +184,7 @@ __global__ __launch_bounds__(KL_NT) void k_kvloc_lds(int n1, int n2, int n3, int
   }
 }
 
-// sum over the workgroup of NV values per thread (NV <= KL_NQ2); every
+// sum over the workgroup of nv values per thread (nv <= KL_NQ2); every
 // thread gets the sums in out[] (LDS)
 constexpr int KL_NQ2 = 32;   // projector rows (real view) the fused CG iteration takes
 __device__ __forceinline__ void kl_block_sums(double* v, int nv, double (*red)[KL_NT / 64], double* out) {
@@ -198,48 +209,117 @@ __device__ __forceinline__ void kl_block_sums(double* v, int nv, double (*red)[K
 }
 
 // One CG iteration of the Sternheimer solve at a k point for listed column
-// lb < *nc (band col = l2i[lb]), one workgroup per column, the grid in LDS:
+// lb < *nc (band col = l2i[lb]), one workgroup per column:
 //   h = -h + beta hold, bc = h                                (226-240)
-//   t = (H_k - e + alpha P_v) h: local term on the LDS grid, |k+G|^2 - e,
+//   t = (H_k - e + alpha P_v) h: local term in LDS, |k+G|^2 - e,
 //       and t += Q2 (s * (Q2^T h)) in the real view of the projectors  (251)
 //   a = Re <h|g>, c = Re <h|t>; x -= a/c h, g -= a/c t, hold = h  (253-321)
 //   h = g / max(1, g2kin/eprec), rho[col] = Re <h|g> (the next 150-205)
 // q2: real view of the projector block (2 ld rows, nq2 columns), qs: its
-// row scales.  Each thread keeps the plane waves ig = tid + k KL_NT in every
+// row scales.  Each thread keeps the plane waves ig = tid + k NT in every
 // phase, so the values it writes to bc and tc it reads back itself.
-struct KlCgArgs {
-  int n1, n2, n3, p1, npw;
-  long ld;
-  const int* nl;
-  const double* vrs;
-  const double* g2;
-  int nq2;
-  const double* q2;
-  const double* qs;
-  const int* l2i;
-  const int* nc;
-  const double* beta;
-  const double* eu;
-  const double* ep;
-  z64* h;
-  z64* hold;
-  z64* x;
-  z64* g;
-  z64* bc;
-  z64* tc;
-  double* rho;
-  const KlKpoint* ktab;
-  int cols_per_k;
-  const z64* b;   // FIRST: the right-hand sides
-};
-
+//
+// LDS holds only the rows |i| <= imax of the grid, [i][a3][a2]: about half of
+// it (24 x 20 x 18: 11 of 24 rows, 66 KB), so two workgroups share a CU.  The
+// a3 lines of the columns that hold points, the a2 lines of the rows, and
+// the a1 lines -- zero-padded from the rows in registers, V(r) between their
+// inverse and forward transforms -- are one line per thread each, so five
+// passes and as many barriers make the local term.  Bound by FP64 issue and
+// the passes' latency: 864 columns of that grid take 62 us an iteration (with
+// the whole grid in LDS, every line transformed, one workgroup a CU: 145; with
+// the columns' sticks in LDS and the planes in batches through two-radix
+// passes, 85 barriers: 138).  256 threads may use 256 registers each, which a
+// 24-point line with V(r) needs; 320 and 384 threads spill (chi0 of that case
+// 2.3 ms against 3.3 and 3.9).
 // FIRST: the CG's first step instead (127-205), every launched column in
 // order (col = lb, eu = e by column): the operator acts on x, then
 // g = A x - b, h = g / max(1, g2kin/eprec), rho[col] = Re <h|g>.
+struct KlRows {
+  int n1, n2, n3, imax, nct, p2;   // p2: odd pitch along a2
+  const int* col_pos;              // (i + imax) n2 + (j mod n2) of each column
+};
+
+// widest |i| the a1 lines take: the sphere spans at most (n + 1) / 4 either
+// way, and the k point less than one more
+constexpr int kl_row_bound(int n) { return n / 4 + 1; }
+
+// a1 line from and to the rows: v(x) at p[(x or x - n1) rs], |x| <= imax
+// (elements beyond kl_row_bound are known zeros)
+template <int N>
+__device__ __forceinline__ void kl_line_rows(z64* p, int rs, int imax, const double* vr, int vs, double sc) {
+  constexpr int BX = kl_row_bound(N);
+  rs = kl_opaque(rs);
+  imax = kl_opaque(imax);
+  vs = kl_opaque(vs);
+  z64 v[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    if (i > BX && i < N - BX) {
+      v[i] = mk(0.0, 0.0);
+    } else {
+      // (a load that is always in range, then the choice: no branch per element)
+      const int f = i <= BX ? i : i - N;
+      const z64 w = p[max(min(f, imax), -imax) * rs];
+      v[i] = f <= imax && f >= -imax ? w : mk(0.0, 0.0);
+    }
+  }
+  fft_line<double, N, +1>(v);
+  // V(r) is loaded here, not ahead of the inverse transform (register pressure)
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int i = 0; i < N; ++i) v[i] = cscale(v[i], vr[i * vs] * sc);
+  fft_line<double, N, -1>(v);
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+    if (i <= BX || i >= N - BX) {
+      const int f = i <= BX ? i : i - N;
+      if (f <= imax && f >= -imax) p[f * rs] = v[i];
+    }
+}
+
+__device__ __forceinline__ void kl_pass_rows(int n, z64* p, int rs, int imax, const double* vr, int vs, double sc) {
+  switch (n) {
+#define WH_KL_CASE(NN)                                 \
+  case NN:                                             \
+    kl_line_rows<NN>(p, rs, imax, vr, vs, sc);         \
+    break;
+    WH_KL_SIZES(WH_KL_CASE)
+#undef WH_KL_CASE
+    default: break;
+  }
+}
+
+template <int NT, int MAXV>
+__device__ __forceinline__ void kl_sums(const double* v, int nv, double (*red)[NT / 64], double* out) {
+  const int lane = threadIdx.x & 63;
+  const int w = threadIdx.x >> 6;
+#pragma unroll
+  for (int i = 0; i < MAXV; ++i) {
+    if (i < nv) {
+      double x = v[i];
+      for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
+      if (lane == 0) red[i][w] = x;
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x < nv) {
+    double x = 0.0;
+#pragma unroll
+    for (int q = 0; q < NT / 64; ++q) x += red[threadIdx.x][q];
+    out[threadIdx.x] = x;
+  }
+  __syncthreads();
+}
+
+constexpr int KR_NT = 256;
+
 template <bool FIRST>
-__global__ __launch_bounds__(KL_NT) void k_cg_iter_lds(KlCgArgs a) {
+__global__ __launch_bounds__(KR_NT) __attribute__((amdgpu_waves_per_eu(2))) void k_cg_iter_rows(KlRows R,
+                                                                                             const KStick* stab,
+                                                                                             KlCgArgs a) {
+  constexpr int NT = KR_NT;
   extern __shared__ char smem_raw[];
-  __shared__ double red[KL_NQ2][KL_NT / 64];
+  __shared__ double red[KL_NQ2][NT / 64];
   __shared__ double sums[KL_NQ2];
   __shared__ double c2s[KL_NQ2];
   z64* grid = reinterpret_cast<z64*>(smem_raw);
@@ -248,17 +328,10 @@ __global__ __launch_bounds__(KL_NT) void k_cg_iter_lds(KlCgArgs a) {
   if (!FIRST && lb >= *a.nc) return;   // whole workgroup
   const int col = FIRST ? lb : a.l2i[lb];
   const long ld = a.ld;
-  int npw = a.npw;
-  const int* nl = a.nl;
-  const double* g2 = a.g2;
-  const double* q2 = a.q2;
-  if (a.ktab) {   // the column's k point
-    const KlKpoint kp = a.ktab[col / a.cols_per_k];
-    npw = kp.npw;
-    nl = kp.nl;
-    g2 = kp.g2;
-    q2 = kp.q2;
-  }
+  const int ik = a.ktab ? col / a.cols_per_k : 0;
+  const KStick K = stab[ik];
+  const double* q2 = a.ktab ? a.ktab[ik].q2 : a.q2;
+  const int npw = K.npw;
   const int nq2 = a.nq2;
   const long ldr = 2 * ld;   // real view
   z64* hc = a.h + col * ld;
@@ -267,15 +340,24 @@ __global__ __launch_bounds__(KL_NT) void k_cg_iter_lds(KlCgArgs a) {
   z64* ho = FIRST ? nullptr : a.hold + col * ld;
   z64* bb = FIRST ? nullptr : a.bc + lb * ld;
   z64* tt = FIRST ? nullptr : a.tc + lb * ld;
-  const int np = a.p1 * a.n2 * a.n3;
-  for (int i = tid; i < np; i += KL_NT) grid[i] = mk(0.0, 0.0);
+  const int n1 = R.n1, n2 = R.n2, n3 = R.n3, p2 = R.p2, imax = R.imax;
+  const int nrows = 2 * imax + 1;
+  const int rs = n3 * p2;   // row stride
+  for (int i = tid; i < nrows * rs; i += NT) grid[i] = mk(0.0, 0.0);
   __syncthreads();
-  // new direction (FIRST: x), scattered into the grid; bra sums of the projectors
+  // a column's a3 line starts at its row and a2 position, stride p2
+  auto line = [=](int c) {
+    const int pos = R.col_pos[c];
+    const int r = pos / n2;
+    return r * rs + (pos - r * n2);
+  };
+  auto slot = [=](int ig) {
+    const int k = K.pt_k[ig];
+    return line(K.pt_col[ig]) + (k < 0 ? k + n3 : k) * p2;
+  };
+  // new direction (FIRST: x) onto the lines; bra sums of the projectors
   const double bt = FIRST ? 0.0 : a.beta[lb];
-  double acc[KL_NQ2];
-#pragma unroll
-  for (int i = 0; i < KL_NQ2; ++i) acc[i] = 0.0;
-  for (int ig = tid; ig < ld; ig += KL_NT) {
+  for (int ig = tid; ig < ld; ig += NT) {
     z64 v;
     if constexpr (FIRST) {
       v = xc[ig];
@@ -284,93 +366,117 @@ __global__ __launch_bounds__(KL_NT) void k_cg_iter_lds(KlCgArgs a) {
       hc[ig] = v;
       bb[ig] = v;
     }
-    if (ig < npw) {
-      const int r = nl[ig];
-      grid[r % a.n1 + a.p1 * (r / a.n1)] = v;
-#pragma unroll
-      for (int i = 0; i < KL_NQ2; ++i)
-        if (i < nq2) acc[i] += q2[i * ldr + 2 * ig] * v.x + q2[i * ldr + 2 * ig + 1] * v.y;
-    }
+    if (ig < npw) grid[slot(ig)] = v;
   }
-  kl_block_sums(acc, nq2, red, sums);
-  if (tid < nq2) c2s[tid] = a.qs[tid] * sums[tid];
-  // (kl_block_sums ends with a barrier: the grid is complete)
-  kl_local(grid, a.n1, a.n2, a.n3, a.p1, a.vrs);
+  // (four projector rows at a time: all 32 unrolled keep 32 base addresses and
+  // sums live and spill)
+  const z64* vc = FIRST ? xc : bb;
+  for (int i0 = 0; i0 < nq2; i0 += 4) {
+    double acc[4] = {0.0, 0.0, 0.0, 0.0};
+    const z64* qr = reinterpret_cast<const z64*>(q2 + i0 * ldr);
+    for (int ig = tid; ig < npw; ig += NT) {
+      const z64 v = vc[ig];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (i0 + j < nq2) {
+          const z64 w = qr[j * ld + ig];
+          acc[j] += w.x * v.x + w.y * v.y;
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (i0 + j < nq2) {
+        double x = acc[j];
+        for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
+        if ((tid & 63) == 0) red[i0 + j][tid >> 6] = x;
+      }
+  }
+  __syncthreads();
+  if (tid < nq2) {
+    double x = 0.0;
+#pragma unroll
+    for (int q = 0; q < NT / 64; ++q) x += red[tid][q];
+    c2s[tid] = a.qs[tid] * x;
+  }
+  for (int c = tid; c < R.nct; c += NT) kl_pass<+1>(n3, grid + line(c), p2);
+  __syncthreads();
+  for (int l = tid; l < nrows * n3; l += NT) kl_pass<+1>(n2, grid + l * p2, 1);
+  __syncthreads();
+  const double sc = 1.0 / (static_cast<double>(n1) * n2 * n3);
+  for (int l = tid; l < n2 * n3; l += NT) {
+    const int z = l / n2, y = l - z * n2;
+    kl_pass_rows(n1, grid + imax * rs + z * p2 + y, rs, imax, a.vrs + z * n1 * n2 + y, n2, sc);
+  }
+  __syncthreads();
+  for (int l = tid; l < nrows * n3; l += NT) kl_pass<-1>(n2, grid + l * p2, 1);
+  __syncthreads();
+  for (int c = tid; c < R.nct; c += NT) kl_pass<-1>(n3, grid + line(c), p2);
+  __syncthreads();
   // t: local + kinetic + projectors; dots of the new direction
-  const double sc = 1.0 / (static_cast<double>(a.n1) * a.n2 * a.n3);
   const double eb = a.eu[lb];
+  const double e = a.ep[col];
+  auto tval = [&](int ig, z64 v) {
+    const z64 t = grid[slot(ig)] + cscale(v, K.g2[ig] - eb);
+    double kr = 0.0, ki = 0.0;
+    const z64* qr = reinterpret_cast<const z64*>(q2) + ig;
+#pragma unroll 4
+    for (int i = 0; i < nq2; ++i) {
+      const z64 w = qr[i * ld];
+      kr += w.x * c2s[i];
+      ki += w.y * c2s[i];
+    }
+    return t + mk(kr, ki);
+  };
   if constexpr (FIRST) {
     const z64* bcol = a.b + col * ld;
-    const double e = a.ep[col];
     double rr[1] = {0.0};
-    for (int ig = tid; ig < ld; ig += KL_NT) {
+    for (int ig = tid; ig < ld; ig += NT) {
       if (ig >= npw) {
         gc[ig] = mk(0.0, 0.0) - bcol[ig];
         hc[ig] = mk(0.0, 0.0);
         continue;
       }
-      const int r = nl[ig];
-      const z64 v = xc[ig];
-      z64 t = cscale(grid[r % a.n1 + a.p1 * (r / a.n1)], sc) + cscale(v, g2[ig] - eb);
-      double kr = 0.0, ki = 0.0;
-#pragma unroll
-      for (int i = 0; i < KL_NQ2; ++i)
-        if (i < nq2) {
-          kr += q2[i * ldr + 2 * ig] * c2s[i];
-          ki += q2[i * ldr + 2 * ig + 1] * c2s[i];
-        }
-      t = t + mk(kr, ki);
-      const z64 gn = t - bcol[ig];
+      const z64 gn = tval(ig, xc[ig]) - bcol[ig];
       gc[ig] = gn;
-      const z64 hn = cscale(gn, 1.0 / fmax(1.0, g2[ig] / e));
+      const z64 hn = cscale(gn, 1.0 / fmax(1.0, K.g2[ig] / e));
       hc[ig] = hn;
       rr[0] += hn.x * gn.x + hn.y * gn.y;
     }
-    kl_block_sums(rr, 1, red, sums);
+    kl_sums<NT, 1>(rr, 1, red, sums);
     if (tid == 0) a.rho[col] = sums[0];
-    return;
   } else {
-  double dots[2] = {0.0, 0.0};
-  for (int ig = tid; ig < ld; ig += KL_NT) {
-    if (ig >= npw) {
-      tt[ig] = mk(0.0, 0.0);
-      continue;
-    }
-    const int r = nl[ig];
-    const z64 v = bb[ig];
-    z64 t = cscale(grid[r % a.n1 + a.p1 * (r / a.n1)], sc) + cscale(v, g2[ig] - eb);
-    double kr = 0.0, ki = 0.0;
-#pragma unroll
-    for (int i = 0; i < KL_NQ2; ++i)
-      if (i < nq2) {
-        kr += q2[i * ldr + 2 * ig] * c2s[i];
-        ki += q2[i * ldr + 2 * ig + 1] * c2s[i];
+    double dots[2] = {0.0, 0.0};
+    for (int ig = tid; ig < ld; ig += NT) {
+      if (ig >= npw) {
+        tt[ig] = mk(0.0, 0.0);
+        continue;
       }
-    t = t + mk(kr, ki);
-    tt[ig] = t;
-    dots[0] += v.x * gc[ig].x + v.y * gc[ig].y;
-    dots[1] += v.x * t.x + v.y * t.y;
-  }
-  kl_block_sums(dots, 2, red, sums);
-  const double st = sums[0] / sums[1];
-  const double e = a.ep[col];
-  double rr[1] = {0.0};
-  for (int ig = tid; ig < ld; ig += KL_NT) {
-    const z64 v = bb[ig];
-    const z64 gn = gc[ig] - cscale(tt[ig], st);
-    xc[ig] = xc[ig] - cscale(v, st);
-    gc[ig] = gn;
-    ho[ig] = v;
-    if (ig < npw) {
-      const z64 hn = cscale(gn, 1.0 / fmax(1.0, g2[ig] / e));
-      hc[ig] = hn;
-      rr[0] += hn.x * gn.x + hn.y * gn.y;
-    } else {
-      hc[ig] = mk(0.0, 0.0);
+      const z64 v = bb[ig];
+      const z64 t = tval(ig, v);
+      tt[ig] = t;
+      const z64 gv = gc[ig];
+      dots[0] += v.x * gv.x + v.y * gv.y;
+      dots[1] += v.x * t.x + v.y * t.y;
     }
-  }
-  kl_block_sums(rr, 1, red, sums);
-  if (tid == 0) a.rho[col] = sums[0];
+    kl_sums<NT, 2>(dots, 2, red, sums);
+    const double st = sums[0] / sums[1];
+    double rr[1] = {0.0};
+    for (int ig = tid; ig < ld; ig += NT) {
+      const z64 v = bb[ig];
+      const z64 gn = gc[ig] - cscale(tt[ig], st);
+      xc[ig] = xc[ig] - cscale(v, st);
+      gc[ig] = gn;
+      ho[ig] = v;
+      if (ig < npw) {
+        const z64 hn = cscale(gn, 1.0 / fmax(1.0, K.g2[ig] / e));
+        hc[ig] = hn;
+        rr[0] += hn.x * gn.x + hn.y * gn.y;
+      } else {
+        hc[ig] = mk(0.0, 0.0);
+      }
+    }
+    kl_sums<NT, 1>(rr, 1, red, sums);
+    if (tid == 0) a.rho[col] = sums[0];
   }
 }
 
@@ -544,8 +650,8 @@ __global__ void k_sum_k(int nks, int m, int npwq, long ldq, const z64* __restric
 }
 
 constexpr size_t kKlMaxSmem = 160u * 1024u;
-// LDS the fused CG iteration uses besides the grid (its reduction arrays)
-constexpr size_t kKlCgStatic = sizeof(double) * (KL_NQ2 * (KL_NT / 64) + 2 * KL_NQ2);
+// LDS the fused CG iteration uses besides the rows (its reduction arrays)
+constexpr size_t kKlCgStatic = sizeof(double) * (KL_NQ2 * (KR_NT / 64) + 2 * KL_NQ2);
 
 size_t kl_smem(int n1, int n2, int n3) { return sizeof(z64) * static_cast<size_t>(n1 | 1) * n2 * n3; }
 
@@ -553,11 +659,6 @@ size_t kl_smem(int n1, int n2, int n3) { return sizeof(z64) * static_cast<size_t
 
 bool kvloc_lds_available(int n1, int n2, int n3) {
   return kl_size(n1) && kl_size(n2) && kl_size(n3) && kl_smem(n1, n2, n3) <= kKlMaxSmem;
-}
-
-bool cg_iter_lds_available(int n1, int n2, int n3, int nq2) {
-  return kl_size(n1) && kl_size(n2) && kl_size(n3) && nq2 >= 0 && nq2 <= KL_NQ2 &&
-         kl_smem(n1, n2, n3) + kKlCgStatic <= kKlMaxSmem;
 }
 
 namespace {
@@ -611,43 +712,35 @@ void density_lds(int n1, int n2, int n3, int nks, int nb, int m, long ld, const 
   WH_HIP(hipGetLastError());
 }
 
-void cg_iter_lds(int n1, int n2, int n3, int npw, long ld, const int* nl, const double* vrs, const double* g2,
-                 int nq2, const double* q2, const double* qs, int cap, const int* l2i, const int* nc,
-                 const double* beta, const double* eu, const double* ep, z64* h, z64* hold, z64* x, z64* g, z64* bc,
-                 z64* tc, double* rho, hipStream_t s, const KlKpoint* ktab, int cols_per_k) {
-  WH_REQUIRE(cg_iter_lds_available(n1, n2, n3, nq2), "cg_iter_lds: grid or projector count not supported");
-  WH_REQUIRE(!ktab || cols_per_k > 0, "cg_iter_lds: cols_per_k must be > 0");
-  if (cap <= 0) return;
-  const size_t dyn = kl_smem(n1, n2, n3);
-  static const bool attr_set = [] {   // once per process (thread-safe static initialisation)
-    WH_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_cg_iter_lds<false>),
-                               hipFuncAttributeMaxDynamicSharedMemorySize,
-                               static_cast<int>(kKlMaxSmem - kKlCgStatic)));
-    return true;
-  }();
-  (void)attr_set;
-  const KlCgArgs a{n1, n2, n3, n1 | 1, npw, ld, nl, vrs, g2, nq2, q2, qs, l2i, nc, beta, eu, ep,
-                   h, hold, x, g, bc, tc, rho, ktab, cols_per_k, nullptr};
-  k_cg_iter_lds<false><<<cap, KL_NT, dyn, s>>>(a);
-  WH_HIP(hipGetLastError());
+namespace {
+size_t kl_rows_smem(const StickPlanDev& P) {
+  return sizeof(z64) * static_cast<size_t>(P.nrows) * P.n3 * (P.n2 | 1);
+}
+}  // namespace
+
+int cg_iter_wgs(const StickPlan& p, int nq2) {
+  const StickPlanDev& P = p.dev;
+  if (P.nct <= 0 || nq2 < 0 || nq2 > KL_NQ2 || !kl_size(P.n1) || !kl_size(P.n2) || !kl_size(P.n3)) return 0;
+  if (P.imax > kl_row_bound(P.n1)) return 0;
+  return static_cast<int>(kKlMaxSmem / (kl_rows_smem(P) + kKlCgStatic));
 }
 
-void cg_first_lds(int n1, int n2, int n3, long ld, const double* vrs, int nq2, const double* qs, int m,
-                  const double* e, const double* ep, const z64* x, const z64* b, z64* g, z64* h, double* rho,
-                  const KlKpoint* ktab, int cols_per_k, hipStream_t s) {
-  WH_REQUIRE(cg_iter_lds_available(n1, n2, n3, nq2), "cg_first_lds: grid or projector count not supported");
-  WH_REQUIRE(ktab && cols_per_k > 0, "cg_first_lds: a k-point table and cols_per_k > 0 are required");
+void cg_iter_rows(const StickPlan& p, const KStick* stab, bool first, int m, const KlCgArgs& a, hipStream_t s) {
+  WH_REQUIRE(cg_iter_wgs(p, a.nq2) > 0, "cg_iter_rows: grid or projector count not supported");
+  WH_REQUIRE(!a.ktab || a.cols_per_k > 0, "cg_iter_rows: cols_per_k must be > 0");
   if (m <= 0) return;
   static const bool attr_set = [] {   // once per process (thread-safe static initialisation)
-    WH_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_cg_iter_lds<true>),
-                               hipFuncAttributeMaxDynamicSharedMemorySize,
-                               static_cast<int>(kKlMaxSmem - kKlCgStatic)));
+    for (const void* k : {reinterpret_cast<const void*>(k_cg_iter_rows<false>),
+                          reinterpret_cast<const void*>(k_cg_iter_rows<true>)})
+      WH_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                 static_cast<int>(kKlMaxSmem - kKlCgStatic)));
     return true;
   }();
   (void)attr_set;
-  const KlCgArgs a{n1, n2, n3, n1 | 1, 0, ld, nullptr, vrs, nullptr, nq2, nullptr, qs, nullptr, nullptr, nullptr,
-                   e, ep, h, nullptr, const_cast<z64*>(x), g, nullptr, nullptr, rho, ktab, cols_per_k, b};
-  k_cg_iter_lds<true><<<m, KL_NT, kl_smem(n1, n2, n3), s>>>(a);
+  const StickPlanDev& P = p.dev;
+  const KlRows r{P.n1, P.n2, P.n3, P.imax, P.nct, P.n2 | 1, P.col_pos};
+  if (first) k_cg_iter_rows<true><<<m, KR_NT, kl_rows_smem(P), s>>>(r, stab, a);
+  else k_cg_iter_rows<false><<<m, KR_NT, kl_rows_smem(P), s>>>(r, stab, a);
   WH_HIP(hipGetLastError());
 }
 

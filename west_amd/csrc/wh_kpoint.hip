@@ -98,13 +98,14 @@ struct KPath {
   KlKpoint* ktab = nullptr;   // device: each k point's sphere and projectors (batched CG)
   double* sck = nullptr;      // device: 2 w_k / (Omega N_r) per k point (densities at q)
   // stick transforms (grids beyond the LDS): k-point vectors are in stick order
-  bool sticks_want = false;   // the grid has the z kernels
+  bool sticks_want = false;   // stick order in use
   bool sticks_built = false;  // the plan below holds every registered k sphere
-  bool sticks_ok = false;     // ... and the grid has plane kernels for it
+  bool sticks_ok = false;     // ... and the grid has z and plane kernels for it
   StickPlan plan;             // union of the k spheres' columns
   KStick* stab = nullptr;     // device, per k point
   const double** qptr = nullptr;   // device, per k point: q2
-  double* vrs_plane = nullptr;     // vrs in the plane kernels' layout
+  double* vrs_t = nullptr;         // vrs as the two-radix plane kernels read it, [a3][a1][a2]
+  int cg_wgs = 0;                  // workgroups per CU of the fused CG iteration (0: none)
   std::vector<void*> stick_allocs;
   DevBuf w_sa, w_sb, w_ident, w_grp;
   DevBuf w_dk;                // densities per (k point, perturbation) before the sum over k
@@ -580,15 +581,16 @@ static bool ksticks_enabled() {
 // The stick plan of the registered k points: the union of their columns, so
 // that one plane launch takes items of any of them.  Built at the first use
 // after a registration.
-static bool sticks_ready(KPath& K) {
-  if (!K.sticks_want) return false;
-  if (K.sticks_built) return K.sticks_ok;
+static void build_sticks(KPath& K) {
+  if (!K.sticks_want || K.sticks_built) return;
   Context& c = ctx();
   WH_HIP(hipStreamSynchronize(c.stream));
   for (void* p : K.stick_allocs) (void)hipFree(p);
   K.stick_allocs.clear();
   K.stab = nullptr;
+  K.vrs_t = nullptr;
   K.sticks_ok = false;
+  K.cg_wgs = 0;
   std::map<std::pair<int, int>, int> at;
   for (const KPointDev& P : K.k)
     for (size_t q = 0; q < P.col_i.size(); ++q) at[{P.col_i[q], P.col_j[q]}] = 0;
@@ -599,7 +601,9 @@ static bool sticks_ready(KPath& K) {
     cj.push_back(e.first.second);
   }
   K.sticks_built = true;
-  if (ci.empty() || !K.plan.build_columns(K.fft.n1, K.fft.n2, K.fft.n3, ci, cj)) return false;
+  if (ci.empty()) return;
+  const bool planes = K.plan.build_columns(K.fft.n1, K.fft.n2, K.fft.n3, ci, cj);
+  if (K.plan.dev.nct == 0) return;
   auto up = [&](const auto& h) {
     using V = typename std::decay_t<decltype(h)>::value_type;
     V* d = nullptr;
@@ -624,16 +628,24 @@ static bool sticks_ready(KPath& K) {
   }
   K.stab = up(tab);
   K.qptr = up(qp);
-  K.vrs_plane = K.vrs;
-  if (K.plan.transposed_grid()) {
-    double* v = nullptr;
-    WH_HIP(hipMalloc(&v, sizeof(double) * K.fft.nnr()));
-    K.stick_allocs.push_back(v);
-    rect_transpose_grid(K.fft.n1, K.fft.n2, K.fft.n3, K.vrs, v, c.stream);
-    K.vrs_plane = v;
-  }
-  K.sticks_ok = true;
-  return true;
+  WH_HIP(hipMalloc(&K.vrs_t, sizeof(double) * K.fft.nnr()));
+  K.stick_allocs.push_back(K.vrs_t);
+  rect_transpose_grid(K.fft.n1, K.fft.n2, K.fft.n3, K.vrs, K.vrs_t, c.stream);
+  // (a third axis of three or more radices has no z kernel)
+  K.sticks_ok = planes && kz_available(K.fft.n3);
+  K.cg_wgs = cg_iter_wgs(K.plan, 2 * (K.nbndval + K.nkb));
+}
+
+static bool sticks_ready(KPath& K) {
+  build_sticks(K);
+  return K.sticks_ok;
+}
+
+// The fused CG iteration: where the LDS holds a column's rows
+static bool cg_fused(KPath& K) {
+  if (!klds_enabled() || ctx().l_kinetic_only) return false;
+  build_sticks(K);
+  return K.cg_wgs >= 1;
 }
 
 // t = F^-1 V F x + (|k+G|^2 - e) x through sticks for m columns (cols_per_k,
@@ -656,7 +668,8 @@ static void vloc_sticks(KPath& K, int ik, int cols_per_k, const int* l2i, const 
   for (int c0 = 0; c0 < m; c0 += chunk) {
     const int n = std::min(chunk, m - c0);
     WH_TIMED("kzinv", launch_kzinv(K.plan, tab, l2i, cols_per_k, c0, n, d_nc, x, ld, sa, s));
-    WH_TIMED("plane_vloc", launch_plane_vloc(K.plan, items + c0, n, sa, sb, K.vrs_plane, 0, scale, s));
+    WH_TIMED("plane_vloc", launch_plane_vloc(K.plan, items + c0, n, sa, sb,
+                                             K.plan.transposed_grid() ? K.vrs_t : K.vrs, 0, scale, s));
     WH_TIMED("kzfwd", launch_kzfwd(K.plan, tab, l2i, cols_per_k, c0, n, d_nc, sb, x, d_e, t, ld, s));
   }
 }
@@ -814,18 +827,21 @@ static int linsolve_k(KPath& K, int ik, int nkb, int cols, z64* b, z64* x, const
   WH_HIP(hipMemsetAsync(hold, 0, sizeof(z64) * vec, s));
   WH_HIP(hipMemsetAsync(d_conv, 0, sizeof(int) * (static_cast<size_t>(m) + 4), s));
   // small grids with few projector rows: the iteration after cg_select is
-  // one workgroup per column (cg_iter_lds) instead of five launches
+  // one workgroup per column instead of five launches or more
   const int nq2 = 2 * (K.nbndval + K.nkb);
-  const bool fused = klds_enabled() && !c.l_kinetic_only &&
-                     cg_iter_lds_available(K.fft.n1, K.fft.n2, K.fft.n3, nq2);
+  const bool fused = cg_fused(K);
   WH_REQUIRE(fused || nkb == 1 || (!c.l_kinetic_only && sticks_ready(K)),
              "linsolve_k: several k points need the fused iteration or the stick operator");
   const KlKpoint* tab = nkb > 1 ? K.ktab : nullptr;
   if (fused) set_qscale2(K, K.alpha_pv);
   // step 1 (127-138): g = A x - b, and h = M^-1 g, rho of every band
-  if (nkb > 1 && fused) {   // every k point's columns in one launch
-    WH_TIMED("cg_iter_lds", cg_first_lds(K.fft.n1, K.fft.n2, K.fft.n3, ld, K.vrs, nq2, K.qscale2, m, d_e, d_ep, x,
-                                         b, g, h, d_rhob, K.ktab, cols, s));
+  KlCgArgs ca{};
+  if (fused) {
+    ca = KlCgArgs{ld, K.vrs_t, nq2, reinterpret_cast<const double*>(P.q2), K.qscale2, d_l2i, d_nc, d_beta, d_eu, d_ep,
+                  h, hold, x, g, bc, tc, d_rhob, tab, cols, b};
+    KlCgArgs first = ca;
+    first.eu = d_e;   // by column
+    WH_TIMED("cg_iter_lds", cg_iter_rows(K.plan, nkb > 1 ? K.stab : K.stab + ik, true, m, first, s));
     c.nstern += m;
   } else {
     iota(d_l2i, m, s);
@@ -850,10 +866,7 @@ static int linsolve_k(KPath& K, int ik, int nkb, int cols, z64* b, z64* x, const
     // convergence test, compaction, beta (208-224)
     cg_select(m, tr2, it == 1 ? 1 : 0, group, d_rhob, d_rhoold, d_conv, d_e, d_l2i, d_beta, d_eu, d_nc, d_rec, s);
     if (fused) {
-      WH_TIMED("cg_iter_lds", cg_iter_lds(K.fft.n1, K.fft.n2, K.fft.n3, P.npw, ld, P.nl, K.vrs, P.g2kin, nq2,
-                                          reinterpret_cast<const double*>(P.q2), K.qscale2, cap, d_l2i, d_nc,
-                                          d_beta, d_eu, d_ep, h, hold, x, g, bc, tc, d_rhob, s,
-                                          nkb > 1 ? K.ktab : nullptr, cols));
+      WH_TIMED("cg_iter_lds", cg_iter_rows(K.plan, nkb > 1 ? K.stab : K.stab + ik, false, cap, ca, s));
     } else {
       k_cg_dir<<<blocks(static_cast<long>(cap) * ld), NT, 0, s>>>(cap, d_nc, d_l2i, ld, d_beta, d_e, h, hold, bc,
                                                                   d_eu);
@@ -890,7 +903,7 @@ static void cg_k_count(const int* rec, int last) {
 // real view) and the solve's vectors (seven of nks m nbndval columns), the
 // states at k - q and density scratch grids and the per-k densities fit the
 // grid budget.
-static bool kbatch_ok(const KPath& K, int m) {
+static bool kbatch_ok(KPath& K, int m) {
   const char* ev = std::getenv("WH_KBATCH");   // read per call: 0 keeps the k points one after another
   if (ev && ev[0] == '0') return false;
   const Context& c = ctx();
@@ -899,7 +912,7 @@ static bool kbatch_ok(const KPath& K, int m) {
   const long bytes = static_cast<long>(sizeof(z64)) * (7 * all * K.npwx + grids * K.fft.nnr() +
                                                        static_cast<long>(K.nks) * m * K.npwqx);
   return K.nks > 1 && klds_enabled() && !c.l_kinetic_only && all <= (1L << 24) &&
-         cg_iter_lds_available(K.fft.n1, K.fft.n2, K.fft.n3, 2 * (K.nbndval + K.nkb)) &&
+         kvloc_lds_available(K.fft.n1, K.fft.n2, K.fft.n3) && 2 * K.nbndval <= 32 && cg_fused(K) &&
          bytes <= static_cast<long>(K.grid_budget);
 }
 
@@ -1335,9 +1348,7 @@ int wh_set_kgrid(int nr1, int nr2, int nr3, double omega, const double* vrs, int
     std::vector<double> v(nnr);
     WH_HIP(hipMemcpy(v.data(), vrs, sizeof(double) * nnr, hipMemcpyDefault));
     K->vrs = upload(*K, v.data(), v.size());
-    // stick order beyond the LDS grids (an axis of three or more radices has no z kernel)
-    K->sticks_want = ksticks_enabled() && kz_available(nr3) &&
-                     !(klds_enabled() && kvloc_lds_available(nr1, nr2, nr3));
+    K->sticks_want = ksticks_enabled();
     K->k.resize(nks);
     K->q.resize(nqs);
   } catch (...) {
