@@ -8,14 +8,25 @@
 // apply_alpha_pc_to_m_wfcs.f90:59, apply_alpha_pv_to_m_wfcs.f90:71) and the
 // Davidson subspace products (Wstat/wstat_tools.f90 build_hr/update/refresh).
 //
-// Tile 128 x 128 x 16 per 256-thread workgroup: four wavefronts in a 2 x 2
-// arrangement, each owning 64 x 64 = 4 x 4 MFMA 16x16 blocks, with the next
-// K tile prefetched into registers while the current one is multiplied out
-// of a double-buffered LDS tile.  The projection ("bra") products have a
-// small M (occupied bands + projectors) and a long K (2 npw), so they split K
-// over blockIdx.z; the partial products are summed in a fixed order by the
-// epilogue kernel, which also applies the G = 0 correction of glbrak_gamma
-// (its DGER) and the per-row scale, so results do not depend on scheduling.
+// Tile 128 x (32 WN) x 16 per 256-thread workgroup (WN = 4, 2 or 1): four
+// wavefronts in a 2 x 2 arrangement, each owning 64 x 16 WN = 4 x WN MFMA
+// 16x16 blocks.  One tile is multiplied out of LDS while the next goes from
+// registers to the other half of the double buffer and the one after is on its
+// way from memory; both are issued between the two halves of the K steps, so
+// neither is waited for at the barrier.  Bound: the FP64 matrix pipe (64
+// cycles an instruction and SIMD); what is left is the address and LDS work
+// between the matrix instructions, so tiles are loaded 16 bytes a lane and
+// read from LDS two K steps at a time.  TFLOP/s with 8-byte loads, [k][x] tiles
+// for both operands and fixed splits -> now: bra 384 x N over K = 18,278:
+// N = 8,192 55 -> 60, 4,096 50 -> 60, 1,000 43 -> 50, 128 27.5 -> 28.6; ket of
+// the same sizes 50 -> 57, 49 -> 56, 47 -> 51, 26.5 -> 29.5; bra / ket 1,296 x 432
+// over 61,446 42.5 -> 46 / 40 -> 48; 8,192^3 60 -> 66.
+//
+// The projection ("bra") products have a small M (occupied bands +
+// projectors) and a long K (2 npw), so they split K (pick_split); the partial
+// products are summed in a fixed order by the epilogue kernel, which also
+// applies the G = 0 correction of glbrak_gamma (its DGER) and the per-row
+// scale, so results do not depend on scheduling.
 //
 // Operand layout of the 16x16x4 f64 instruction (checked on the device):
 // lane l holds A[l%16][l/16] and B[l/16][l%16]; result register r of lane l
@@ -42,58 +53,144 @@ namespace {
 constexpr int BM = 128;
 constexpr int BK = 16;
 constexpr int NT = 256;
-constexpr int PAD = 2;
 
 typedef double v4d __attribute__((ext_vector_type(4)));
 
-// Tile loads, BK * XT / 256 elements per thread, mapped so that each load
-// instruction of a wavefront reads contiguous memory:
+// Tile loads, 16 bytes at a time (8-byte alignment is enough), mapped so that
+// each load instruction of a wavefront reads contiguous memory:
 //  * x-contiguous operand (element (k, x) at P[k*ld + x]: A of the plain
-//    product, XT = 128): x = tid % 128, k = tid / 128 + 2q  (512 bytes per
-//    instruction);
+//    product, XT = 128): x = 2 (tid % 64), k = tid / 64 + 4q  (1 kB per
+//    instruction); in LDS [k][x] with rows of 132;
 //  * k-contiguous operand (element (k, x) at P[x*ld + k]: A of the bra
-//    product, B of both): k = tid % 16, x = tid / 16 + 16q  (four 128-byte runs).
+//    product, B of both): k = 2 (tid % 8), x = tid / 8 + 32q  (eight 128-byte
+//    runs); in LDS [x][k] (kc_at), so that a lane reads two K steps of its
+//    row at once.
+// The rows' addresses are scalar sums and one 32-bit offset per thread.
+// An MFMA's four k may be any four of the tile as long as both operands agree:
+// lanes 16 g .. 16 g + 15 take k = 4 g + step, which are adjacent in the
+// k-contiguous rows.  No operand read has a bank conflict ([k][x]: a row 4
+// steps on is 32 banks on).
 // CHK: zero-fill outside [0, X) x [k0, kend) (edge tiles only).
+typedef double d2 __attribute__((ext_vector_type(2), aligned(8)));
+
+template <bool KCONT, int XT>
+constexpr int tile_elems() { return KCONT ? XT * BK : BK * 132; }
+// k-contiguous rows: 16-byte chunk c of row x sits at chunk c ^ ((x / 2) % 8),
+// so that 16 rows' same chunk covers all banks without padding (49 kB for the
+// 128 x 64 tiles: three workgroups a CU)
+__device__ __forceinline__ int kc_at(int x, int c) { return x * BK + 2 * (c ^ ((x >> 1) & 7)); }
+template <int XT>
+constexpr int tile_loads() { return BK * XT / NT / 2; }
+
 template <bool KCONT, bool CHK, int XT>
-__device__ __forceinline__ void load_tile(double (&r)[BK * XT / NT], const double* __restrict__ P, long ld, int X,
+__device__ __forceinline__ void load_tile(d2 (&r)[tile_loads<XT>()], const double* __restrict__ P, long ld, int X,
                                           int x0, int k0, int kend) {
   const int tid = threadIdx.x;
+  static_assert(KCONT || XT == 128, "x-contiguous tiles are 128 wide");
+  const unsigned ldu = static_cast<unsigned>(ld);
   if (KCONT) {
-    const int gk = k0 + (tid & 15);
+    const int tk = 2 * (tid & 7), tx = tid >> 3;
+    const unsigned off = tx * ldu + tk;
 #pragma unroll
-    for (int q = 0; q < BK * XT / NT; ++q) {
-      const int gx = x0 + (tid >> 4) + 16 * q;
-      if (CHK) r[q] = (gx < X && gk < kend) ? P[static_cast<long>(gx) * ld + gk] : 0.0;
-      else r[q] = P[static_cast<long>(gx) * ld + gk];
+    for (int q = 0; q < tile_loads<XT>(); ++q) {
+      const double* row = P + static_cast<long>(x0 + 32 * q) * ld + k0;
+      if (CHK) {
+        const bool in = x0 + 32 * q + tx < X;
+        r[q].x = in && k0 + tk < kend ? row[off] : 0.0;
+        r[q].y = in && k0 + tk + 1 < kend ? row[off + 1] : 0.0;
+      } else {
+        r[q] = *reinterpret_cast<const d2*>(row + off);
+      }
     }
   } else {
-    static_assert(KCONT || XT == 128, "x-contiguous tiles are 128 wide");
-    const int gx = x0 + (tid & 127);
+    const int tx = 2 * (tid & 63), tk = tid >> 6;
+    const unsigned off = tk * ldu + tx;
 #pragma unroll
-    for (int q = 0; q < BK * XT / NT; ++q) {
-      const int gk = k0 + (tid >> 7) + 2 * q;
-      if (CHK) r[q] = (gx < X && gk < kend) ? P[static_cast<long>(gk) * ld + gx] : 0.0;
-      else r[q] = P[static_cast<long>(gk) * ld + gx];
+    for (int q = 0; q < tile_loads<XT>(); ++q) {
+      const double* row = P + static_cast<long>(k0 + 4 * q) * ld + x0;
+      if (CHK) {
+        const bool in = k0 + 4 * q + tk < kend;
+        r[q].x = in && x0 + tx < X ? row[off] : 0.0;
+        r[q].y = in && x0 + tx + 1 < X ? row[off + 1] : 0.0;
+      } else {
+        r[q] = *reinterpret_cast<const d2*>(row + off);
+      }
     }
   }
 }
 
-// the LDS tile is [k][x] for both operands
 template <bool KCONT, int XT>
-__device__ __forceinline__ void store_tile(double (*S)[XT + PAD], const double (&r)[BK * XT / NT]) {
+__device__ __forceinline__ void store_tile(double* S, const d2 (&r)[tile_loads<XT>()]) {
   const int tid = threadIdx.x;
-  if (KCONT) {
 #pragma unroll
-    for (int q = 0; q < BK * XT / NT; ++q) S[tid & 15][(tid >> 4) + 16 * q] = r[q];
-  } else {
-#pragma unroll
-    for (int q = 0; q < BK * XT / NT; ++q) S[(tid >> 7) + 2 * q][tid & 127] = r[q];
+  for (int q = 0; q < tile_loads<XT>(); ++q) {
+    const int o = KCONT ? kc_at((tid >> 3) + 32 * q, tid & 7) : ((tid >> 6) + 4 * q) * 132 + 2 * (tid & 63);
+    *reinterpret_cast<double2*>(S + o) = make_double2(r[q].x, r[q].y);
   }
 }
 
-// Tiles (bx, by, kz): gx x gy output tiles times gz K chunks, k range
-// [kz*kchunk, min(K, (kz+1)*kchunk)); gz > 1: raw partial sums go to
-// C + kz*pstride (alpha, beta ignored).  The grid is 1D and its blocks are
+// operand rows x0 + 16 i + lane % 16 for the K steps 2 h, 2 h + 1
+template <bool KCONT, int NB>
+__device__ __forceinline__ void read_ops(double (&v)[NB][2], const double* S, int x0, int lane, int h) {
+  const int g = lane >> 4, x = x0 + (lane & 15);
+#pragma unroll
+  for (int i = 0; i < NB; ++i) {
+    if (KCONT) {
+      const double2 w = *reinterpret_cast<const double2*>(S + kc_at(x + 16 * i, 2 * g + h));
+      v[i][0] = w.x;
+      v[i][1] = w.y;
+    } else {
+      v[i][0] = S[(4 * g + 2 * h) * 132 + x + 16 * i];
+      v[i][1] = S[(4 * g + 2 * h + 1) * 132 + x + 16 * i];
+    }
+  }
+}
+
+// K chunks of a split product: the cost of s chunks is the rounds of slots_of
+// workgroups, each with its share of the K steps and about kOvh more for its
+// first loads and its stores, and the partial sums' write and read at about
+// 1.7 kB a cycle; candidates fill one or two rounds (up to four measured the
+// same).  Whole numbers throughout: the host, which sizes grids and buffers,
+// and the device must come to the same answer.
+// (Three fixed splits, aimed at 512, 1,024 or 2,048 workgroups and timed
+// against each other, left a last round nearly empty, e.g. 576 workgroups for
+// 384 x 8,192, and were sized for the launch's columns, not the active ones.)
+__host__ __device__ constexpr int slots_of(int wn) { return wn == 4 ? 512 : 768; }   // workgroups the chip holds
+constexpr int kMaxRounds = 2;
+constexpr int kMaxSplit = 64;
+constexpr int kOvh = 5;
+__host__ __device__ inline int pick_split(int M, int N, int K, int wn) {
+  const int tiles = ((M + BM - 1) / BM) * ((N + 32 * wn - 1) / (32 * wn));
+  const int kt = max((K + BK - 1) / BK, 1);
+  const int slots = slots_of(wn);
+  int best = 1;
+  long cost = 0;
+  for (int r = 0; r <= kMaxRounds; ++r) {
+    // each chunk at least 16 steps long
+    const int s = r == 0 ? 1 : min(min(slots * r / max(tiles, 1), kMaxSplit), kt / 16);
+    if (s < 1) continue;
+    const int per = (kt + s - 1) / s;
+    const int n = (kt + per - 1) / per;   // chunks that the steps fill
+    const int rounds = (tiles * n + slots - 1) / slots;
+    const long c = static_cast<long>(rounds) * (per + kOvh) * (wn == 4 ? 8192 : 3072 * wn) +
+                   (n > 1 ? static_cast<long>(M) * N * n * 5 / 512 : 0L);
+    if (r == 0 || c < cost) {
+      cost = c;
+      best = n;
+    }
+  }
+  return best;
+}
+__host__ __device__ inline int split_chunk(int K, int split) {
+  const int kt = (K + BK - 1) / BK;
+  return (kt + split - 1) / split * BK;
+}
+
+// Tiles (bx, by, kz): gx x gy output tiles times split K chunks of
+// split_chunk(K, split).  partial: raw partial sums go to C + kz ldc N (alpha,
+// beta ignored; N the active columns).  d_split (with d_n): where fewer than
+// the launch's columns are active, the split is pick_split of those, and the
+// one taken is left in *d_split for the epilogue.  The grid is 1D and its blocks are
 // dispatched round-robin over the 8 XCDs (block L on XCD L % 8); tile
 // W = (L % 8) * ceil(tiles / 8) + L / 8 puts consecutive tiles, which share
 // their B panel (same by, kz) or A panel (same bx, kz), on one XCD and its L2.
@@ -106,11 +203,10 @@ __host__ __device__ inline int xcd_blocks(int tiles) { return (tiles + kXcds - 1
 // GRP: the columns fall into groups with a left operand of their own (device
 // tables G); a tile lies within one group.
 template <bool TA, int WN, bool GRP = false>
-__global__ __launch_bounds__(NT, 2) void k_dgemm(int M, int N, int K, int kchunk, double alpha,
+__global__ __launch_bounds__(NT, WN == 4 ? 2 : 3) void k_dgemm(int M, int N, int K, int split, bool partial, double alpha,
                                               const double* __restrict__ A, long lda, const double* __restrict__ B,
-                                              long ldb, double beta, double* __restrict__ C, long ldc, long pstride,
-                                              int gx, int gy, int gz, const int* __restrict__ d_n,
-                                              DgemmGroups G) {
+                                              long ldb, double beta, double* __restrict__ C, long ldc,
+                                              int gx, int gy, const int* __restrict__ d_n, int* d_split, DgemmGroups G) {
   constexpr int TN = 32 * WN;
   if (GRP) {
     gy = G.tstart[G.ng];
@@ -118,17 +214,25 @@ __global__ __launch_bounds__(NT, 2) void k_dgemm(int M, int N, int K, int kchunk
   } else if (d_n) {
     // columns the device left active: the tiles of the active columns are
     // renumbered over the whole grid, so they still spread over all XCDs
-    N = min(N, *d_n);
-    gy = min(gy, (N + TN - 1) / TN);
+    const int na = min(N, *d_n);
+    gy = min(gy, (na + TN - 1) / TN);
+    if (gy == 0) return;   // no active column
+    if (d_split) {
+      if (na < N) split = pick_split(M, na, K, WN);
+      if (blockIdx.x == 0 && threadIdx.x == 0) *d_split = split;
+    }
+    N = na;
   }
-  __shared__ double As[2][BK][BM + PAD];
-  __shared__ double Bs[2][BK][TN + PAD];
+  const long pstride = ldc * N;   // (grouped: of the launch's N)
+  const int kchunk = split_chunk(K, split);
+  __shared__ __align__(16) double As[2][tile_elems<TA, BM>()];
+  __shared__ __align__(16) double Bs[2][tile_elems<true, TN>()];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = tid >> 6;
   const int wm = wave & 1;
   const int wn = wave >> 1;
-  const int tiles = gx * gy * gz;
+  const int tiles = gx * gy * split;
   // (with fewer active tiles than the grid was sized for, only the first
   // xcd_blocks(tiles) workgroups take part, so each tile has exactly one)
   if (static_cast<int>(blockIdx.x) >= xcd_blocks(tiles)) return;
@@ -154,9 +258,10 @@ __global__ __launch_bounds__(NT, 2) void k_dgemm(int M, int N, int K, int kchunk
   const int kend = min(K, kbeg + kchunk);
   // interior tiles load without bounds checks (all but a short last K step)
   const bool interior = m0 + BM <= M && n0 + TN <= N;
-  const bool partial = gz > 1;
   // C = alpha AB + beta C on an interior tile: the C loads of a row block are
-  // issued while the previous block is combined and stored
+  // issued while the previous block is combined and stored.  (Accumulators
+  // that start from C, their loads under the first tiles', measured 2-4 %
+  // faster, but every partial sum is then rounded at the size of C.)
   const bool rmw = !partial && beta != 0.0 && interior;
   double* Cz = C + (partial ? static_cast<long>(kz) * pstride : 0L);
   const int row0 = m0 + wm * 64 + (lane & 15);
@@ -174,7 +279,7 @@ __global__ __launch_bounds__(NT, 2) void k_dgemm(int M, int N, int K, int kchunk
 #pragma unroll
     for (int j = 0; j < WN; ++j) acc[i][j] = v4d{0.0, 0.0, 0.0, 0.0};
   const int ntile = kend > kbeg ? (kend - kbeg + BK - 1) / BK : 0;
-  double ra[BK * BM / NT], rb[BK * TN / NT];
+  d2 ra[tile_loads<BM>()], rb[tile_loads<TN>()];
   auto load = [&](int k0) {
     if (interior && k0 + BK <= kend) {
       load_tile<TA, false, BM>(ra, A, lda, M, m0, k0, kend);
@@ -184,31 +289,37 @@ __global__ __launch_bounds__(NT, 2) void k_dgemm(int M, int N, int K, int kchunk
       load_tile<true, true, TN>(rb, B, ldb, N, n0, k0, kend);
     }
   };
+  auto store = [&](int buf) {
+    store_tile<TA, BM>(As[buf], ra);
+    store_tile<true, TN>(Bs[buf], rb);
+  };
   if (ntile > 0) {
     load(kbeg);
-    store_tile<TA, BM>(As[0], ra);
-    store_tile<true, TN>(Bs[0], rb);
+    store(0);
+    if (ntile > 1) load(kbeg + BK);
   }
   __syncthreads();
+  // Per tile: half of the K steps, then the next tile goes to the other LDS
+  // buffer (free since the last barrier) and the loads of the one after are
+  // issued, so neither is waited for at the barrier, then the other half.
   for (int t = 0; t < ntile; ++t) {
     const int cur = t & 1;
-    if (t + 1 < ntile) load(kbeg + (t + 1) * BK);
 #pragma unroll
-    for (int kk = 0; kk < BK; kk += 4) {
-      const int kr = kk + (lane >> 4);
-      double a[4], b[WN];
+    for (int h = 0; h < 2; ++h) {
+      double a[4][2], b[WN][2];
+      read_ops<TA, 4>(a, As[cur], wm * 64, lane, h);
+      read_ops<true, WN>(b, Bs[cur], wn * (16 * WN), lane, h);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) a[i] = As[cur][kr][wm * 64 + i * 16 + (lane & 15)];
+      for (int st = 0; st < 2; ++st)
 #pragma unroll
-      for (int j = 0; j < WN; ++j) b[j] = Bs[cur][kr][wn * (16 * WN) + j * 16 + (lane & 15)];
+        for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < WN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(b[j], a[i], acc[i][j], 0, 0, 0);
-    }
-    if (t + 1 < ntile) {
-      store_tile<TA, BM>(As[cur ^ 1], ra);
-      store_tile<true, TN>(Bs[cur ^ 1], rb);
+          for (int j = 0; j < WN; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(b[j][st], a[i][st], acc[i][j], 0, 0, 0);
+      if (h == 0) {
+        if (t + 1 < ntile) store(cur ^ 1);
+        if (t + 2 < ntile) load(kbeg + (t + 2) * BK);
+      }
     }
     __syncthreads();
   }
@@ -344,15 +455,18 @@ __global__ __launch_bounds__(NTS) void k_ket_skinny(int M, int K, double alpha, 
 
 // C(i, j) = s_i * (alpha * sum_z P_z(i, j) - g0 * a(1, i) * b(1, j))
 //   P_z: split partials (ldc, stride pstride); a(1, i) = A[i*lda], b(1, j) = B[j*ldb]
+// pstride 0: ldc x the active columns; d_split: k_dgemm's split of those
 __global__ void k_reduce_g0(int M, int N, int nsplit, const double* P, long pstride, double alpha, double g0,
                             const double* A, long lda, const double* B, long ldb, const double* s, double* C,
-                            long ldc, const int* d_n) {
+                            long ldc, const int* d_n, const int* d_split) {
   if (d_n) N = min(N, *d_n);
+  if (pstride == 0) pstride = ldc * N;
   const long idx = static_cast<long>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (idx >= static_cast<long>(M) * N) return;
   const int i = static_cast<int>(idx % M);
   const int j = static_cast<int>(idx / M);
   const long o = static_cast<long>(j) * ldc + i;
+  if (d_split) nsplit = *d_split;
   double acc = 0.0;
   for (int z = 0; z < nsplit; ++z) acc += P[static_cast<long>(z) * pstride + o];
   double v = alpha * acc;
@@ -404,24 +518,27 @@ Scratch& partials() {
 
 }  // namespace
 
+// split: K chunks; more than one, or partial: partial sums.  d_split: see k_dgemm
 template <bool TA, int WN>
-static void launch_tiles(int M, int N, int K, int kchunk, int gz, double alpha, const double* A, long lda,
-                         const double* B, long ldb, double beta, double* C, long ldc, long pstride, hipStream_t s,
-                         const int* d_n) {
+static void launch_tiles(int M, int N, int K, int split, bool partial, double alpha, const double* A, long lda,
+                         const double* B, long ldb, double beta, double* C, long ldc, hipStream_t s, const int* d_n,
+                         int* d_split) {
   const int gx = ceil_div(M, BM), gy = ceil_div(N, 32 * WN);
-  k_dgemm<TA, WN><<<xcd_blocks(gx * gy * gz), NT, 0, s>>>(M, N, K, kchunk, alpha, A, lda, B, ldb, beta, C, ldc,
-                                                          pstride, gx, gy, gz, d_n, DgemmGroups{});
+  // fewer active columns than N may be cut into more chunks: the most workgroups any split makes
+  const int wgs = d_split ? std::max(gx * gy * split, slots_of(WN) * kMaxRounds) : gx * gy * split;
+  k_dgemm<TA, WN><<<xcd_blocks(wgs), NT, 0, s>>>(M, N, K, split, partial, alpha, A, lda, B, ldb, beta, C, ldc, gx, gy,
+                                                 d_n, d_split, DgemmGroups{});
   WH_HIP(hipGetLastError());
 }
 
 // tile width variants: WN = 4, 2, 1 (128-, 64- and 32-column tiles)
 template <bool TA>
-static void launch_wn(int v, int M, int N, int K, int kchunk, int gz, double alpha, const double* A, long lda,
-                      const double* B, long ldb, double beta, double* C, long ldc, long pstride, hipStream_t s,
-                      const int* d_n = nullptr) {
-  if (v == 0) launch_tiles<TA, 4>(M, N, K, kchunk, gz, alpha, A, lda, B, ldb, beta, C, ldc, pstride, s, d_n);
-  else if (v == 1) launch_tiles<TA, 2>(M, N, K, kchunk, gz, alpha, A, lda, B, ldb, beta, C, ldc, pstride, s, d_n);
-  else launch_tiles<TA, 1>(M, N, K, kchunk, gz, alpha, A, lda, B, ldb, beta, C, ldc, pstride, s, d_n);
+static void launch_wn(int v, int M, int N, int K, int split, bool partial, double alpha, const double* A, long lda,
+                      const double* B, long ldb, double beta, double* C, long ldc, hipStream_t s,
+                      const int* d_n = nullptr, int* d_split = nullptr) {
+  if (v == 0) launch_tiles<TA, 4>(M, N, K, split, partial, alpha, A, lda, B, ldb, beta, C, ldc, s, d_n, d_split);
+  else if (v == 1) launch_tiles<TA, 2>(M, N, K, split, partial, alpha, A, lda, B, ldb, beta, C, ldc, s, d_n, d_split);
+  else launch_tiles<TA, 1>(M, N, K, split, partial, alpha, A, lda, B, ldb, beta, C, ldc, s, d_n, d_split);
 }
 constexpr int kWnVariants = 3;
 inline int wn_of(int v) { return 4 >> v; }
@@ -476,10 +593,10 @@ void dgemm(bool transa, int M, int N, int K, double alpha, const double* A, long
     WH_HIP(hipGetLastError());
     return;
   }
-  const int K0 = std::max(K, 0), kc = std::max(K, 1);
+  const int K0 = std::max(K, 0);
   auto run = [&](int v, double* Cv) {
-    if (transa) launch_wn<true>(v, M, N, K0, kc, 1, alpha, A, lda, B, ldb, beta, Cv, ldc, 0, s, d_n);
-    else launch_wn<false>(v, M, N, K0, kc, 1, alpha, A, lda, B, ldb, beta, Cv, ldc, 0, s, d_n);
+    if (transa) launch_wn<true>(v, M, N, K0, 1, false, alpha, A, lda, B, ldb, beta, Cv, ldc, s, d_n);
+    else launch_wn<false>(v, M, N, K0, 1, false, alpha, A, lda, B, ldb, beta, Cv, ldc, s, d_n);
   };
   // tile width, timed once per (op, M, log2 K, log2 N)
   const VariantKey key{0, transa ? 1 : 0, M, log2_bucket(std::max(K, 1)), log2_bucket(N)};
@@ -504,33 +621,30 @@ void dgemm(bool transa, int M, int N, int K, double alpha, const double* A, long
   run(pick, C);
 }
 
-// v = 3 * d + w: K split aimed at 512 << d workgroups (512: two per compute
-// unit), tile width variant w.  Returns the split depth and K chunk.
-static void bra_split(int M, int N, int K, int v, int& split, int& kchunk) {
-  const int w = v % kWnVariants;
-  const int wg_target = 512 << (v / kWnVariants);
-  const int tiles = ceil_div(M, BM) * ceil_div(N, 32 * wn_of(w));
-  // enough workgroups for the compute units (few output tiles, as in the
-  // narrow products of a partial batch, need a deep split), each K chunk at
-  // least 16 steps long
-  split = std::max(1, std::min(64, ceil_div(wg_target, tiles)));
-  split = std::max(1, std::min(split, K / (16 * BK)));
-  kchunk = ceil_div(ceil_div(std::max(K, 1), split), BK) * BK;
-  split = ceil_div(std::max(K, 1), kchunk);
+// doubles of partial sums for N columns, or (upto) for any count up to N:
+// pick_split gives at most slots_of kMaxRounds workgroups beyond one chunk
+static long partials_doubles(int M, int N, int K, long ldc, int wn, bool upto) {
+  if (!upto) return static_cast<long>(pick_split(M, N, K, wn)) * ldc * N;
+  const long cols = std::max<long>(N, static_cast<long>(slots_of(wn)) * kMaxRounds * 32 * wn / ceil_div(M, BM));
+  return std::min<long>(cols, static_cast<long>(kMaxSplit) * N) * ldc;
 }
 
-// P: room for the split-K partial sums (null: the per-thread scratch)
+// v: tile width variant.  P: room for the split-K partial sums (null: the per-thread scratch)
 static void dgemm_bra_own(int M, int N, int K, double alpha, const double* A, long lda, const double* B, long ldb,
                           double g0, const double* scale, double* C, long ldc, hipStream_t s, int v = 0,
                           double* P = nullptr, const int* d_n = nullptr) {
-  int split = 1, kchunk = 1;
-  bra_split(M, N, K, v, split, kchunk);
-  const long pstride = static_cast<long>(ldc) * N;
-  if (!P) P = partials().get(static_cast<size_t>(split) * pstride, s);
-  launch_wn<true>(v % kWnVariants, M, N, K, kchunk, split, 1.0, A, lda, B, ldb, 0.0, P, ldc, pstride, s, d_n);
+  const int wn = wn_of(v);
+  int* d_split = nullptr;   // behind the partial sums
+  if (!P) {
+    const long n = partials_doubles(M, N, K, ldc, wn, d_n != nullptr);
+    P = partials().get(static_cast<size_t>(n) + 1, s);
+    if (d_n) d_split = reinterpret_cast<int*>(P + n);
+  }
+  const int split = pick_split(M, N, K, wn);
+  launch_wn<true>(v, M, N, std::max(K, 0), split, true, 1.0, A, lda, B, ldb, 0.0, P, ldc, s, d_n, d_split);
   const long n = static_cast<long>(M) * N;
-  k_reduce_g0<<<ceil_div(n, 256), 256, 0, s>>>(M, N, split, P, pstride, alpha, g0, A, lda, B, ldb, scale, C, ldc,
-                                               d_n);
+  k_reduce_g0<<<ceil_div(n, 256), 256, 0, s>>>(M, N, split, P, 0, alpha, g0, A, lda, B, ldb, scale, C, ldc, d_n,
+                                               d_split);
   WH_HIP(hipGetLastError());
 }
 
@@ -565,7 +679,7 @@ static void dgemm_bra_skinny(int M, int N, int K, double alpha, const double* A,
   WH_HIP(hipGetLastError());
   const long n = static_cast<long>(M) * N;
   k_reduce_g0<<<ceil_div(n, 256), 256, 0, s>>>(M, N, split, P, pstride, alpha, g0, A, lda, B, ldb, scale, C, ldc,
-                                               d_n);
+                                               d_n, nullptr);
   WH_HIP(hipGetLastError());
 }
 
@@ -576,10 +690,10 @@ void dgemm_bra(int M, int N, int K, double alpha, const double* A, long lda, con
   // empty (with many columns the tiles' reuse of A wins again)
   if (M <= 32 && N <= 256 && K > 0)
     return dgemm_bra_skinny(M, N, K, alpha, A, lda, B, ldb, g0, scale, C, ldc, s, nullptr, d_n);
-  if (K <= 0 || N < 32) return dgemm_bra_own(M, N, K, alpha, A, lda, B, ldb, g0, scale, C, ldc, s, 0, nullptr, d_n);
-  // variants: K split depth (3) x tile width (3), timed once per (M, K, log2 N);
-  // C is written (not accumulated), so the timing runs on the call's own output
-  constexpr int nv = 3 * kWnVariants;
+  if (K <= 0 || N < 32) return dgemm_bra_own(M, N, K, alpha, A, lda, B, ldb, g0, scale, C, ldc, s, 2, nullptr, d_n);
+  // tile widths, timed once per (M, K, log2 N); C is written (not accumulated),
+  // so the timing runs on the call's own output
+  constexpr int nv = kWnVariants;
   auto run = [&](int v) { dgemm_bra_own(M, N, K, alpha, A, lda, B, ldb, g0, scale, C, ldc, s, v, nullptr, d_n); };
   const VariantKey key{1, 1, M, K, log2_bucket(N)};
   std::unique_lock<std::mutex> lk(g_variant_mutex);
@@ -589,8 +703,8 @@ void dgemm_bra(int M, int N, int K, double alpha, const double* A, long lda, con
     const int best = time_variants(nv, run, s, t);
     if (tune_log()) {
       std::fprintf(stderr, "[west_hip] dgemm_bra M=%d N=%d K=%d:", M, N, K);
-      for (int v = 0; v < nv; ++v) std::fprintf(stderr, " split%d/tile128x%d %.3f", 512 << (v / kWnVariants),
-                                                32 * wn_of(v % kWnVariants), t[v]);
+      for (int v = 0; v < nv; ++v) std::fprintf(stderr, " 128x%d split %d %.3f", 32 * wn_of(v),
+                                                pick_split(M, N, K, wn_of(v)), t[v]);
       std::fprintf(stderr, " ms -> %d\n", best);
     }
     it = chosen_variants().emplace(key, best).first;
@@ -607,35 +721,32 @@ void dgemm_bra(int M, int N, int K, double alpha, const double* A, long lda, con
 static_assert(kGroupTile == 64, "the grouped products run k_dgemm's WN = 2 tiles");
 
 template <bool TA>
-static void launch_groups(const DgemmGroups& G, int M, int N, int K, int kchunk, int gz, double alpha, long lda,
-                          const double* B, long ldb, double beta, double* C, long ldc, long pstride, hipStream_t s) {
+static void launch_groups(const DgemmGroups& G, int M, int N, int K, int split, bool partial, double alpha, long lda,
+                          const double* B, long ldb, double beta, double* C, long ldc, hipStream_t s) {
   const int gx = ceil_div(M, BM), gy = ceil_div(N, kGroupTile) + G.ng;
-  k_dgemm<TA, 2, true><<<xcd_blocks(gx * gy * gz), NT, 0, s>>>(M, N, K, kchunk, alpha, nullptr, lda, B, ldb, beta, C,
-                                                               ldc, pstride, gx, gy, gz, nullptr, G);
+  k_dgemm<TA, 2, true><<<xcd_blocks(gx * gy * split), NT, 0, s>>>(M, N, K, split, partial, alpha, nullptr, lda, B, ldb,
+                                                                  beta, C, ldc, gx, gy, nullptr, nullptr, G);
   WH_HIP(hipGetLastError());
 }
 
 void dgemm_bra_groups(const DgemmGroups& G, int M, int N, int K, long lda, const double* B, long ldb,
                       const double* scale, double* C, long ldc, hipStream_t s, const int* d_n) {
   if (M <= 0 || N <= 0) return;
-  // as bra_split, for the fewest tiles N columns can make
-  const int tiles = ceil_div(M, BM) * ceil_div(N, kGroupTile);
-  int split = std::max(1, std::min({64, ceil_div(512, tiles), K / (16 * BK)}));
-  const int kchunk = ceil_div(ceil_div(std::max(K, 1), split), BK) * BK;
-  split = ceil_div(std::max(K, 1), kchunk);
+  // as pick_split, for the fewest tiles N columns can make
+  const int split = pick_split(M, N, K, kGroupTile / 32);
   const long pstride = static_cast<long>(ldc) * N;
   double* P = partials().get(static_cast<size_t>(split) * pstride, s);
-  launch_groups<true>(G, M, N, K, kchunk, split, 1.0, lda, B, ldb, 0.0, P, ldc, pstride, s);
+  launch_groups<true>(G, M, N, K, split, true, 1.0, lda, B, ldb, 0.0, P, ldc, s);
   const long n = static_cast<long>(M) * N;
   k_reduce_g0<<<ceil_div(n, 256), 256, 0, s>>>(M, N, split, P, pstride, 1.0, 0.0, nullptr, 0, nullptr, 0, scale, C,
-                                               ldc, d_n);
+                                               ldc, d_n, nullptr);
   WH_HIP(hipGetLastError());
 }
 
 void dgemm_ket_groups(const DgemmGroups& G, int M, int N, int K, long lda, const double* B, long ldb, double beta,
                       double* C, long ldc, hipStream_t s) {
   if (M <= 0 || N <= 0) return;
-  launch_groups<false>(G, M, N, K, std::max(K, 1), 1, 1.0, lda, B, ldb, beta, C, ldc, 0, s);
+  launch_groups<false>(G, M, N, K, 1, false, 1.0, lda, B, ldb, beta, C, ldc, s);
 }
 
 // ---- products for callers that neither allocate nor time -------------------
@@ -647,9 +758,8 @@ static int chosen_or(const VariantKey& key, int dflt) {
 }
 
 static int bra_untimed_variant(int M, int N, int K) {
-  // default: K split aimed at 2048 workgroups on 128 x 64 tiles (the most
-  // frequent winner of the timing)
-  return (K <= 0 || N < 32) ? 0 : chosen_or(VariantKey{1, 1, M, K, log2_bucket(N)}, 7);
+  // default: 128 x 64 tiles (the most frequent winner of the timing)
+  return (K <= 0 || N < 32) ? 2 : chosen_or(VariantKey{1, 1, M, K, log2_bucket(N)}, 1);
 }
 
 long bra_partials_doubles(int M, int N, int K, long ldc, int* variant) {
@@ -660,7 +770,7 @@ long bra_partials_doubles(int M, int N, int K, long ldc, int* variant) {
     skinny_split(N, K, split, kchunk);
   } else {
     *variant = bra_untimed_variant(M, N, K);
-    bra_split(M, N, K, *variant, split, kchunk);
+    return partials_doubles(M, N, K, ldc, wn_of(*variant), false);
   }
   return static_cast<long>(split) * ldc * N;
 }
@@ -684,9 +794,9 @@ void dgemm_untimed(bool transa, int M, int N, int K, double alpha, const double*
       break;
     }
   const int v = chosen_or(VariantKey{0, transa ? 1 : 0, M, log2_bucket(std::max(K, 1)), log2_bucket(N)}, dflt);
-  const int K0 = std::max(K, 0), kc = std::max(K, 1);
-  if (transa) launch_wn<true>(v, M, N, K0, kc, 1, alpha, A, lda, B, ldb, beta, C, ldc, 0, s);
-  else launch_wn<false>(v, M, N, K0, kc, 1, alpha, A, lda, B, ldb, beta, C, ldc, 0, s);
+  const int K0 = std::max(K, 0);
+  if (transa) launch_wn<true>(v, M, N, K0, 1, false, alpha, A, lda, B, ldb, beta, C, ldc, s);
+  else launch_wn<false>(v, M, N, K0, 1, false, alpha, A, lda, B, ldb, beta, C, ldc, s);
 }
 
 void g0_fix_scale(int M, int N, double g0, const double* A, long lda, const double* B, long ldb,
