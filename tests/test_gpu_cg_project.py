@@ -1,0 +1,64 @@
+"""The CG iteration for few projector rows (operator by band, then one kernel)
+against the general iteration, at the edges of its register and row splits."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _state(cell, nr, nv, nproj, pad, seed):
+    from west_amd.groundstate import GroundState, from_real
+    from west_amd.gsphere import make_gamma_basis
+    b = make_gamma_basis(np.eye(3) * cell, 16.0, nr=(nr, nr, nr))
+    n = b.npw
+    rng = np.random.default_rng(seed)
+    # (33 rows whatever the pad, so that both sides get the same ones)
+    x = rng.normal(size=(2 * n - 1, nv + 33)) / (1.0 + np.concatenate([b.g2kin, b.g2kin[1:]]))[:, None]
+    rows = from_real(np.linalg.qr(x)[0].T.copy(), n, n, 2)[:nv + nproj + pad]
+    dvan = np.concatenate([0.1 + rng.random(33)[:nproj], np.zeros(pad)])
+    return GroundState(basis=b, npwx=n, vrs=np.random.default_rng(1).random(b.nnr), vkb=rows[nv:], dvan=dvan, evc=rows[:nv], et=np.zeros(nv),
+                       nbndval=nv, occ=np.ones(nv), weight=2.0, alpha_pv=1.0)
+
+
+# npw 258 to 9,200 (4 or 9 elements a thread of 1,024), 1 to 32 rows in groups of 1 to
+# 7, up to 256 columns; 33 rows (those added have coefficient zero) take the
+# general products
+@pytest.mark.parametrize("cell, nr, nv, nproj, m, kin", [
+    (8.0, 24, 1, 0, 1, False), (8.0, 24, 2, 1, 256, False), (14.2, 45, 2, 0, 3, False), (14.2, 45, 4, 3, 5, False),
+    (14.2, 45, 4, 5, 5, False), (14.2, 45, 16, 16, 7, False), (19.5, 54, 5, 0, 2, False), (19.5, 54, 4, 0, 1, True),
+    (19.8, 54, 1, 0, 2, False), (19.8, 54, 2, 0, 1, False), (19.8, 54, 6, 0, 3, False), (25.7, 72, 4, 1, 2, False),
+    (25.7, 72, 20, 11, 2, True)])
+def test_linsolve(gpu, cell, nr, nv, nproj, m, kin):
+    if kin:   # the bands are the only rows
+        nproj = 0
+    tr2 = 1e-20
+    out = []
+    for pad in (0, 33 - nproj):
+        gs = _state(cell, nr, nv, nproj, pad, 7)
+        # (kinetic only: bands beyond nv, with no column of their own, cannot be added; the dense solution instead)
+        gpu.set_ground_state(gs, l_kinetic_only=kin)
+        rng = np.random.default_rng(m)
+        b = (rng.normal(size=(m, gs.npwx)) + 1j * rng.normal(size=(m, gs.npwx))) / (1.0 + gs.basis.g2kin)
+        b[:, 0] = b[:, 0].real
+        x = np.zeros_like(b)
+        e = -0.5 - rng.random(m)
+        assert gpu.linsolve_sternheimer_m_wfcts(nv, m, b.copy(), x, e, np.full(m, 1.5), tr2) == 0
+        out.append(x)
+        if kin:
+            # (g2 - e) x + sum_v |v><v|x> = b, by the small system of <v|x>
+            d = 1.0 / (gs.basis.g2kin[None] - e[:, None])
+
+            def dot(u, w):
+                return 2.0 * (u.real @ w.real.T + u.imag @ w.imag.T) - np.outer(u[:, 0].real, w[:, 0].real)
+
+            ref = np.zeros_like(b)
+            for i in range(m):
+                w = gs.evc * d[i]
+                c = np.linalg.solve(np.eye(nv) + dot(gs.evc, w), dot(gs.evc, (d[i] * b[i])[None])[:, 0])
+                ref[i] = d[i] * b[i] - c @ w
+            out.append(ref)
+            break
+    # <M^-1 r|r> < 1e-20 in each solve, M <= 16/1.5 and the operator above 0.5:
+    # each is within sqrt(1e-20 11) / 0.5 = 7e-10 of the solution (two-norm)
+    err = np.sqrt(2.0 * np.sum(np.abs(out[0] - out[1]) ** 2, axis=1))
+    assert err.max() <= 1.4e-9

@@ -46,15 +46,6 @@ Context& ctx() {
   return *c;
 }
 
-// true when this process holds one system: a stream capture must then not
-// meet another thread's device-wide synchronisation
-static bool single_system() {
-  std::lock_guard<std::mutex> lk(g_sys_mutex);
-  int n = 0;
-  for (Context* c : g_sys) n += c != nullptr;
-  return n == 1;
-}
-
 static Context* new_context(int device) {
   Context* c = new Context();
   c->device = device;
@@ -226,6 +217,25 @@ void glbrak_q(int row0, int nq, const z64* f, int m, double* cmat) {
 //   (DFPT_kernel/apply_sternheimerop_to_m_wfcs.f90:49-76; QE h_psi_ at Gamma:
 //    kinetic + vloc_psi + calbec/add_vuspsi)
 // ---------------------------------------------------------------------------
+
+// its local part, kinetic energy and -e, by pairs of rows; plane items by pair
+// (dev) or the same chunk of them every time
+static void vloc_pairs(const z64* x, z64* t, const double* d_e, FftItem* items, FftItem* ident, int npair, int chunk,
+                       bool dev, const SternWs* ws) {
+  Context& c = ctx();
+  hipStream_t s = c.stream;
+  const long ld = c.npw;
+  z64* sa = ws ? ws->sa : c.w_sticks_a.as<z64>(static_cast<size_t>(chunk) * c.plan.sticks_elems());
+  z64* sb = ws ? ws->sb : c.w_sticks_b.as<z64>(static_cast<size_t>(chunk) * c.plan.sticks_elems());
+  ZfwdArgs za{ZFWD_PAIR_STERN, 1.0, c.d_g2kin, d_e, nullptr, 0};
+  for (int q0 = 0; q0 < npair; q0 += chunk) {
+    const int nq = std::min(chunk, npair - q0);
+    WH_TIMED("zinv", launch_zinv(c.plan, items + q0, nq, x, ld, sa, ZINV_PAIR, s));
+    WH_TIMED("plane_vloc", launch_plane_vloc(c.plan, dev ? ident + q0 : ident, nq, sa, sb, c.d_vrs, 0, 1.0 / c.nnr, s));
+    WH_TIMED("zfwd", launch_zfwd(c.plan, items + q0, nq, sb, x, ld, t, ld, za, s));
+  }
+}
+
 void stern_apply(const z64* x, z64* t, const double* d_e, int m, double alpha, const SternWs* ws,
                  const int* d_nc) {
   Context& c = ctx();
@@ -237,30 +247,15 @@ void stern_apply(const z64* x, z64* t, const double* d_e, int m, double alpha, c
     WH_TIMED("kinetic", kinetic_minus_e(m, npw, x, t, ld, c.d_g2kin, d_e, s));
   } else {
     const int npair = (m + 1) / 2;
-    const int cap = ws ? ws->chunk : c.items_capacity();
-    const int chunk = std::min(cap, npair);
+    const int chunk = ws ? std::min(ws->chunk, npair) : std::min(c.items_capacity(), npair);
+    // (with d_nc, cg_select has made the items)
     FftItem* items = ws ? ws->items : c.w_items.as<FftItem>(npair);
-    FftItem* ident = nullptr;
-    if (d_nc) {
-      // items of the inactive tail are switched off on the device
-      fill_pairs_dev(items, npair, d_nc, s);
-      ident = c.w_items_id.as<FftItem>(npair);
-      fill_ident_dev(ident, npair, chunk, d_nc, s);
-    } else {
+    FftItem* ident = ws ? ws->ident : c.w_items_id.as<FftItem>(d_nc ? npair : chunk);
+    if (!d_nc) {
       fill_pairs(items, m, 0, s);
-      ident = ws ? ws->ident : c.w_items_id.as<FftItem>(chunk);
       fill_ident(ident, chunk, s);
     }
-    z64* sa = ws ? ws->sa : c.w_sticks_a.as<z64>(static_cast<size_t>(chunk) * c.plan.sticks_elems());
-    z64* sb = ws ? ws->sb : c.w_sticks_b.as<z64>(static_cast<size_t>(chunk) * c.plan.sticks_elems());
-    ZfwdArgs za{ZFWD_PAIR_STERN, 1.0, c.d_g2kin, d_e, nullptr, 0};
-    for (int q0 = 0; q0 < npair; q0 += chunk) {
-      const int nq = std::min(chunk, npair - q0);
-      WH_TIMED("zinv", launch_zinv(c.plan, items + q0, nq, x, ld, sa, ZINV_PAIR, s));
-      WH_TIMED("plane_vloc", launch_plane_vloc(c.plan, d_nc ? ident + q0 : ident, nq, sa, sb, c.d_vrs, 0,
-                                               1.0 / c.nnr, s));
-      WH_TIMED("zfwd", launch_zfwd(c.plan, items + q0, nq, sb, x, ld, t, ld, za, s));
-    }
+    vloc_pairs(x, t, d_e, items, ident, npair, chunk, d_nc != nullptr, ws);
   }
   // projector part: rows [evc ; vkb] (or evc only for the kinetic-only operator)
   const int nq = c.l_kinetic_only ? c.nbndval : c.nbndval + c.nkb;
@@ -324,7 +319,6 @@ int linsolve_dev(int m, z64* b, z64* x, const std::vector<double>& e_col, const 
   double* d_rhoold = c.w_rho.as<double>(m);
   int* d_conv = c.w_conv.as<int>(static_cast<size_t>(m) + 4);
   int* d_nc = d_conv + m;       // active count of the current iteration
-  int* d_rec = d_conv + m + 1;  // (active count, perturbations among them)
   const RhoOut rho_out{c.d_g2kin, d_eprec_col, d_rhob};
   const int itmax = maxiter > 0 ? maxiter : c.n_dfpt_maxiter;
   // one record per iteration, read by the host two iterations late
@@ -336,6 +330,20 @@ int linsolve_dev(int m, z64* b, z64* x, const std::vector<double>& e_col, const 
   axpby(static_cast<long>(vec), -1.0, b, 1.0, g, s);
   iota(d_l2i, m, s);
   WH_TIMED("cg_prec", prec_rho(m, npw, c.gstart, d_l2i, g, ld, c.d_g2kin, d_eprec_col, d_rhob, s, true));
+  const int nqp = c.l_kinetic_only ? c.nbndval : c.nbndval + c.nkb;
+  // few projector rows: the operator's local part by band, then one kernel
+  const bool project = cg_project_fits(nqp, m, npw);
+  if (project) {
+    // the first direction (beta = 0)
+    WH_HIP(hipMemsetAsync(d_beta, 0, sizeof(double) * m, s));
+    WH_TIMED("cg_dir", direction(m, npw, d_l2i, d_beta, g, c.d_g2kin, d_eprec_col, h, h, tc, ld, s));
+  }
+  // the operator's work items, made by cg_select
+  const int mpair = c.l_kinetic_only ? 0 : (m + 1) / 2;
+  CgSelect sel{};
+  sel.items = c.w_items.as<FftItem>(mpair);
+  sel.ident = c.w_items_id.as<FftItem>(mpair);
+  sel.by_band = project;
   // The loop (linsolve_sternheimer_m_wfcts.f90:146-330) runs on the device:
   // each iteration starts with cg_select (convergence test, compaction,
   // beta), and its kernels are launched for a capacity -- the active count
@@ -345,21 +353,9 @@ int linsolve_dev(int m, z64* b, z64* x, const std::vector<double>& e_col, const 
   // finished while the next one is queued), to size the launches and to stop
   // once a count of zero is seen; iterations launched after the last band
   // converged do nothing.
-  // Narrow batches (every product a streaming kernel, launch-bound) replay
-  // an iteration captured in a HIP graph the second time the same capacity
-  // and h/hold assignment come up; WH_GRAPH=0 keeps every iteration eager;
-  // so do the profiler's timed mode and a process holding several systems
-  // (their threads' device-wide synchronisations may not meet a capture).
-  const int nqp = c.l_kinetic_only ? c.nbndval : c.nbndval + c.nkb;
-  const char* genv = std::getenv("WH_GRAPH");
-  const bool graphs = !(genv && genv[0] == '0') && !c.prof.on && nqp <= 32 && m <= 256 && single_system();
-  struct CgGraph {
-    int cap;
-    const void* h;
-    hipGraphExec_t exec;
-  };
-  std::vector<CgGraph> cg_graphs;
-  std::vector<std::pair<int, const void*>> eager_seen;
+  // Few projector rows: five launches an iteration (replaying them as a
+  // captured graph was slower than queueing them: 2.72 against 2.47 ms for a
+  // solve of 35 bands on 50^3 points).
   hipEvent_t ev[3];
   for (hipEvent_t& e : ev) WH_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   int last = 0;   // iterations launched
@@ -374,42 +370,29 @@ int linsolve_dev(int m, z64* b, z64* x, const std::vector<double>& e_col, const 
       cap = std::min(m, p2);
     }
     const int first = iter == 1 ? 1 : 0;
-    auto body = [&]() {
-      WH_TIMED("cg_select", cg_select(m, tr2, first, group, d_rhob, d_rhoold, d_conv, d_e_col, d_l2i, d_beta, d_eu,
-                                      d_nc, d_rec, s));
+    const int npair = mpair ? (cap + 1) / 2 : 0;
+    sel.rec = rec + 2 * iter;
+    sel.npair = npair;
+    sel.chunk = std::max(1, std::min(c.items_capacity(), npair));
+    WH_TIMED("cg_select", cg_select(m, tr2, first, group, d_rhob, d_rhoold, d_conv, d_e_col, d_l2i, d_beta, d_eu, d_nc,
+                                    sel, s));
+    if (project) {
+      // (kinetic only: all m bands, the converged ones' rows are not used)
+      if (c.l_kinetic_only) kinetic_minus_e(m, npw, h, tc, ld, c.d_g2kin, d_e_col, s);
+      else vloc_pairs(h, tc, d_e_col, sel.items, sel.ident, npair, sel.chunk, true, nullptr);
+      WH_TIMED("cg_project", cg_project(cap, npw, c.gstart, nqp, d_l2i, c.d_q, c.d_qscale, h, g, tc, x, c.d_g2kin,
+                                        d_eprec_col, d_rhob, d_nc, s));
+    } else {
       WH_TIMED("cg_dir", direction(cap, npw, d_l2i, d_beta, g, c.d_g2kin, d_eprec_col, h, hold, bc, ld, s, d_nc));
       stern_apply(bc, tc, d_eu, cap, c.alpha_pv, nullptr, d_nc);
       WH_TIMED("cg_update", cg_update(cap, npw, c.gstart, d_l2i, h, g, tc, x, ld, nullptr, s, &rho_out, d_nc));
-    };
-    const CgGraph* cached = nullptr;
-    for (const CgGraph& gr : cg_graphs)
-      if (gr.cap == cap && gr.h == h) cached = &gr;
-    const std::pair<int, const void*> key{cap, h};
-    if (cached && !first) {
-      WH_HIP(hipGraphLaunch(cached->exec, s));
-    } else if (graphs && !first &&
-               std::find(eager_seen.begin(), eager_seen.end(), key) != eager_seen.end()) {
-      hipGraph_t graph = nullptr;
-      WH_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeRelaxed));
-      body();
-      WH_HIP(hipStreamEndCapture(s, &graph));
-      hipGraphExec_t exec = nullptr;
-      WH_HIP(hipGraphInstantiateWithFlags(&exec, graph, 0));
-      WH_HIP(hipGraphDestroy(graph));
-      cg_graphs.push_back({cap, h, exec});
-      WH_HIP(hipGraphLaunch(exec, s));
-    } else {
-      body();
-      if (!first) eager_seen.push_back(key);
+      std::swap(h, hold);   // hold <- h  (linsolve 319)
     }
-    WH_HIP(hipMemcpyAsync(rec + 2 * iter, d_rec, 2 * sizeof(int), hipMemcpyDeviceToHost, s));
     WH_HIP(hipEventRecord(ev[iter % 3], s));
     last = iter;
-    std::swap(h, hold);   // hold <- h  (linsolve 319)
   }
   WH_HIP(hipStreamSynchronize(s));
   for (hipEvent_t e : ev) WH_HIP(hipEventDestroy(e));
-  for (const CgGraph& gr : cg_graphs) WH_HIP(hipGraphExecDestroy(gr.exec));
   // counters: an iteration counts when it had active bands
   for (int it = 1; it <= last; ++it) {
     const int n = rec[2 * it];

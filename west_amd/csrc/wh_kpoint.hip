@@ -820,7 +820,6 @@ static int linsolve_k(KPath& K, int ik, int nkb, int cols, z64* b, z64* x, const
   double* d_eu = K.w_eu.as<double>(m);
   int* d_conv = K.w_conv.as<int>(static_cast<size_t>(m) + 4);
   int* d_nc = d_conv + m;       // active count of the current iteration
-  int* d_rec = d_conv + m + 1;  // (active count, perturbations among them)
   if (!K.cg_ev[0])
     for (hipEvent_t& e : K.cg_ev) WH_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   const int itmax = c.n_dfpt_maxiter;
@@ -864,7 +863,7 @@ static int linsolve_k(KPath& K, int ik, int nkb, int cols, z64* b, z64* x, const
       cap = std::min(m, p2);
     }
     // convergence test, compaction, beta (208-224)
-    cg_select(m, tr2, it == 1 ? 1 : 0, group, d_rhob, d_rhoold, d_conv, d_e, d_l2i, d_beta, d_eu, d_nc, d_rec, s);
+    cg_select(m, tr2, it == 1 ? 1 : 0, group, d_rhob, d_rhoold, d_conv, d_e, d_l2i, d_beta, d_eu, d_nc, CgSelect{rec + 2 * it}, s);
     if (fused) {
       WH_TIMED("cg_iter_lds", cg_iter_rows(K.plan, nkb > 1 ? K.stab : K.stab + ik, false, cap, ca, s));
     } else {
@@ -875,7 +874,6 @@ static int linsolve_k(KPath& K, int ik, int nkb, int cols, z64* b, z64* x, const
       k_cg_step<<<cap, NT, 0, s>>>(d_l2i, d_nc, P.npw, ld, P.g2kin, d_ep, x, g, h, tc, hold, d_rhob, tab, cols);
       WH_HIP(hipGetLastError());
     }
-    WH_HIP(hipMemcpyAsync(rec + 2 * it, d_rec, 2 * sizeof(int), hipMemcpyDeviceToHost, s));
     WH_HIP(hipEventRecord(K.cg_ev[it % (kCgLag + 1)], s));
     last = it;
   }

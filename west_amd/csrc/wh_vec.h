@@ -60,15 +60,28 @@ void fill_pairs(FftItem* items, int m, int row0, hipStream_t s);
 // one workgroup marks bands whose rho < tr2 as converged, compacts the rest
 // into l2i (ascending band order) with beta = rho / rhoold (0 on the first
 // iteration) and e, sets rhoold = rho for them, and writes the active count
-// to *nc and rec[0], and to rec[1] the perturbations among them (groups of
-// `group` consecutive bands; group <= 0: one)
+// to *nc and with the perturbations among them (groups of `group` consecutive
+// bands; group <= 0: one) to sel.rec
+struct CgSelect {
+  int* rec = nullptr;   // (active count, perturbations), pinned host memory
+  // work items of npair pairs of columns and of their sticks in chunks (none: npair 0)
+  FftItem* items = nullptr;
+  FftItem* ident = nullptr;
+  int npair = 0, chunk = 1;
+  bool by_band = false;   // items: band numbers, not compacted columns
+};
 void cg_select(int m, double tr2, int first, int group, const double* rhob, double* rhoold, int* conv,
-               const double* e_col, int* l2i, double* beta, double* eu, int* nc, int* rec, hipStream_t s);
-// pair items (2i, 2i+1) of the first *nc rows, inactive (a = -1) beyond, for cap items
-void fill_pairs_dev(FftItem* items, int cap, const int* nc, hipStream_t s);
-// plane items of chunked launches: item q -> sticks slot q % chunk while q
-// is below the active pair count of *nc rows, inactive beyond (cap items)
-void fill_ident_dev(FftItem* items, int cap, int chunk, const int* nc, hipStream_t s);
+               const double* e_col, int* l2i, double* beta, double* eu, int* nc, const CgSelect& sel, hipStream_t s);
+// The rest of an iteration after the local operator (t by band, not stored
+// again) for nq <= kCgProjRows projector rows, m <= 256 columns (one workgroup
+// a compute unit; with more, the matrix-core products share their reads of the
+// rows) and a band in the registers of 1,024 threads: projectors, update, rho
+// and the next direction in h.
+constexpr int kCgProjRows = 32;
+bool cg_project_fits(int nq, int m, int npw);
+void cg_project(int nc, int npw, int gstart, int nq, const int* l2i, const z64* q, const double* scale, z64* h, z64* g,
+                const z64* t, z64* x, const double* g2kin, const double* eprec, double* rho, const int* d_nc,
+                hipStream_t s);
 void iota(int* v, int n, hipStream_t s);
 void fill_ident(FftItem* items, int n, hipStream_t s);
 void eprec_of(int nb, int npw, const z64* evc, long ld, const double* g2kin, double* eprec, hipStream_t s);

@@ -5,6 +5,8 @@
 // (DFPT_kernel/linsolve_sternheimer_m_wfcts.f90:162-181, 253-276).
 #include "wh_vec.h"
 
+#include <type_traits>
+
 namespace wh {
 
 namespace {
@@ -199,6 +201,166 @@ __global__ __launch_bounds__(NTU) void k_cg_update_reg(int npw, int gstart, cons
   }
 }
 
+// R values summed over the wavefront: lane l returns the sum of v[l % R].
+// (log2 R exchange steps halve the values, the rest carry one: 10 exchanges
+// for eight sums instead of 48.)
+template <int R>
+__device__ __forceinline__ double wave_sums(double (&v)[R]) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int n = R / 2; n > 0; n >>= 1) {
+    const bool up = lane & n;
+#pragma unroll
+    for (int i = 0; i < n; ++i) {
+      const double send = up ? v[i] : v[i + n];
+      const double keep = up ? v[i + n] : v[i];
+      v[i] = keep + __shfl_xor(send, n, 64);
+    }
+  }
+  double t = v[0];
+#pragma unroll
+  for (int o = R; o < 64; o <<= 1) t += __shfl_xor(t, o, 64);
+  return t;
+}
+
+// a value that is the same in every lane, in scalar registers
+__device__ __forceinline__ double uniform(double v) {
+  const long b = __double_as_longlong(v);
+  const unsigned lo = __builtin_amdgcn_readfirstlane(static_cast<int>(b));
+  const unsigned hi = __builtin_amdgcn_readfirstlane(static_cast<int>(b >> 32));
+  return __longlong_as_double(static_cast<long>((static_cast<unsigned long>(hi) << 32) | lo));
+}
+
+// One band's share of a CG iteration after the local part of the operator, for
+// few projector rows: t += Q s (Q^T h) (the projector part), a = <h|g>,
+// c = <h|t>, x -= (a/c) h, g -= (a/c) t, rho = <M^-1 g|g> and the next
+// direction h <- -M^-1 g + (rho / rho_old) h, one workgroup a band with h and
+// M^-1 g in registers.  <h|Q s Q^T h> is the sum of s_i (Q_i^T h)^2, so t is complete
+// only in the second pass and never stored.  (kCgProjRows rows: their two
+// passes come from the L2 and cost 2 npw rows 16 bytes a band.)
+// Bound: one compute unit's load path (64 bytes a cycle; the rows twice and
+// nine passes of the vectors) and three block-wide sums.  Before, the same work
+// was the products' three launches, the update and the direction: 35 bands, 7
+// rows, npw = 3,761: 12.2 + 4.3 + 4.5 + 8.9 + 4.1 -> 18 us; 192 bands, 6 rows,
+// npw = 6,147: 10.3 + 4.9 + 7.5 + 16.7 + 8.5 -> 31 us; and four gaps less.
+// Rows in groups of RG; beyond nq the last one is repeated and not used.
+template <int E, int RG>
+__global__ __launch_bounds__(NTU) void k_cg_project(unsigned npw, int gstart, int nq, const int* l2i, const z64* q,
+                                                   const double* scale, z64* h, z64* g, const z64* t, z64* x,
+                                                   const double* g2kin, const double* eprec, double* rho,
+                                                   const int* d_nc) {
+  constexpr int NW = NTU / 64;
+  auto row = [&](int r) { return q + static_cast<long>(min(r, nq - 1)) * npw; };
+  __shared__ double red[NW][kCgProjRows + 2];
+  __shared__ double cs[kCgProjRows], cp[kCgProjRows];
+  const int lb = blockIdx.x;
+  if (lb >= *d_nc) return;   // uniform per workgroup
+  const int ib = __builtin_amdgcn_readfirstlane(l2i[lb]);   // (scalar row addresses)
+  const long o = static_cast<long>(ib) * npw;
+  h += o;
+  g += o;
+  t += o;
+  x += o;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  z64 hv[E], pv[E];
+  double d[2] = {0.0, 0.0};
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const unsigned i = tid + e * NTU;
+    hv[e] = mk(0.0, 0.0);
+    if (i < npw) {
+      hv[e] = h[i];
+      const z64 gq = g[i], tq = t[i];
+      d[0] += hv[e].x * gq.x + hv[e].y * gq.y;
+      d[1] += hv[e].x * tq.x + hv[e].y * tq.y;
+    }
+    if (E > 4 && e % 3 == 2) __builtin_amdgcn_sched_barrier(0);   // no more loads ahead than registers for them
+  }
+  const double h0 = uniform(gstart == 2 ? h[0].x : 0.0);
+  const double g0 = uniform(g[0].x), t0 = uniform(t[0].x), rho_old = uniform(rho[ib]), ep = uniform(eprec[ib]);
+  const double dw = wave_sums<2>(d);
+  if (lane < 2) red[w][kCgProjRows + lane] = dw;
+#pragma unroll 1
+  for (int r0 = 0; r0 < nq; r0 += RG) {
+    constexpr int R2 = RG > 4 ? 8 : RG > 2 ? 4 : RG;
+    double p[R2];
+#pragma unroll
+    for (int r = 0; r < R2; ++r) p[r] = 0.0;
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      // beyond npw h is zero: any element of the row may be read
+      const unsigned i = min(static_cast<unsigned>(tid + e * NTU), npw - 1u);
+#pragma unroll
+      for (int r = 0; r < RG; ++r) {
+        const z64 v = row(r0 + r)[i];
+        p[r] += v.x * hv[e].x + v.y * hv[e].y;
+      }
+      if (E > 4 || e % 2) __builtin_amdgcn_sched_barrier(0);
+    }
+    const double pw = wave_sums<R2>(p);
+    if (lane < R2 && r0 + lane < kCgProjRows) red[w][r0 + lane] = pw;
+  }
+  __syncthreads();   // also: every thread has read h[0] and g[0]
+  if (tid < nq) {
+    double v = 0.0;
+    for (int k = 0; k < NW; ++k) v += red[k][tid];
+    v = 2.0 * v - h0 * q[static_cast<long>(tid) * npw].x;
+    cs[tid] = scale[tid] * v;
+    cp[tid] = v;
+  }
+  double a = 0.0, c = 0.0;
+  for (int k = 0; k < NW; ++k) {
+    a += red[k][kCgProjRows];
+    c += red[k][kCgProjRows + 1];
+  }
+  __syncthreads();
+  a = 2.0 * a - h0 * g0;
+  c = 2.0 * c - h0 * t0;
+  for (int r = 0; r < nq; ++r) c += cs[r] * cp[r];
+  const double step = uniform(a / c);
+  double s[2] = {0.0, 0.0};
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const unsigned i = tid + e * NTU;
+    if (i < npw) {
+      z64 tq = t[i];   // (again, from the L2: held through the first pass it would spill)
+#pragma unroll 1
+      for (int r0 = 0; r0 < nq; r0 += RG) {
+#pragma unroll
+        for (int r = 0; r < RG; ++r) {
+          const z64 v = row(r0 + r)[i];
+          const double f = r0 + r < nq ? uniform(cs[r0 + r]) : 0.0;
+          tq.x += f * v.x;
+          tq.y += f * v.y;
+        }
+      }
+      const z64 xv = x[i], gv = g[i];
+      x[i] = mk(xv.x - step * hv[e].x, xv.y - step * hv[e].y);
+      const z64 gn = mk(gv.x - step * tq.x, gv.y - step * tq.y);
+      g[i] = gn;
+      const double f = 1.0 / fmax(1.0, g2kin[i] / ep);
+      pv[e] = mk(gn.x * f, gn.y * f);   // M^-1 g
+      s[0] += pv[e].x * gn.x + pv[e].y * gn.y;
+      if (i == 0) s[1] = pv[e].x * gn.x;
+    }
+    if (E > 4) __builtin_amdgcn_sched_barrier(0);
+  }
+  const double sw = wave_sums<2>(s);
+  // (the first sums' last readers are behind the barrier above)
+  if (lane < 2) red[w][lane] = sw;
+  __syncthreads();
+  double r = 0.0;
+  for (int k = 0; k < NW; ++k) r += red[k][0];
+  r = 2.0 * r - (gstart == 2 ? red[0][1] : 0.0);   // element 0 is thread 0's
+  if (tid == 0) rho[ib] = r;
+  const double beta = r / rho_old;
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const unsigned i = tid + e * NTU;
+    if (i < npw) h[i] = mk(-pv[e].x + beta * hv[e].x, -pv[e].y + beta * hv[e].y);
+  }
+}
+
 // out[r][s] = in[r][perm[s]] * (w ? w[s] : 1)     caller order -> stick order
 __global__ void k_gather(int m, int npw, const int* perm, const z64* in, long ldin, z64* out, long ldout,
                          const double* w) {
@@ -338,30 +500,6 @@ __global__ void k_fill_pairs(FftItem* items, int n, int m, int row0) {
   items[q] = it;
 }
 
-__global__ void k_fill_pairs_dev(FftItem* items, int cap, const int* nc) {
-  const int q = blockIdx.x * NT + threadIdx.x;
-  if (q >= cap) return;
-  const int m = *nc;
-  FftItem it;
-  it.a = (2 * q < m) ? 2 * q : -1;
-  it.b = (2 * q + 1 < m) ? 2 * q + 1 : -1;
-  it.pot = -1;
-  it.pad = 0;
-  items[q] = it;
-}
-
-__global__ void k_fill_ident_dev(FftItem* items, int cap, int chunk, const int* nc) {
-  const int q = blockIdx.x * NT + threadIdx.x;
-  if (q >= cap) return;
-  const int npair = (*nc + 1) / 2;
-  FftItem it;
-  it.a = q < npair ? q % chunk : -1;
-  it.b = -1;
-  it.pot = -1;
-  it.pad = 0;
-  items[q] = it;
-}
-
 __global__ void k_iota(int* v, int n) {
   const int q = blockIdx.x * NT + threadIdx.x;
   if (q < n) v[q] = q;
@@ -370,14 +508,17 @@ __global__ void k_iota(int* v, int n) {
 // Convergence test, compaction and coefficients of one CG iteration on the
 // device (linsolve_sternheimer_m_wfcts.f90:190-240): one workgroup walks the
 // bands in order, so the active list keeps the ascending band order of
-// map_lbnd2ibnd.
+// map_lbnd2ibnd.  Along with it, the operator's work items of the launch's
+// sel.npair pairs of columns (switched off beyond the active ones): the columns
+// are the compacted ones, or (by_band) the bands themselves.  The count goes to
+// sel.rec (host memory: the host reads it without a copy in between).
 constexpr int NTS_SEL = 1024;
 __global__ __launch_bounds__(NTS_SEL) void k_cg_select(int m, double tr2, int first, int group,
                                                        const double* __restrict__ rhob, double* __restrict__ rhoold,
                                                        int* __restrict__ conv, const double* __restrict__ e_col,
                                                        int* __restrict__ l2i, double* __restrict__ beta,
                                                        double* __restrict__ eu, int* __restrict__ nc_out,
-                                                       int* __restrict__ rec) {
+                                                       CgSelect sel) {
   __shared__ int wcount[NTS_SEL / 64];
   __shared__ int base_s;
   __shared__ int calls_w[NTS_SEL / 64];
@@ -417,6 +558,19 @@ __global__ __launch_bounds__(NTS_SEL) void k_cg_select(int m, double tr2, int fi
     __syncthreads();
   }
   const int nc = base_s;
+  const int npair = (nc + 1) / 2;
+  for (int q = tid; q < sel.npair; q += NTS_SEL) {
+    const int a = 2 * q, b = 2 * q + 1;
+    FftItem it;
+    it.pot = -1;
+    it.pad = 0;
+    it.a = a < nc ? (sel.by_band ? l2i[a] : a) : -1;
+    it.b = b < nc ? (sel.by_band ? l2i[b] : b) : -1;
+    sel.items[q] = it;
+    it.a = q < npair ? q % sel.chunk : -1;
+    it.b = -1;
+    sel.ident[q] = it;
+  }
   // perturbations among the active bands (the list is ascending)
   int calls = 0;
   for (int pos = tid; pos < nc; pos += NTS_SEL) {
@@ -431,8 +585,8 @@ __global__ __launch_bounds__(NTS_SEL) void k_cg_select(int m, double tr2, int fi
     int tot = 0;
     for (int k = 0; k < NTS_SEL / 64; ++k) tot += calls_w[k];
     *nc_out = nc;
-    rec[0] = nc;
-    rec[1] = tot;
+    __hip_atomic_store(sel.rec, nc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(sel.rec + 1, tot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
 
@@ -527,6 +681,37 @@ void cg_update(int nc, int npw, int gstart, const int* l2i, const z32* h, z32* g
   cg_update_any<float>(nc, npw, gstart, l2i, h, g, tc, x, ld, ac_out, rho, s, nullptr);
 }
 
+bool cg_project_fits(int nq, int m, int npw) { return nq <= kCgProjRows && m <= 256 && npw <= 9 * NTU; }
+
+void cg_project(int nc, int npw, int gstart, int nq, const int* l2i, const z64* q, const double* scale, z64* h, z64* g,
+                const z64* t, z64* x, const double* g2kin, const double* eprec, double* rho, const int* d_nc,
+                hipStream_t s) {
+  if (nc <= 0) return;
+  WH_REQUIRE(cg_project_fits(nq, nc, npw), "cg_project: outside the kernel's range");
+  // groups of rows that leave none over, as far as the registers go
+  auto run = [&](auto e, auto rg) {
+    k_cg_project<decltype(e)::value, decltype(rg)::value><<<nc, NTU, 0, s>>>(npw, gstart, nq, l2i, q, scale, h, g, t, x,
+                                                                             g2kin, eprec, rho, d_nc);
+  };
+  using std::integral_constant;
+  const integral_constant<int, 4> e4;
+  const integral_constant<int, 9> e9;
+  if (npw <= 4 * NTU) {
+    if (nq <= 1) run(e4, integral_constant<int, 1>());
+    else if (nq == 2) run(e4, integral_constant<int, 2>());
+    else if (nq == 5) run(e4, integral_constant<int, 5>());
+    else if (nq == 7) run(e4, integral_constant<int, 7>());
+    else if (nq % 3 == 0) run(e4, integral_constant<int, 3>());
+    else run(e4, integral_constant<int, 4>());
+  } else {
+    if (nq <= 1) run(e9, integral_constant<int, 1>());
+    else if (nq == 2) run(e9, integral_constant<int, 2>());
+    else if (nq % 3 == 0) run(e9, integral_constant<int, 3>());
+    else run(e9, integral_constant<int, 4>());
+  }
+  WH_HIP(hipGetLastError());
+}
+
 void gather_sticks(int m, int npw, const int* perm, const z64* in, long ldin, z64* out, long ldout, const double* w,
                    hipStream_t s) {
   if (m <= 0) return;
@@ -619,18 +804,6 @@ void fill_pairs(FftItem* items, int m, int row0, hipStream_t s) {
   WH_HIP(hipGetLastError());
 }
 
-void fill_pairs_dev(FftItem* items, int cap, const int* nc, hipStream_t s) {
-  if (cap <= 0) return;
-  k_fill_pairs_dev<<<ceil_div(cap, NT), NT, 0, s>>>(items, cap, nc);
-  WH_HIP(hipGetLastError());
-}
-
-void fill_ident_dev(FftItem* items, int cap, int chunk, const int* nc, hipStream_t s) {
-  if (cap <= 0) return;
-  k_fill_ident_dev<<<ceil_div(cap, NT), NT, 0, s>>>(items, cap, chunk, nc);
-  WH_HIP(hipGetLastError());
-}
-
 void iota(int* v, int n, hipStream_t s) {
   if (n <= 0) return;
   k_iota<<<ceil_div(n, NT), NT, 0, s>>>(v, n);
@@ -638,8 +811,8 @@ void iota(int* v, int n, hipStream_t s) {
 }
 
 void cg_select(int m, double tr2, int first, int group, const double* rhob, double* rhoold, int* conv,
-               const double* e_col, int* l2i, double* beta, double* eu, int* nc, int* rec, hipStream_t s) {
-  k_cg_select<<<1, NTS_SEL, 0, s>>>(m, tr2, first, group, rhob, rhoold, conv, e_col, l2i, beta, eu, nc, rec);
+               const double* e_col, int* l2i, double* beta, double* eu, int* nc, const CgSelect& sel, hipStream_t s) {
+  k_cg_select<<<1, NTS_SEL, 0, s>>>(m, tr2, first, group, rhob, rhoold, conv, e_col, l2i, beta, eu, nc, sel);
   WH_HIP(hipGetLastError());
 }
 
