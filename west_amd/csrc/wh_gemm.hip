@@ -11,16 +11,18 @@
 // Tile 128 x (32 WN) x 16 per 256-thread workgroup (WN = 4, 2 or 1): four
 // wavefronts in a 2 x 2 arrangement, each owning 64 x 16 WN = 4 x WN MFMA
 // 16x16 blocks.  One tile is multiplied out of LDS while the next goes from
-// registers to the other half of the double buffer and the one after is on its
-// way from memory; both are issued between the two halves of the K steps, so
-// neither is waited for at the barrier.  Bound: the FP64 matrix pipe (64
-// cycles an instruction and SIMD); what is left is the address and LDS work
+// registers to the other half of the double buffer and the ones after are on
+// their way from memory; both are issued between the two halves of the K
+// steps, so neither is waited for at the barrier.  Bound: the FP64 matrix pipe
+// (64 cycles an instruction and SIMD); what is left is the address and LDS work
 // between the matrix instructions, so tiles are loaded 16 bytes a lane and
-// read from LDS two K steps at a time.  TFLOP/s with 8-byte loads, [k][x] tiles
-// for both operands and fixed splits -> now: bra 384 x N over K = 18,278:
-// N = 8,192 55 -> 60, 4,096 50 -> 60, 1,000 43 -> 50, 128 27.5 -> 28.6; ket of
-// the same sizes 50 -> 57, 49 -> 56, 47 -> 51, 26.5 -> 29.5; bra / ket 1,296 x 432
-// over 61,446 42.5 -> 46 / 40 -> 48; 8,192^3 60 -> 66.
+// read from LDS two K steps at a time; with few columns, reading the long
+// operand once.  TFLOP/s with 8-byte loads, [k][x] tiles for both operands,
+// fixed splits and partial sums added a load at a time -> now: bra 384 x N over
+// K = 18,278: N = 8,192 55 -> 64, 4,096 50 -> 60, 1,000 43 -> 46, 128 27.5 -> 38;
+// ket of the same sizes 50 -> 56, 49 -> 55, 47 -> 49, 26.5 -> 27.5; bra / ket
+// 1,296 x 432 over 61,446 38 -> 41 / 40 -> 45; 260 x 40 over 18,278 6.2 -> 7.7 /
+// 9.2; 8,192^3 60 -> 66.
 //
 // The projection ("bra") products have a small M (occupied bands +
 // projectors) and a long K (2 npw), so they split K (pick_split); the partial
@@ -279,30 +281,35 @@ __global__ __launch_bounds__(NT, WN == 4 ? 2 : 3) void k_dgemm(int M, int N, int
 #pragma unroll
     for (int j = 0; j < WN; ++j) acc[i][j] = v4d{0.0, 0.0, 0.0, 0.0};
   const int ntile = kend > kbeg ? (kend - kbeg + BK - 1) / BK : 0;
-  d2 ra[tile_loads<BM>()], rb[tile_loads<TN>()];
-  auto load = [&](int k0) {
+  // PF tiles on their way from memory: narrow tiles have the registers for
+  // two, and little else to cover the latency with
+  constexpr int PF = WN == 4 ? 1 : 2;
+  d2 ra[PF][tile_loads<BM>()], rb[PF][tile_loads<TN>()];
+  auto load = [&](int t, d2 (&qa)[tile_loads<BM>()], d2 (&qb)[tile_loads<TN>()]) {
+    if (t >= ntile) return;
+    const int k0 = kbeg + t * BK;
     if (interior && k0 + BK <= kend) {
-      load_tile<TA, false, BM>(ra, A, lda, M, m0, k0, kend);
-      load_tile<true, false, TN>(rb, B, ldb, N, n0, k0, kend);
+      load_tile<TA, false, BM>(qa, A, lda, M, m0, k0, kend);
+      load_tile<true, false, TN>(qb, B, ldb, N, n0, k0, kend);
     } else {
-      load_tile<TA, true, BM>(ra, A, lda, M, m0, k0, kend);
-      load_tile<true, true, TN>(rb, B, ldb, N, n0, k0, kend);
+      load_tile<TA, true, BM>(qa, A, lda, M, m0, k0, kend);
+      load_tile<true, true, TN>(qb, B, ldb, N, n0, k0, kend);
     }
   };
-  auto store = [&](int buf) {
-    store_tile<TA, BM>(As[buf], ra);
-    store_tile<true, TN>(Bs[buf], rb);
+  auto store = [&](int buf, const d2 (&qa)[tile_loads<BM>()], const d2 (&qb)[tile_loads<TN>()]) {
+    store_tile<TA, BM>(As[buf], qa);
+    store_tile<true, TN>(Bs[buf], qb);
   };
-  if (ntile > 0) {
-    load(kbeg);
-    store(0);
-    if (ntile > 1) load(kbeg + BK);
-  }
+  load(0, ra[0], rb[0]);
+  if (PF > 1) load(1, ra[PF - 1], rb[PF - 1]);
+  if (ntile > 0) store(0, ra[0], rb[0]);
+  load(PF, ra[0], rb[0]);
   __syncthreads();
-  // Per tile: half of the K steps, then the next tile goes to the other LDS
-  // buffer (free since the last barrier) and the loads of the one after are
-  // issued, so neither is waited for at the barrier, then the other half.
-  for (int t = 0; t < ntile; ++t) {
+  // Per tile: half of the K steps, then the next tile (in the registers q)
+  // goes to the other LDS buffer (free since the last barrier) and the loads
+  // of the one PF after are issued, so neither is waited for at the barrier,
+  // then the other half.
+  auto step = [&](int t, d2 (&qa)[tile_loads<BM>()], d2 (&qb)[tile_loads<TN>()]) {
     const int cur = t & 1;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -317,11 +324,16 @@ __global__ __launch_bounds__(NT, WN == 4 ? 2 : 3) void k_dgemm(int M, int N, int
           for (int j = 0; j < WN; ++j)
             acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(b[j][st], a[i][st], acc[i][j], 0, 0, 0);
       if (h == 0) {
-        if (t + 1 < ntile) store(cur ^ 1);
-        if (t + 2 < ntile) load(kbeg + (t + 2) * BK);
+        if (t + 1 < ntile) store(cur ^ 1, qa, qb);
+        load(t + 1 + PF, qa, qb);
       }
     }
     __syncthreads();
+  };
+  for (int t = 0; t < ntile; t += PF) {
+    // tile t + 1 is in set (t + 1) % PF
+    step(t, ra[PF - 1], rb[PF - 1]);
+    if (PF > 1 && t + 1 < ntile) step(t + 1, ra[0], rb[0]);
   }
   // block (i, j) holds the transposed product: register r of lane l is
   // C(row i*16 + l%16, column j*16 + l/16 + 4r), so lanes 0..15 (and each
@@ -467,8 +479,18 @@ __global__ void k_reduce_g0(int M, int N, int nsplit, const double* P, long pstr
   const int j = static_cast<int>(idx / M);
   const long o = static_cast<long>(j) * ldc + i;
   if (d_split) nsplit = *d_split;
+  // in order, four loads at a time
   double acc = 0.0;
-  for (int z = 0; z < nsplit; ++z) acc += P[static_cast<long>(z) * pstride + o];
+  const double* p = P + o;
+  int z = 0;
+  for (; z + 4 <= nsplit; z += 4, p += 4 * pstride) {
+    const double a0 = p[0], a1 = p[pstride], a2 = p[2 * pstride], a3 = p[3 * pstride];
+    acc += a0;
+    acc += a1;
+    acc += a2;
+    acc += a3;
+  }
+  for (; z < nsplit; ++z, p += pstride) acc += *p;
   double v = alpha * acc;
   if (g0 != 0.0) v -= g0 * A[static_cast<long>(i) * lda] * B[static_cast<long>(j) * ldb];
   if (s) v *= s[i];
