@@ -62,3 +62,21 @@ def test_linsolve(gpu, cell, nr, nv, nproj, m, kin):
     # each is within sqrt(1e-20 11) / 0.5 = 7e-10 of the solution (two-norm)
     err = np.sqrt(2.0 * np.sum(np.abs(out[0] - out[1]) ** 2, axis=1))
     assert err.max() <= 1.4e-9
+
+
+@pytest.mark.parametrize("cell, nr, nv, m", [(8.0, 24, 1, 256), (14.2, 45, 2, 3), (14.2, 45, 5, 2), (14.2, 45, 7, 1),
+                                             (14.2, 45, 31, 2), (19.5, 54, 6, 1), (19.8, 54, 1, 2), (19.8, 54, 2, 2),
+                                             (19.8, 54, 9, 1), (25.7, 72, 32, 2), (25.7, 72, 4, 1)])
+def test_projector(gpu, cell, nr, nv, m):
+    """The operator's projector part for few columns against NumPy."""
+    gs = _state(cell, nr, nv, 0, 0, 5)
+    gs.vrs = np.zeros_like(gs.vrs)
+    gpu.set_ground_state(gs)
+    rng = np.random.default_rng(m)
+    x = rng.normal(size=(m, gs.npwx)) + 1j * rng.normal(size=(m, gs.npwx))
+    x[:, 0] = x[:, 0].real
+    got = gpu.apply_sternheimerop_to_m_wfcs(nv, x, np.zeros(m), 0.75)
+    ps = 2.0 * (gs.evc.real @ x.real.T + gs.evc.imag @ x.imag.T) - np.outer(gs.evc[:, 0].real, x[:, 0].real)
+    ref = gs.basis.g2kin * x + 0.75 * (ps.T @ gs.evc)
+    # kinetic terms up to 16 and sums of 18,000 terms
+    assert np.abs(got - ref).max() <= 1e-12 * np.abs(ref).max()

@@ -152,14 +152,17 @@ void wait_for_caller(Context& c) {
   WH_HIP(hipStreamWaitEvent(c.stream, c.ev_caller, 0));
 }
 
-// device view of an input array (copied if it is host memory)
+// device view of an input array (copied if it is host memory); one wait orders
+// all of a call's inputs (12 us each: a call's second array took as long as a
+// short kernel)
 template <typename T>
-static const T* dev_in(const T* p, size_t count, DevBuf& tmp) {
+static const T* dev_in(const T* p, size_t count, DevBuf& tmp, bool& waited) {
   if (on_device(p)) {
     // the library's stream does not synchronise with the null stream by
     // itself: order it after the caller's null-stream work (a device array
     // produced on another stream must be complete when the call is made)
-    wait_for_caller(ctx());
+    if (!waited) wait_for_caller(ctx());
+    waited = true;
     return p;
   }
   T* d = tmp.as<T>(count);
@@ -251,10 +254,7 @@ void stern_apply(const z64* x, z64* t, const double* d_e, int m, double alpha, c
     // (with d_nc, cg_select has made the items)
     FftItem* items = ws ? ws->items : c.w_items.as<FftItem>(npair);
     FftItem* ident = ws ? ws->ident : c.w_items_id.as<FftItem>(d_nc ? npair : chunk);
-    if (!d_nc) {
-      fill_pairs(items, m, 0, s);
-      fill_ident(ident, chunk, s);
-    }
+    if (!d_nc) fill_pairs(items, m, 0, s, ident, chunk);
     vloc_pairs(x, t, d_e, items, ident, npair, chunk, d_nc != nullptr, ws);
   }
   // projector part: rows [evc ; vkb] (or evc only for the kinetic-only operator)
@@ -263,13 +263,15 @@ void stern_apply(const z64* x, z64* t, const double* d_e, int m, double alpha, c
     const long k2 = 2L * npw;
     const double* q = reinterpret_cast<const double*>(c.d_q);
     const double* xr = reinterpret_cast<const double*>(x);
-    if (ws) {
+    if (!ws) set_qscale_alpha(alpha);
+    if (!d_nc && cg_project_fits(nq, m, npw)) {
+      WH_TIMED("project", project(m, npw, c.gstart, nq, c.d_q, ws ? ws->qscale : c.d_qscale, x, t, s));
+    } else if (ws) {
       WH_TIMED("gemm_bra", dgemm_bra_into(nq, m, static_cast<int>(k2), 2.0, q, k2, xr, k2, c.gstart == 2 ? 1.0 : 0.0,
                                           ws->qscale, ws->cmat, nq, ws->partials, ws->bra_variant, s));
       WH_TIMED("gemm_ket", dgemm_untimed(false, static_cast<int>(k2), m, nq, 1.0, q, k2, ws->cmat, nq, 1.0,
                                          reinterpret_cast<double*>(t), k2, s));
     } else {
-      set_qscale_alpha(alpha);
       double* cm = c.w_cmat.as<double>(static_cast<size_t>(nq) * m);
       WH_TIMED("gemm_bra", dgemm_bra(nq, m, static_cast<int>(k2), 2.0, q, k2, xr, k2, c.gstart == 2 ? 1.0 : 0.0,
                                      c.d_qscale, cm, nq, s, d_nc));
@@ -468,10 +470,9 @@ void stern_apply32(const z32* x, z32* t, const double* d_e, int m, double alpha)
     const int npair = (m + 1) / 2;
     const int cap = c.items_capacity();
     FftItem* items = c.w_items.as<FftItem>(npair);
-    fill_pairs(items, m, 0, s);
-    FftItem* ident = c.w_items_id.as<FftItem>(std::min(cap, npair));
-    fill_ident(ident, std::min(cap, npair), s);
     const int chunk = std::min(cap, npair);
+    FftItem* ident = c.w_items_id.as<FftItem>(chunk);
+    fill_pairs(items, m, 0, s, ident, chunk);
     z32* sa = c.w_sticks_a.as<z32>(static_cast<size_t>(chunk) * c.plan.sticks_elems());
     z32* sb = c.w_sticks_b.as<z32>(static_cast<size_t>(chunk) * c.plan.sticks_elems());
     const float* v32 = static_cast<const float*>(c.m_vrs32.p);
@@ -1157,8 +1158,9 @@ int wh_apply_sternheimerop_to_m_wfcs(int nbndval, const double* psi, double* hps
   double a[2] = {0.0, 0.0};
   WH_HIP(hipMemcpy(a, alpha, sizeof(double) * 2, hipMemcpyDefault));
   const size_t cin = static_cast<size_t>(m) * c.npwx;
-  const z64* pin = dev_in(reinterpret_cast<const z64*>(psi), cin, c.w_in);
-  const double* pe = dev_in(e, m, c.w_ecol);
+  bool waited = false;
+  const z64* pin = dev_in(reinterpret_cast<const z64*>(psi), cin, c.w_in, waited);
+  const double* pe = dev_in(e, m, c.w_ecol, waited);
   z64* x = c.w_x.as<z64>(static_cast<size_t>(m) * c.npw);
   z64* t = c.w_t.as<z64>(static_cast<size_t>(m) * c.npw);
   gather_sticks(m, c.npw, c.d_perm, pin, c.npwx, x, c.npw, nullptr, s);
@@ -1205,9 +1207,10 @@ int wh_linsolve_sternheimer_m_wfcts(int nbndval, int m, double* b, double* x, co
   WH_HIP(hipMemcpyAsync(dep, ep.data(), sizeof(double) * m, hipMemcpyHostToDevice, s));
   z64* db = c.w_b.as<z64>(static_cast<size_t>(m) * c.npw);
   z64* dx = c.w_x.as<z64>(static_cast<size_t>(m) * c.npw);
-  const z64* bin = dev_in(reinterpret_cast<const z64*>(b), cin, c.w_in);
+  bool waited = false;
+  const z64* bin = dev_in(reinterpret_cast<const z64*>(b), cin, c.w_in, waited);
   gather_sticks(m, c.npw, c.d_perm, bin, c.npwx, db, c.npw, nullptr, s);
-  const z64* xin = dev_in(reinterpret_cast<const z64*>(x), cin, c.w_out);
+  const z64* xin = dev_in(reinterpret_cast<const z64*>(x), cin, c.w_out, waited);
   gather_sticks(m, c.npw, c.d_perm, xin, c.npwx, dx, c.npw, nullptr, s);
   const int nc = c.precision != 0 ? linsolve_mixed(m, db, dx, e_col, de, dep, tr2, nullptr)
                                   : linsolve_dev(m, db, dx, e_col, de, dep, tr2, nullptr);
@@ -1231,7 +1234,8 @@ static int dfpt_entry(int m, const double* dvg, double* dng, double tr2, int iq,
   hipStream_t s = c.stream;
   const size_t cin = static_cast<size_t>(m) * c.npwx;
   if (m == 0) return 0;
-  const z64* din = dev_in(reinterpret_cast<const z64*>(dvg), cin, c.w_in);
+  bool waited = false;
+  const z64* din = dev_in(reinterpret_cast<const z64*>(dvg), cin, c.w_in, waited);
   z64* dvk = c.w_dvin.as<z64>(static_cast<size_t>(m) * c.npw);
   gather_sticks(m, c.npw, c.d_perm, din, c.npwx, dvk, c.npw, coulomb ? c.d_sqvc : nullptr, s);
   z64* dn = c.w_dng.as<z64>(static_cast<size_t>(m) * c.npw);

@@ -55,7 +55,8 @@ void precondition(int m, int npw, const z64* f, z64* pf, long ld, const double* 
 void kinetic_minus_e(int m, int npw, const z64* x, z64* t, long ld, const double* g2kin, const double* e,
                      hipStream_t s);
 void axpby(long n, double a, const z64* x, double b, z64* y, hipStream_t s);
-void fill_pairs(FftItem* items, int m, int row0, hipStream_t s);
+// pairs of m rows, and (ident) the chunk <= their number of stick slots they go through
+void fill_pairs(FftItem* items, int m, int row0, hipStream_t s, FftItem* ident = nullptr, int chunk = 0);
 // device-driven CG (linsolve_sternheimer_m_wfcts.f90:146-222 on the device):
 // one workgroup marks bands whose rho < tr2 as converged, compacts the rest
 // into l2i (ascending band order) with beta = rho / rhoold (0 on the first
@@ -79,11 +80,13 @@ void cg_select(int m, double tr2, int first, int group, const double* rhob, doub
 // and the next direction in h.
 constexpr int kCgProjRows = 32;
 bool cg_project_fits(int nq, int m, int npw);
+// the projector part alone, t += Q s (Q^T x), same range
+void project(int m, int npw, int gstart, int nq, const z64* q, const double* scale, const z64* x, z64* t,
+             hipStream_t s);
 void cg_project(int nc, int npw, int gstart, int nq, const int* l2i, const z64* q, const double* scale, z64* h, z64* g,
                 const z64* t, z64* x, const double* g2kin, const double* eprec, double* rho, const int* d_nc,
                 hipStream_t s);
 void iota(int* v, int n, hipStream_t s);
-void fill_ident(FftItem* items, int n, hipStream_t s);
 void eprec_of(int nb, int npw, const z64* evc, long ld, const double* g2kin, double* eprec, hipStream_t s);
 
 }  // namespace wh
