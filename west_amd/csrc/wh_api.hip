@@ -264,7 +264,7 @@ void stern_apply(const z64* x, z64* t, const double* d_e, int m, double alpha, c
     const double* q = reinterpret_cast<const double*>(c.d_q);
     const double* xr = reinterpret_cast<const double*>(x);
     if (!ws) set_qscale_alpha(alpha);
-    if (!d_nc && cg_project_fits(nq, m, npw)) {
+    if (!d_nc && project_pays(nq, m, npw)) {
       WH_TIMED("project", project(m, npw, c.gstart, nq, c.d_q, ws ? ws->qscale : c.d_qscale, x, t, s));
     } else if (ws) {
       WH_TIMED("gemm_bra", dgemm_bra_into(nq, m, static_cast<int>(k2), 2.0, q, k2, xr, k2, c.gstart == 2 ? 1.0 : 0.0,

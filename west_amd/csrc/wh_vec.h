@@ -80,7 +80,9 @@ void cg_select(int m, double tr2, int first, int group, const double* rhob, doub
 // and the next direction in h.
 constexpr int kCgProjRows = 32;
 bool cg_project_fits(int nq, int m, int npw);
-// the projector part alone, t += Q s (Q^T x), same range
+// the projector part alone, t += Q s (Q^T x), same range; project_pays: and it is
+// the faster way there
+bool project_pays(int nq, int m, int npw);
 void project(int m, int npw, int gstart, int nq, const z64* q, const double* scale, const z64* x, z64* t,
              hipStream_t s);
 void cg_project(int nc, int npw, int gstart, int nq, const int* l2i, const z64* q, const double* scale, z64* h, z64* g,

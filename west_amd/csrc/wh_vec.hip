@@ -363,9 +363,9 @@ __global__ __launch_bounds__(NTU) void k_cg_project(unsigned npw, int gstart, in
 
 // The projector part alone, t += Q s (Q^T x), for the operator on few columns:
 // as in k_cg_project, one workgroup a column with x in registers.  One launch
-// where the products are three (one column, 6 rows, npw = 6,147: 8.2 + 3.5 +
-// 3.4 us and two gaps; a whole call 96 -> 84 us with one item list and one wait
-// for the caller's inputs).
+// where the products are three (one column, 6 rows, npw = 6,147: 17 us against
+// 8.2 + 3.5 + 3.4 and two gaps; a whole call 96 -> 83 us with one item list and
+// one wait for the caller's inputs).  project_pays: where it wins.
 template <int E, int RG>
 __global__ __launch_bounds__(NTU) void k_project(unsigned npw, int gstart, int nq, const z64* q, const double* scale,
                                                 const z64* x, z64* t) {
@@ -744,6 +744,16 @@ void cg_update(int nc, int npw, int gstart, const int* l2i, const z32* h, z32* g
 }
 
 bool cg_project_fits(int nq, int m, int npw) { return nq <= kCgProjRows && m <= 256 && npw <= 9 * NTU; }
+
+// k_project against the three products (a call, us; 1, 16, 256 columns): up to
+// 4 elements a thread it wins throughout (npw = 1,820: 8 rows 69 / 70 / 140 against
+// 92 / 92 / 175, 31 rows 86 / 88 / 161 against 102 / 104 / 213); with 9 the one
+// compute unit of a column takes too long over many rows unless the columns
+// fill the chip (npw = 6,147: 8 rows 86 / 101 / 309 against 84 / 97 / 327, 31 rows
+// 142 / 170 / 402 against 103 / 128 / 475).
+bool project_pays(int nq, int m, int npw) {
+  return cg_project_fits(nq, m, npw) && (npw <= 4 * NTU || nq <= 6 || m > 128);
+}
 
 // run(elements a thread, rows a group): groups of rows that leave none over, as
 // far as the registers go
