@@ -577,6 +577,12 @@ void set_smem(K kernel, size_t bytes) {
   done[key] = bytes;
 }
 
+// WH_FFT_GENERIC=1: the run-time-size kernels on every grid
+bool generic_only() {
+  const char* ev = std::getenv("WH_FFT_GENERIC");
+  return ev && ev[0] == '1';
+}
+
 }  // namespace
 
 void StickPlan::release() {
@@ -672,15 +678,15 @@ void StickPlan::build(int nr1, int nr2, int nr3, int npw, const int* nl, const i
   // the workgroup-level FFTs must fit their register staging
   pick_maxe(static_cast<long>(nrows) * nr2);
   pick_maxe(static_cast<long>(2 * kCPW) * nr3);
-  // kernels specialised on the grid size, unless WH_FFT_GENERIC is set
-  const char* gen = std::getenv("WH_FFT_GENERIC");
-  const bool generic = gen && gen[0] == '1';
+  // kernels specialised on the grid size or with two radices a length, unless
+  // WH_FFT_GENERIC is set
+  const bool generic = generic_only();
   tpl = generic ? nullptr : tpl_kernels_f64(dev);
   tplz = generic ? nullptr : tpl_z_kernels_f64(dev);
   tpl32 = tpl_kernels_f32(dev);
   // (a grid of the FP32 operator keeps the layout that its kernels read)
   rect = RectPlan{};
-  if (!tpl && !tpl32) rect_plan(dev, rect);
+  if (!generic && !tpl && !tpl32) rect_plan(dev, rect);
   // plane-kernel variant: WH_PLANE_OCC (1..9) fixes it, else timed on the first large launch
   const char* occ_env = std::getenv("WH_PLANE_OCC");
   const int occ = (occ_env && occ_env[0] >= '1' && occ_env[0] <= '9') ? occ_env[0] - '0' : 0;
@@ -716,9 +722,10 @@ bool StickPlan::build_columns(int nr1, int nr2, int nr3, const std::vector<int>&
   d.tw1 = upload_twiddles(nr1, allocations);
   d.tw2 = upload_twiddles(nr2, allocations);
   d.tw3 = upload_twiddles(nr3, allocations);
+  vloc_occ = 0;
+  if (generic_only()) return false;
   tpl = tpl_kernels_f64(dev);
   if (!tpl) rect_plan(dev, rect);
-  vloc_occ = 0;
   return tpl || rect.ok;
 }
 
