@@ -69,3 +69,16 @@ def test_runtime_size_kernels_at_q(gpu, kgs_30, monkeypatch):
         out.append(r)
     # solves to tr2 = 1e-18
     assert np.abs(out[0] - out[1]).max() <= 1e-9 * np.abs(out[0]).max()
+
+
+def test_plane_variant_at_q(gpu, monkeypatch):
+    # 30 x 30 x 18: compiled plane kernels
+    at = np.diag((9.0, 9.0, 5.3)) + np.array([[0, 0.1, 0.2], [0, 0, 0.1], [0, 0, 0]])
+    kgs = make_k_ground_state(make_h2_crystal(25.0, cell=at), (1, 1, 2), nbnd=4)
+    out = []
+    for v in ("1", "9"):   # LDS passes, the last of the register-line kernels
+        monkeypatch.setenv("WH_PLANE_OCC", v)
+        gpu.set_k_ground_state(kgs)
+        out.append(_at_q(gpu, kgs)[0])
+    assert np.abs(out[0] - out[1]).max() <= 1e-9 * np.abs(out[0]).max()
+    assert not np.array_equal(out[0], out[1])

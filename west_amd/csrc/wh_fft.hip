@@ -577,6 +577,12 @@ void set_smem(K kernel, size_t bytes) {
   done[key] = bytes;
 }
 
+// WH_PLANE_OCC=1..9: the plane-kernel variant; 0: timed on the first large launch
+int plane_occ_env() {
+  const char* ev = std::getenv("WH_PLANE_OCC");
+  return (ev && ev[0] >= '1' && ev[0] <= '9') ? ev[0] - '0' : 0;
+}
+
 // WH_FFT_GENERIC=1: the run-time-size kernels on every grid
 bool generic_only() {
   const char* ev = std::getenv("WH_FFT_GENERIC");
@@ -687,11 +693,7 @@ void StickPlan::build(int nr1, int nr2, int nr3, int npw, const int* nl, const i
   // (a grid of the FP32 operator keeps the layout that its kernels read)
   rect = RectPlan{};
   if (!generic && !tpl && !tpl32) rect_plan(dev, rect);
-  // plane-kernel variant: WH_PLANE_OCC (1..9) fixes it, else timed on the first large launch
-  const char* occ_env = std::getenv("WH_PLANE_OCC");
-  const int occ = (occ_env && occ_env[0] >= '1' && occ_env[0] <= '9') ? occ_env[0] - '0' : 0;
-  vloc_occ = occ;
-  vloc32_occ = occ;
+  vloc_occ = vloc32_occ = plane_occ_env();
 }
 
 bool StickPlan::build_columns(int nr1, int nr2, int nr3, const std::vector<int>& ci, const std::vector<int>& cj) {
@@ -722,7 +724,7 @@ bool StickPlan::build_columns(int nr1, int nr2, int nr3, const std::vector<int>&
   d.tw1 = upload_twiddles(nr1, allocations);
   d.tw2 = upload_twiddles(nr2, allocations);
   d.tw3 = upload_twiddles(nr3, allocations);
-  vloc_occ = 0;
+  vloc_occ = plane_occ_env();
   if (generic_only()) return false;
   tpl = tpl_kernels_f64(dev);
   if (!tpl) rect_plan(dev, rect);
