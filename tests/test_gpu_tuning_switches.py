@@ -82,3 +82,21 @@ def test_plane_variant_at_q(gpu, monkeypatch):
         out.append(_at_q(gpu, kgs)[0])
     assert np.abs(out[0] - out[1]).max() <= 1e-9 * np.abs(out[0]).max()
     assert not np.array_equal(out[0], out[1])
+
+
+def test_full_grid_switch_leaves_lds_grids(gpu, kgs_30, monkeypatch):
+    """WH_KSTICKS=0 is about grids beyond the LDS: on one that fits, the fused CG
+    iteration and the solve over all k points stay, bit for bit."""
+    at = np.diag((7.2, 5.9, 5.3)) + np.array([[0, 0.1, 0.2], [0, 0, 0.1], [0, 0, 0]])   # 24 x 20 x 18
+    kgs = make_k_ground_state(make_h2_crystal(25.0, cell=at), (2, 1, 1), nbnd=4)
+    out = []
+    for v in ("1", "0"):
+        monkeypatch.setenv("WH_KSTICKS", v)
+        gpu.set_k_ground_state(kgs)
+        r, n = _at_q(gpu, kgs)
+        assert n["cg_iter_lds"] > 0 and n["kgrid_lds"] > 0 and n["kzinv"] == 0
+        out.append(r)
+    assert np.array_equal(out[0], out[1])
+    # beyond the LDS it does keep the full grid
+    gpu.set_k_ground_state(kgs_30)
+    assert _at_q(gpu, kgs_30)[1]["kzinv"] == 0

@@ -11,9 +11,9 @@
 //
 // Layout: rows of npwx or npwqx complex.  Away from Gamma a wave function has
 // no Hermitian partner, so there is no two-band packing and no half sphere.
-// Grids that fit the LDS keep the caller's order and transform each band in
-// one workgroup (wh_kfft_lds.hip).  On larger grids the k-point vectors are in
-// stick order (columns of constant (i, j), k ascending) and the operator runs
+// The k-point vectors are in stick order (columns of constant (i, j), k
+// ascending).  Grids that fit the LDS transform each band in one workgroup
+// (wh_kfft_lds.hip).  On larger grids the operator runs
 // through sticks: z transforms of the columns that hold points
 // (wh_kfft_sticks.hip) around the Gamma path's plane kernels, which take one
 // complex function per item.  One column set holds every k sphere, so a
@@ -55,8 +55,8 @@ struct KPointDev {
   std::vector<double> eprec;  // nbndval: 1.35 sum |evc|^2 |k+G|^2 (Tools/set_eprec.f90:40-56)
   double* d_et = nullptr;     // the same two on the device
   double* d_eprec = nullptr;
-  // stick order (KPath::sticks_want): caller index of each stick position, and
-  // the columns (i, j) with the points' column and k
+  // stick order: caller index of each stick position, and the columns (i, j)
+  // with the points' column and k
   int* perm = nullptr;
   std::vector<int> col_i, col_j, pt_col, pt_k;
   bool set = false;
@@ -97,10 +97,11 @@ struct KPath {
   hipEvent_t cg_ev[4] = {nullptr, nullptr, nullptr, nullptr};   // lagged reads of the CG loop
   KlKpoint* ktab = nullptr;   // device: each k point's sphere and projectors (batched CG)
   double* sck = nullptr;      // device: 2 w_k / (Omega N_r) per k point (densities at q)
-  // stick transforms (grids beyond the LDS): k-point vectors are in stick order
-  bool sticks_want = false;   // stick order in use
+  // the spheres' columns: the operator through sticks (grids beyond the LDS) and
+  // the fused CG iteration
+  bool sticks_want = false;   // the operator may go through sticks
   bool sticks_built = false;  // the plan below holds every registered k sphere
-  bool sticks_ok = false;     // ... and the grid has z and plane kernels for it
+  bool sticks_ok = false;     // ... and the operator does: the grid has z and plane kernels for it
   StickPlan plan;             // union of the k spheres' columns
   KStick* stab = nullptr;     // device, per k point
   const double** qptr = nullptr;   // device, per k point: q2
@@ -571,8 +572,8 @@ static bool klds_enabled() {
   return on;
 }
 
-// WH_KSTICKS=0: the full-grid transforms also where the grid has stick kernels
-// (read when the k grid is registered)
+// WH_KSTICKS=0: on grids beyond the LDS, the full-grid transforms also where
+// there are stick kernels (read when the k grid is registered)
 static bool ksticks_enabled() {
   const char* ev = std::getenv("WH_KSTICKS");
   return !(ev && ev[0] == '0');
@@ -582,7 +583,7 @@ static bool ksticks_enabled() {
 // that one plane launch takes items of any of them.  Built at the first use
 // after a registration.
 static void build_sticks(KPath& K) {
-  if (!K.sticks_want || K.sticks_built) return;
+  if (K.sticks_built) return;
   Context& c = ctx();
   WH_HIP(hipStreamSynchronize(c.stream));
   for (void* p : K.stick_allocs) (void)hipFree(p);
@@ -632,7 +633,7 @@ static void build_sticks(KPath& K) {
   K.stick_allocs.push_back(K.vrs_t);
   rect_transpose_grid(K.fft.n1, K.fft.n2, K.fft.n3, K.vrs, K.vrs_t, c.stream);
   // (a third axis of three or more radices has no z kernel)
-  K.sticks_ok = planes && kz_available(K.fft.n3);
+  K.sticks_ok = K.sticks_want && planes && kz_available(K.fft.n3);
   K.cg_wgs = cg_iter_wgs(K.plan, 2 * (K.nbndval + K.nkb));
 }
 
@@ -644,6 +645,7 @@ static bool sticks_ready(KPath& K) {
 // The fused CG iteration: where the LDS holds a column's rows
 static bool cg_fused(KPath& K) {
   if (!klds_enabled() || ctx().l_kinetic_only) return false;
+  if (!K.sticks_want && !kvloc_lds_available(K.fft.n1, K.fft.n2, K.fft.n3)) return false;
   build_sticks(K);
   return K.cg_wgs >= 1;
 }
@@ -1157,10 +1159,10 @@ int kpath_apply_sternheimerop(int nbndval, const double* psi, double* hpsi, cons
   const double* pe = dev_in(e, m, K.w_ecol);
   z64* t = K.w_t.as<z64>(cin);
   const KPointDev& P = K.k[ik];
-  if (P.perm) pin = to_stick_order(K, P, pin, m, K.w_x.as<z64>(cin));
+  pin = to_stick_order(K, P, pin, m, K.w_x.as<z64>(cin));
   stern_k(K, ik, pin, t, pe, m, a[0]);
   ++c.nstern_calls;
-  if (P.perm) t = to_caller_order(K, P, t, m, K.w_x.as<z64>(cin));
+  t = to_caller_order(K, P, t, m, K.w_x.as<z64>(cin));
   WH_HIP(hipMemcpyAsync(hpsi, t, sizeof(z64) * cin, hipMemcpyDefault, c.stream));
   finish();
   return 0;
@@ -1181,11 +1183,11 @@ int kpath_linsolve(int nbndval, int m, double* b, double* x, const double* e, co
   z64* db = K.w_dv.as<z64>(cin);
   z64* dx = K.w_x.as<z64>(cin);
   const KPointDev& P = K.k[ik];
-  z64* stage = P.perm ? K.w_in.as<z64>(cin) : nullptr;
-  WH_HIP(hipMemcpyAsync(P.perm ? stage : db, b, sizeof(z64) * cin, hipMemcpyDefault, s));
-  if (P.perm) to_stick_order(K, P, stage, m, db);
-  WH_HIP(hipMemcpyAsync(P.perm ? stage : dx, x, sizeof(z64) * cin, hipMemcpyDefault, s));
-  if (P.perm) to_stick_order(K, P, stage, m, dx);
+  z64* stage = K.w_in.as<z64>(cin);
+  WH_HIP(hipMemcpyAsync(stage, b, sizeof(z64) * cin, hipMemcpyDefault, s));
+  to_stick_order(K, P, stage, m, db);
+  WH_HIP(hipMemcpyAsync(stage, x, sizeof(z64) * cin, hipMemcpyDefault, s));
+  to_stick_order(K, P, stage, m, dx);
   double* de = K.w_ecol.as<double>(m);
   double* dep = K.w_epcol.as<double>(m);
   WH_HIP(hipMemcpyAsync(de, e, sizeof(double) * m, hipMemcpyDefault, s));
@@ -1198,7 +1200,7 @@ int kpath_linsolve(int nbndval, int m, double* b, double* x, const double* e, co
   WH_HIP(hipMemcpyAsync(&nc, d_nonconv, sizeof(int), hipMemcpyDeviceToHost, s));
   WH_HIP(hipStreamSynchronize(s));
   cg_k_count(rec, last);
-  if (P.perm) dx = to_caller_order(K, P, dx, m, stage);
+  dx = to_caller_order(K, P, dx, m, stage);
   WH_HIP(hipMemcpyAsync(x, dx, sizeof(z64) * cin, hipMemcpyDefault, s));
   finish();
   if (ierr) *ierr = nc;
@@ -1390,41 +1392,39 @@ int wh_set_kpoint(int ik, int npw, const int* nl, const double* g2kin, const dou
   for (int ig = 0; ig < npw; ++ig) perm[ig] = ig;
   P.col_i.clear();
   P.col_j.clear();
-  if (K.sticks_want) {
-    const int n1 = K.fft.n1, n2 = K.fft.n2, n3 = K.fft.n3;
-    auto center = [](int v, int n) { return v > n / 2 ? v - n : v; };
-    std::vector<int> mi(npw), mj(npw), mk3(npw);
-    for (int ig = 0; ig < npw; ++ig) {
-      mi[ig] = center(hnl[ig] % n1, n1);
-      mj[ig] = center((hnl[ig] / n1) % n2, n2);
-      mk3[ig] = center(hnl[ig] / (n1 * n2), n3);
-    }
-    std::sort(perm.begin(), perm.end(), [&](int a, int b) {
-      if (mi[a] != mi[b]) return mi[a] < mi[b];
-      if (mj[a] != mj[b]) return mj[a] < mj[b];
-      return mk3[a] < mk3[b];
-    });
-    P.pt_col.assign(npw, 0);
-    P.pt_k.assign(npw, 0);
-    for (int q = 0; q < npw; ++q) {
-      const int g = perm[q];
-      if (q == 0 || mi[g] != P.col_i.back() || mj[g] != P.col_j.back()) {
-        P.col_i.push_back(mi[g]);
-        P.col_j.push_back(mj[g]);
-      }
-      P.pt_col[q] = static_cast<int>(P.col_i.size()) - 1;
-      P.pt_k[q] = mk3[g];
-    }
-    std::vector<int> nl2(npw);
-    std::vector<double> g22(npw);
-    for (int q = 0; q < npw; ++q) {
-      nl2[q] = hnl[perm[q]];
-      g22[q] = hg2[perm[q]];
-    }
-    hnl.swap(nl2);
-    hg2.swap(g22);
-    P.perm = upload(K, perm.data(), perm.size());
+  const int n1 = K.fft.n1, n2 = K.fft.n2, n3 = K.fft.n3;
+  auto center = [](int v, int n) { return v > n / 2 ? v - n : v; };
+  std::vector<int> mi(npw), mj(npw), mk3(npw);
+  for (int ig = 0; ig < npw; ++ig) {
+    mi[ig] = center(hnl[ig] % n1, n1);
+    mj[ig] = center((hnl[ig] / n1) % n2, n2);
+    mk3[ig] = center(hnl[ig] / (n1 * n2), n3);
   }
+  std::sort(perm.begin(), perm.end(), [&](int a, int b) {
+    if (mi[a] != mi[b]) return mi[a] < mi[b];
+    if (mj[a] != mj[b]) return mj[a] < mj[b];
+    return mk3[a] < mk3[b];
+  });
+  P.pt_col.assign(npw, 0);
+  P.pt_k.assign(npw, 0);
+  for (int q = 0; q < npw; ++q) {
+    const int g = perm[q];
+    if (q == 0 || mi[g] != P.col_i.back() || mj[g] != P.col_j.back()) {
+      P.col_i.push_back(mi[g]);
+      P.col_j.push_back(mj[g]);
+    }
+    P.pt_col[q] = static_cast<int>(P.col_i.size()) - 1;
+    P.pt_k[q] = mk3[g];
+  }
+  std::vector<int> nl2(npw);
+  std::vector<double> g22(npw);
+  for (int q = 0; q < npw; ++q) {
+    nl2[q] = hnl[perm[q]];
+    g22[q] = hg2[perm[q]];
+  }
+  hnl.swap(nl2);
+  hg2.swap(g22);
+  P.perm = upload(K, perm.data(), perm.size());
   std::vector<z64> q2(ld * 2 * std::max(nq, 1), mk(0.0, 0.0));
   P.et.assign(nb, 0.0);
   P.eprec.assign(nb, 0.0);
