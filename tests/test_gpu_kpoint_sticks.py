@@ -98,3 +98,44 @@ def test_iteration_limit_counts_unconverged(gpu, ksys):
         assert list(ierr) == [ksys.nks * ksys.nbndval] * 2
     finally:
         gpu.set_k_ground_state(ksys)
+
+
+# the last: |i| = n1 / 2, a point whose row has no mirror row
+@pytest.mark.parametrize("nr, a1, imax", [((12, 10, 9), 6.4, 5), ((20, 16, 15), 11.5, 9), ((15, 12, 16), 8.9, 7),
+                                          ((12, 10, 9), 7.2, 6)])
+def test_wide_sphere_on_lds_grid(gpu, nr, a1, imax, monkeypatch):
+    """Spheres wider than a quarter of the grid (a density cutoff below four times
+    the wave functions') keep the fused iteration."""
+    import dataclasses
+    from oracle import kpoint as K
+    from west_amd import kpoint
+    from west_amd.gsphere import grid_index, make_gamma_basis
+    at = np.diag((a1, 5.9, 5.3))
+    s = make_h2_crystal(25.0, cell=at)
+    wide, plain = s.basis, kpoint.make_k_basis
+
+    def on_small_grid(_, xk):   # spheres from the full grid, indexed on this one
+        b = plain(wide, xk)
+        return dataclasses.replace(b, nr=nr, nl=(grid_index(b.mill, nr) + 1).astype(np.int32))
+
+    monkeypatch.setattr(kpoint, "make_k_basis", on_small_grid)
+    s = dataclasses.replace(s, basis=make_gamma_basis(at, 25.0, nr=nr))
+    kgs = make_k_ground_state(s, (2, 1, 1), nbnd=4, vrs=-np.random.default_rng(6).random(nr[0] * nr[1] * nr[2]))
+    assert max(int(np.abs(k.basis.mill[:, 0]).max()) for k in kgs.kpts) == imax > nr[0] // 4
+    assert all(len(np.unique(k.basis.nl)) == k.basis.npw for k in kgs.kpts)
+    qb = kgs.qpts[1].basis
+    dv = _smooth(qb.npw, kgs.npwqx, 3, qb.g2kin, 8)
+    h = gpu.system_create()
+    gpu.system_select(h)
+    try:
+        gpu.set_k_ground_state(kgs)
+        gpu.profile(True)
+        out, ierr = gpu.dfpt(3, dv, 1e-22, iq=2, return_ierr=True)
+        assert gpu.profile_query("cg_iter_lds")[1] > 0
+        gpu.profile(False)
+    finally:
+        gpu.system_select(0)
+        gpu.system_destroy(h)
+    assert not ierr.any()
+    # converged solves, as above
+    assert _rel(out, K.dfpt_q(kgs, 1, dv, 1e-22)) < 1e-9

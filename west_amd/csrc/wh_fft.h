@@ -90,8 +90,8 @@ struct StickPlan {
   void build(int nr1, int nr2, int nr3, int npw, const int* nl_1based, const int* nlm_1based);
   // Plane part only, for complex functions with the given columns (i, j): no
   // mirror columns and no points (k points: wh_kfft_sticks.hip's z kernels
-  // bring their own).  False where the grid has neither tpl nor rect kernels;
-  // dev.nct is 0 where the columns do not fit the grid.
+  // bring their own).  False where the grid has neither tpl nor rect kernels or
+  // its columns are too wide for them; the tables are made all the same.
   bool build_columns(int nr1, int nr2, int nr3, const std::vector<int>& ci, const std::vector<int>& cj);
   void release();
   long sticks_elems() const { return static_cast<long>(dev.n3) * dev.nct; }

@@ -710,7 +710,6 @@ bool StickPlan::build_columns(int nr1, int nr2, int nr3, const std::vector<int>&
   tpl = tplz = nullptr;
   tpl32 = nullptr;
   rect = RectPlan{};
-  if (d.nrows > nr1 || 2 * d.jext + 1 > nr2) return false;
   d.n1 = nr1; d.n2 = nr2; d.n3 = nr3;
   d.ncs = d.nct = n;
   col_i = ci;
@@ -725,7 +724,8 @@ bool StickPlan::build_columns(int nr1, int nr2, int nr3, const std::vector<int>&
   d.tw2 = upload_twiddles(nr2, allocations);
   d.tw3 = upload_twiddles(nr3, allocations);
   vloc_occ = plane_occ_env();
-  if (generic_only()) return false;
+  // (the plane kernels give each of -imax .. imax and -jext .. jext a place of its own)
+  if (generic_only() || d.nrows > nr1 || 2 * d.jext + 1 > nr2) return false;
   tpl = tpl_kernels_f64(dev);
   if (!tpl) rect_plan(dev, rect);
   return tpl || rect.ok;

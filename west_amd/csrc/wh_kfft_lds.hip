@@ -235,19 +235,21 @@ __device__ __forceinline__ void kl_block_sums(double* v, int nv, double (*red)[K
 // order (col = lb, eu = e by column): the operator acts on x, then
 // g = A x - b, h = g / max(1, g2kin/eprec), rho[col] = Re <h|g>.
 struct KlRows {
-  int n1, n2, n3, imax, nct, p2;   // p2: odd pitch along a2
+  int n1, n2, n3, imax, nct, p2;   // p2: pitch along a2
   const int* col_pos;              // (i + imax) n2 + (j mod n2) of each column
 };
 
-// widest |i| the a1 lines take: the sphere spans at most (n + 1) / 4 either
-// way, and the k point less than one more
-constexpr int kl_row_bound(int n) { return n / 4 + 1; }
+// widest |i| the a1 lines take: where the grid holds the products of two
+// functions the sphere spans at most (n + 1) / 4 either way, and the k point
+// less than one more.  WIDE: any sphere of the grid, every element may come
+// from a row.
+constexpr int kl_row_bound(int n, bool wide) { return wide ? n / 2 : n / 4 + 1; }
 
 // a1 line from and to the rows: v(x) at p[(x or x - n1) rs], |x| <= imax
 // (elements beyond kl_row_bound are known zeros)
-template <int N>
+template <int N, bool WIDE>
 __device__ __forceinline__ void kl_line_rows(z64* p, int rs, int imax, const double* vr, int vs, double sc) {
-  constexpr int BX = kl_row_bound(N);
+  constexpr int BX = kl_row_bound(N, WIDE);
   rs = kl_opaque(rs);
   imax = kl_opaque(imax);
   vs = kl_opaque(vs);
@@ -277,11 +279,12 @@ __device__ __forceinline__ void kl_line_rows(z64* p, int rs, int imax, const dou
     }
 }
 
+template <bool WIDE>
 __device__ __forceinline__ void kl_pass_rows(int n, z64* p, int rs, int imax, const double* vr, int vs, double sc) {
   switch (n) {
 #define WH_KL_CASE(NN)                                 \
   case NN:                                             \
-    kl_line_rows<NN>(p, rs, imax, vr, vs, sc);         \
+    kl_line_rows<NN, WIDE>(p, rs, imax, vr, vs, sc);   \
     break;
     WH_KL_SIZES(WH_KL_CASE)
 #undef WH_KL_CASE
@@ -313,7 +316,7 @@ __device__ __forceinline__ void kl_sums(const double* v, int nv, double (*red)[N
 
 constexpr int KR_NT = 256;
 
-template <bool FIRST>
+template <bool FIRST, bool WIDE>
 __global__ __launch_bounds__(KR_NT) __attribute__((amdgpu_waves_per_eu(2))) void k_cg_iter_rows(KlRows R,
                                                                                              const KStick* stab,
                                                                                              KlCgArgs a) {
@@ -405,7 +408,7 @@ __global__ __launch_bounds__(KR_NT) __attribute__((amdgpu_waves_per_eu(2))) void
   const double sc = 1.0 / (static_cast<double>(n1) * n2 * n3);
   for (int l = tid; l < n2 * n3; l += NT) {
     const int z = l / n2, y = l - z * n2;
-    kl_pass_rows(n1, grid + imax * rs + z * p2 + y, rs, imax, a.vrs + z * n1 * n2 + y, n2, sc);
+    kl_pass_rows<WIDE>(n1, grid + imax * rs + z * p2 + y, rs, imax, a.vrs + z * n1 * n2 + y, n2, sc);
   }
   __syncthreads();
   for (int l = tid; l < nrows * n3; l += NT) kl_pass<-1>(n2, grid + l * p2, 1);
@@ -713,16 +716,21 @@ void density_lds(int n1, int n2, int n3, int nks, int nb, int m, long ld, const 
 }
 
 namespace {
-size_t kl_rows_smem(const StickPlanDev& P) {
-  return sizeof(z64) * static_cast<size_t>(P.nrows) * P.n3 * (P.n2 | 1);
+size_t kl_rows_smem(const StickPlanDev& P, int p2) {
+  return sizeof(z64) * static_cast<size_t>(P.nrows) * P.n3 * p2;
+}
+// pitch along a2: odd, so that neighbouring rows start on other banks; n2 itself
+// where only that fits
+int kl_rows_pitch(const StickPlanDev& P) {
+  const int p2 = P.n2 | 1;
+  return kl_rows_smem(P, p2) + kKlCgStatic <= kKlMaxSmem ? p2 : P.n2;
 }
 }  // namespace
 
 int cg_iter_wgs(const StickPlan& p, int nq2) {
   const StickPlanDev& P = p.dev;
   if (P.nct <= 0 || nq2 < 0 || nq2 > KL_NQ2 || !kl_size(P.n1) || !kl_size(P.n2) || !kl_size(P.n3)) return 0;
-  if (P.imax > kl_row_bound(P.n1)) return 0;
-  return static_cast<int>(kKlMaxSmem / (kl_rows_smem(P) + kKlCgStatic));
+  return static_cast<int>(kKlMaxSmem / (kl_rows_smem(P, kl_rows_pitch(P)) + kKlCgStatic));
 }
 
 void cg_iter_rows(const StickPlan& p, const KStick* stab, bool first, int m, const KlCgArgs& a, hipStream_t s) {
@@ -730,17 +738,24 @@ void cg_iter_rows(const StickPlan& p, const KStick* stab, bool first, int m, con
   WH_REQUIRE(!a.ktab || a.cols_per_k > 0, "cg_iter_rows: cols_per_k must be > 0");
   if (m <= 0) return;
   static const bool attr_set = [] {   // once per process (thread-safe static initialisation)
-    for (const void* k : {reinterpret_cast<const void*>(k_cg_iter_rows<false>),
-                          reinterpret_cast<const void*>(k_cg_iter_rows<true>)})
+    for (const void* k : {reinterpret_cast<const void*>(k_cg_iter_rows<false, false>),
+                          reinterpret_cast<const void*>(k_cg_iter_rows<true, false>),
+                          reinterpret_cast<const void*>(k_cg_iter_rows<false, true>),
+                          reinterpret_cast<const void*>(k_cg_iter_rows<true, true>)})
       WH_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize,
                                  static_cast<int>(kKlMaxSmem - kKlCgStatic)));
     return true;
   }();
   (void)attr_set;
   const StickPlanDev& P = p.dev;
-  const KlRows r{P.n1, P.n2, P.n3, P.imax, P.nct, P.n2 | 1, P.col_pos};
-  if (first) k_cg_iter_rows<true><<<m, KR_NT, kl_rows_smem(P), s>>>(r, stab, a);
-  else k_cg_iter_rows<false><<<m, KR_NT, kl_rows_smem(P), s>>>(r, stab, a);
+  const int p2 = kl_rows_pitch(P);
+  const size_t sm = kl_rows_smem(P, p2);
+  const KlRows r{P.n1, P.n2, P.n3, P.imax, P.nct, p2, P.col_pos};
+  const bool wide = P.imax > kl_row_bound(P.n1, false);
+  if (first && wide) k_cg_iter_rows<true, true><<<m, KR_NT, sm, s>>>(r, stab, a);
+  else if (first) k_cg_iter_rows<true, false><<<m, KR_NT, sm, s>>>(r, stab, a);
+  else if (wide) k_cg_iter_rows<false, true><<<m, KR_NT, sm, s>>>(r, stab, a);
+  else k_cg_iter_rows<false, false><<<m, KR_NT, sm, s>>>(r, stab, a);
   WH_HIP(hipGetLastError());
 }
 

@@ -604,7 +604,6 @@ static void build_sticks(KPath& K) {
   K.sticks_built = true;
   if (ci.empty()) return;
   const bool planes = K.plan.build_columns(K.fft.n1, K.fft.n2, K.fft.n3, ci, cj);
-  if (K.plan.dev.nct == 0) return;
   auto up = [&](const auto& h) {
     using V = typename std::decay_t<decltype(h)>::value_type;
     V* d = nullptr;
