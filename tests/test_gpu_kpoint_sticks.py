@@ -139,3 +139,42 @@ def test_wide_sphere_on_lds_grid(gpu, nr, a1, imax, monkeypatch):
     assert not ierr.any()
     # converged solves, as above
     assert _rel(out, K.dfpt_q(kgs, 1, dv, 1e-22)) < 1e-9
+
+
+def test_workspace_stays_within_the_grid_budget(gpu):
+    """The solve over every k point and its sticks share one budget of 2 GiB: 8 k
+    points of 16 states on 36^3 points, 40 perturbations (1.8 GiB of vectors and
+    grids; the sticks of their 5,120 columns would be 1.25 GiB more)."""
+    import torch
+    from west_amd.gsphere import make_gamma_basis
+    from west_amd.kpoint import KGroundState, KPoint, make_k_basis, make_qpoint, mp_grid
+    nb, m = 16, 40
+    gb = make_gamma_basis(np.eye(3) * 10.26, 25.0, nr=(36, 36, 36))
+    kc, kx = mp_grid(gb, (2, 2, 2))
+    bases = [make_k_basis(gb, k) for k in kx]
+    npwx = max(b.npw for b in bases)
+    rng = np.random.default_rng(2)
+    kpts = []
+    for b in bases:
+        evc = np.zeros((nb, npwx), complex)
+        evc[:, :b.npw] = np.linalg.qr(rng.normal(size=(b.npw, nb)) + 1j * rng.normal(size=(b.npw, nb)))[0].T
+        kpts.append(KPoint(basis=b, npwx=npwx, evc=evc, et=np.zeros(nb), vkb=np.zeros((0, npwx), complex), weight=0.25))
+    kgs = KGroundState(gbasis=gb, nk=(2, 2, 2), kcryst=kc, kpts=kpts, vrs=rng.random(36 ** 3), dvan=np.zeros(0),
+                       nbndval=nb, alpha_pv=1.0, qpts=[make_qpoint(gb, kc, kc[1])])
+    dv = _smooth(kgs.qpts[0].basis.npw, kgs.npwqx, m, kgs.qpts[0].basis.g2kin, 1)
+    h = gpu.system_create()
+    gpu.system_select(h)
+    try:
+        gpu.set_k_ground_state(kgs, n_dfpt_maxiter=2)
+        free = torch.cuda.mem_get_info()[0]
+        gpu.profile(True)
+        with pytest.warns(UserWarning):   # (two iterations)
+            gpu.dfpt(m, dv, 1e-22, iq=1)
+        assert gpu.profile_query("kzinv")[1] > 0
+        gpu.profile(False)
+        used = free - torch.cuda.mem_get_info()[0]
+    finally:
+        gpu.system_select(0)
+        gpu.system_destroy(h)
+    # and the products' partial sums, the in- and outputs, the sphere's tables
+    assert used <= (2 << 30) + (256 << 20)

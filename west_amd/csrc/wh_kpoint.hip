@@ -108,7 +108,7 @@ struct KPath {
   double* vrs_t = nullptr;         // vrs as the two-radix plane kernels read it, [a3][a1][a2]
   int cg_wgs = 0;                  // workgroups per CU of the fused CG iteration (0: none)
   std::vector<void*> stick_allocs;
-  DevBuf w_sa, w_sb, w_ident, w_grp;
+  DevBuf w_ident, w_grp;
   DevBuf w_dk;                // densities per (k point, perturbation) before the sum over k
 };
 
@@ -124,7 +124,7 @@ void free_kpath(KPath* k) {
   k->fft.release();
   k->plan.release();
   for (void* p : k->stick_allocs) (void)hipFree(p);
-  for (DevBuf* b : {&k->w_sa, &k->w_sb, &k->w_ident, &k->w_grp}) b->release();
+  for (DevBuf* b : {&k->w_ident, &k->w_grp}) b->release();
   for (DevBuf* b : {&k->g_a, &k->g_b, &k->g_c, &k->g_aux, &k->w_x, &k->w_t, &k->w_g, &k->w_h, &k->w_hold, &k->w_bc,
                     &k->w_tc, &k->w_c2, &k->w_l2i, &k->w_rho, &k->w_rhoold, &k->w_conv, &k->w_nonconv, &k->w_beta,
                     &k->w_eu, &k->w_ecol, &k->w_epcol, &k->w_dv, &k->w_dn, &k->w_in, &k->w_out, &k->w_in2})
@@ -650,20 +650,22 @@ static bool cg_fused(KPath& K) {
 }
 
 // t = F^-1 V F x + (|k+G|^2 - e) x through sticks for m columns (cols_per_k,
-// l2i: as in KStick; 0: all of k point ik)
+// l2i: as in KStick; 0: all of k point ik).  The sticks, at most `bytes` of
+// them, lie in the buffer of the grids that a full-grid operator would need:
+// dfpt's own are dead while it is applied.
 static void vloc_sticks(KPath& K, int ik, int cols_per_k, const int* l2i, const z64* x, z64* t, const double* d_e,
-                        int m, const int* d_nc) {
+                        int m, const int* d_nc, long bytes) {
   Context& c = ctx();
   hipStream_t s = c.stream;
   const long ld = K.npwx;
   const long sl = K.plan.sticks_elems();
-  const long fit = static_cast<long>(K.grid_budget) / (2 * sl * static_cast<long>(sizeof(z64)));
+  const long fit = bytes / (2 * sl * static_cast<long>(sizeof(z64)));
   const int chunk = static_cast<int>(std::max<long>(1, std::min<long>({fit, 65535L, m})));
   FftItem* items = K.w_ident.as<FftItem>(m);
   k_ident_cols<<<ceil_div(m, NT), NT, 0, s>>>(items, m, chunk, d_nc);
   WH_HIP(hipGetLastError());
-  z64* sa = K.w_sa.as<z64>(static_cast<size_t>(chunk) * sl);
-  z64* sb = K.w_sb.as<z64>(static_cast<size_t>(chunk) * sl);
+  z64* sa = K.g_a.as<z64>(2 * static_cast<size_t>(chunk) * sl);
+  z64* sb = sa + static_cast<size_t>(chunk) * sl;
   const KStick* tab = cols_per_k > 0 ? K.stab : K.stab + ik;
   const double scale = 1.0 / static_cast<double>(K.fft.nnr());
   for (int c0 = 0; c0 < m; c0 += chunk) {
@@ -687,11 +689,11 @@ static DgemmGroups k_groups(KPath& K, int cols, int m, const int* l2i, const int
 }
 
 static void stern_all(KPath& K, int cols, const z64* x, z64* t, const double* d_e, int m, const int* l2i,
-                      const int* d_nc) {
+                      const int* d_nc, long stick_bytes) {
   Context& c = ctx();
   hipStream_t s = c.stream;
   const long ld = K.npwx;
-  vloc_sticks(K, 0, cols, l2i, x, t, d_e, m, d_nc);
+  vloc_sticks(K, 0, cols, l2i, x, t, d_e, m, d_nc, stick_bytes);
   const int nq = K.nbndval + K.nkb;
   if (nq > 0) {
     set_qscale2(K, K.alpha_pv);
@@ -721,7 +723,7 @@ static void stern_k(KPath& K, int ik, const z64* x, z64* t, const double* d_e, i
     WH_TIMED("kvloc_lds", kvloc_lds(K.fft.n1, K.fft.n2, K.fft.n3, m, P.npw, ld, P.nl, x, K.vrs, P.g2kin, d_e, t, s,
                                     d_nc));
   const bool sticks = !lds && !c.l_kinetic_only && m > 0 && sticks_ready(K);
-  if (sticks) vloc_sticks(K, ik, 0, nullptr, x, t, d_e, m, d_nc);
+  if (sticks) vloc_sticks(K, ik, 0, nullptr, x, t, d_e, m, d_nc, static_cast<long>(K.grid_budget));
   for (int c0 = 0; c0 < (lds || sticks ? 0 : m); c0 += gc) {
     const int mc = std::min(gc, m - c0);
     const z64* xc = x + c0 * ld;
@@ -799,9 +801,10 @@ static void minus_pc_all(KPath& K, int cols, z64* f, int m) {
 // launched to cg_k_count.
 // nkb = 1: the cols columns belong to k point ik.  nkb = nks: columns
 // [k cols, (k + 1) cols) belong to k point k, all in one solve (the fused
-// iteration, kbatch_ok, or the stick operator, kbatch_cols).
+// iteration, kbatch_ok, or the stick operator, kbatch_cols, with sticks of
+// stick_bytes).
 static int linsolve_k(KPath& K, int ik, int nkb, int cols, z64* b, z64* x, const double* d_e, const double* d_ep,
-                      double tr2, int group, int nper, int* rec, int* nonconv) {
+                      double tr2, int group, int nper, int* rec, int* nonconv, long stick_bytes = 0) {
   Context& c = ctx();
   hipStream_t s = c.stream;
   const int m = nkb * cols;
@@ -845,7 +848,7 @@ static int linsolve_k(KPath& K, int ik, int nkb, int cols, z64* b, z64* x, const
     c.nstern += m;
   } else {
     iota(d_l2i, m, s);
-    if (nkb > 1) stern_all(K, cols, x, g, d_e, m, nullptr, nullptr);
+    if (nkb > 1) stern_all(K, cols, x, g, d_e, m, nullptr, nullptr, stick_bytes);
     else stern_k(K, ik, x, g, d_e, m, K.alpha_pv);
     k_sub<<<blocks(static_cast<long>(vec)), NT, 0, s>>>(static_cast<long>(vec), b, g);
     k_cg_prec_rho<<<m, NT, 0, s>>>(d_l2i, nullptr, P.npw, ld, P.g2kin, d_ep, g, h, d_rhob, tab, cols);
@@ -870,7 +873,7 @@ static int linsolve_k(KPath& K, int ik, int nkb, int cols, z64* b, z64* x, const
     } else {
       k_cg_dir<<<blocks(static_cast<long>(cap) * ld), NT, 0, s>>>(cap, d_nc, d_l2i, ld, d_beta, d_e, h, hold, bc,
                                                                   d_eu);
-      if (nkb > 1) stern_all(K, cols, bc, tc, d_eu, cap, d_l2i, d_nc);
+      if (nkb > 1) stern_all(K, cols, bc, tc, d_eu, cap, d_l2i, d_nc, stick_bytes);
       else stern_k(K, ik, bc, tc, d_eu, cap, K.alpha_pv, d_nc);
       k_cg_step<<<cap, NT, 0, s>>>(d_l2i, d_nc, P.npw, ld, P.g2kin, d_ep, x, g, h, tc, hold, d_rhob, tab, cols);
       WH_HIP(hipGetLastError());
@@ -917,8 +920,10 @@ static bool kbatch_ok(KPath& K, int m) {
 
 // On grids beyond the LDS: perturbations per solve over every k point through
 // the stick operator, 0 for the k points one after another.  Counted against
-// the grid budget as above.
-static int kbatch_cols(KPath& K, int m) {
+// the grid budget: the solve's vectors, the states at k - q, the perturbations,
+// the grids of one k point's right-hand sides and its densities.  The sticks
+// take the place of those right-hand sides and what is left, stick_bytes.
+static int kbatch_cols(KPath& K, int m, long& stick_bytes) {
   const char* ev = std::getenv("WH_KBATCH");
   if (ev && ev[0] == '0') return 0;
   const Context& c = ctx();
@@ -929,8 +934,10 @@ static int kbatch_cols(KPath& K, int m) {
   const long room = static_cast<long>(K.grid_budget) - fixed;
   if (room < per) return 0;
   const long fit = std::min<long>({room / per, m, (1L << 24) / (static_cast<long>(K.nks) * K.nbndval)});
-  // equal chunks
-  return fit < 1 ? 0 : ceil_div(m, ceil_div(m, fit));
+  if (fit < 1) return 0;
+  const int mp = ceil_div(m, ceil_div(m, fit));   // equal chunks
+  stick_bytes = room - mp * per + z * mp * K.nbndval * nnr;
+  return mp;
 }
 
 // dng (npwqx, m) = chi0(q) dvg for q point iq (0-based)  (dfpt_module.f90:163-505)
@@ -949,7 +956,8 @@ static int dfpt_q(KPath& K, int iq, int m, const z64* dvg, z64* dng, double tr2,
   if (m == 0 || nb == 0) return 0;
   // perturbations per chunk: their band columns' grids within the budget
   const bool lds_all = tr2 >= 0.0 && kbatch_ok(K, m);
-  const int mall = tr2 >= 0.0 && !lds_all ? kbatch_cols(K, m) : 0;
+  long stick_bytes = 0;
+  const int mall = tr2 >= 0.0 && !lds_all ? kbatch_cols(K, m, stick_bytes) : 0;
   const int mp = mall > 0 ? mall : std::max(1, std::min(m, grid_cols(K) / std::max(nb, 1)));
   // per solve: its CG records (pinned) and iterations launched, read at the end
   const int nsolve = K.nks * ((m + mp - 1) / mp);
@@ -1038,7 +1046,8 @@ static int dfpt_q(KPath& K, int iq, int m, const z64* dvg, z64* dng, double tr2,
                                                                    cols);
       WH_HIP(hipGetLastError());
       int* rec = recs + rec_len * launched.size();
-      launched.push_back(linsolve_k(K, 0, K.nks, cols, dvpsi, dpsi, d_e, d_ep, tr2, nb, mc, rec, d_nonconv + p0));
+      launched.push_back(linsolve_k(K, 0, K.nks, cols, dvpsi, dpsi, d_e, d_ep, tr2, nb, mc, rec, d_nonconv + p0,
+                                    stick_bytes));
       for (int ik = 0; ik < K.nks; ++ik)
         density(ik, p0, mc, psik + static_cast<size_t>(ik) * nb * nnr, dpsi + static_cast<size_t>(ik) * cols * ld);
     }
