@@ -178,3 +178,27 @@ def test_workspace_stays_within_the_grid_budget(gpu):
         gpu.system_destroy(h)
     # and the products' partial sums, the in- and outputs, the sphere's tables
     assert used <= (2 << 30) + (256 << 20)
+
+
+def test_linsolve_waits_for_device_inputs(gpu, ksys):
+    """Device arrays that null-stream work queued before the call still writes."""
+    import torch
+    v = ksys.kpts[0].basis
+    m, nb = 3, ksys.nbndval
+    b = torch.from_numpy(_smooth(v.npw, ksys.npwx, m, v.g2kin, 3)).cuda()
+    e, ep = np.full(m, -1.5), np.full(m, 1.5)
+    big = torch.ones(1 << 28, device="cuda")
+    gpu.set_current_k(1)
+    out = []
+    for late in (False, False, True):   # (the first call sizes the workspaces)
+        x, bb = torch.zeros_like(b), torch.zeros_like(b)
+        torch.cuda.synchronize()
+        if late:
+            for _ in range(20):   # some 10 ms
+                big.mul_(1.0)
+        bb.copy_(b)
+        if not late:
+            torch.cuda.synchronize()
+        assert gpu.linsolve_sternheimer_m_wfcts(nb, m, bb, x, e, ep, 1e-20) == 0
+        out.append(x)
+    assert torch.equal(out[1], out[2])

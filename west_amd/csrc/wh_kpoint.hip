@@ -1192,6 +1192,8 @@ int kpath_linsolve(int nbndval, int m, double* b, double* x, const double* e, co
   z64* dx = K.w_x.as<z64>(cin);
   const KPointDev& P = K.k[ik];
   z64* stage = K.w_in.as<z64>(cin);
+  // the copies below are ordered after the caller's null-stream work
+  if (on_device_mem(b) || on_device_mem(x) || on_device_mem(e) || on_device_mem(eprec)) wait_for_caller(c);
   WH_HIP(hipMemcpyAsync(stage, b, sizeof(z64) * cin, hipMemcpyDefault, s));
   to_stick_order(K, P, stage, m, db);
   WH_HIP(hipMemcpyAsync(stage, x, sizeof(z64) * cin, hipMemcpyDefault, s));
