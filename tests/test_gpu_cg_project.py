@@ -80,3 +80,18 @@ def test_projector(gpu, cell, nr, nv, m):
     ref = gs.basis.g2kin * x + 0.75 * (ps.T @ gs.evc)
     # kinetic terms up to 16 and sums of 18,000 terms
     assert np.abs(got - ref).max() <= 1e-12 * np.abs(ref).max()
+
+
+# npw 4,193 and 9,163 (9 elements a thread): threes, twos and fours of rows, one
+# group and several, and the columns (129 up) that take the kernel with many
+# rows; 4 elements: rows in twos
+@pytest.mark.parametrize("cell, nr, nv, m", [(19.8, 54, 6, 1), (19.8, 54, 5, 3), (25.7, 72, 3, 2), (19.8, 54, 9, 129),
+                                             (25.7, 72, 32, 256), (25.7, 72, 30, 130), (19.8, 54, 10, 131),
+                                             (14.2, 45, 10, 2), (14.2, 45, 13, 3)])
+def test_projector_row_groups(gpu, cell, nr, nv, m):
+    gpu.profile(True)
+    try:
+        test_projector(gpu, cell, nr, nv, m)
+        assert gpu.profile_query("project")[1] == 1
+    finally:
+        gpu.profile(False)

@@ -755,26 +755,45 @@ bool project_pays(int nq, int m, int npw) {
   return cg_project_fits(nq, m, npw) && (npw <= 4 * NTU || nq <= 6 || m > 128);
 }
 
-// run(elements a thread, rows a group): groups of rows that leave none over, as
-// far as the registers go
+// Rows a group.  More of them share the reads of a column's elements and the
+// sums' exchanges; fewer leave registers and repeat fewer rows that are not there.
+// So: all of them where the registers allow (4 elements a thread: up to 7, except
+// that six go faster in threes; 9: up to 4); fours, or threes, that leave none
+// over; else fours unless more than an eighth (9 elements: a quarter) of their
+// loads were for nothing, then twos.  With 9 elements threes stop at nine rows.
+// A solve (cg_project), us, 128 columns, npw = 1,872 / 3,761: 7 rows at once 1,218 /
+// 2,037, in twos 1,239 / 2,060, in fours 1,253 / 2,043; 6 in threes 1,207 / 2,025, at
+// once 1,224 / 2,028; 10 in twos 1,293 / 2,084, in fours 1,317 / 2,095; 21 in threes
+// 1,427 / 2,270, in fours 1,465 / 2,302.  npw = 6,147 / 9,139: 9 in threes 2,591 / 3,609,
+// in fours 2,598 / 3,606 (one column 1,014 / 1,214 and 1,086 / 1,273); 24 in fours 3,009 /
+// 4,205, in threes 3,186 / 4,415; 31 in fours 3,296 / 4,558, in twos 3,462 / 4,750; 5 and
+// one column in twos 949 / 1,107, in fours 1,000 / 1,160.
+static int project_group(int nq, bool small) {
+  if (nq <= 4 || (small && (nq == 5 || nq == 7))) return std::max(nq, 1);
+  if (nq % 4 == 0) return 4;
+  if (nq % 3 == 0 && (small || nq <= 9)) return 3;
+  const int over = ceil_div(nq, 4) * 4 - nq;
+  return (small ? 8 : 4) * over > nq + over ? 2 : 4;
+}
+
+// run(elements a thread, rows a group)
 template <typename F>
 static void project_variant(int npw, int nq, F run) {
   using std::integral_constant;
-  const integral_constant<int, 4> e4;
-  const integral_constant<int, 9> e9;
-  if (npw <= 4 * NTU) {
-    if (nq <= 1) run(e4, integral_constant<int, 1>());
-    else if (nq == 2) run(e4, integral_constant<int, 2>());
-    else if (nq == 5) run(e4, integral_constant<int, 5>());
-    else if (nq == 7) run(e4, integral_constant<int, 7>());
-    else if (nq % 3 == 0) run(e4, integral_constant<int, 3>());
-    else run(e4, integral_constant<int, 4>());
-  } else {
-    if (nq <= 1) run(e9, integral_constant<int, 1>());
-    else if (nq == 2) run(e9, integral_constant<int, 2>());
-    else if (nq % 3 == 0) run(e9, integral_constant<int, 3>());
-    else run(e9, integral_constant<int, 4>());
-  }
+  const bool small = npw <= 4 * NTU;
+  const int rg = project_group(nq, small);
+  auto with = [&](auto e) {
+    if (rg == 1) run(e, integral_constant<int, 1>());
+    else if (rg == 2) run(e, integral_constant<int, 2>());
+    else if (rg == 3) run(e, integral_constant<int, 3>());
+    else if (rg == 4) run(e, integral_constant<int, 4>());
+    else if constexpr (decltype(e)::value == 4) {
+      if (rg == 5) run(e, integral_constant<int, 5>());
+      else run(e, integral_constant<int, 7>());
+    }
+  };
+  if (small) with(integral_constant<int, 4>());
+  else with(integral_constant<int, 9>());
 }
 
 void cg_project(int nc, int npw, int gstart, int nq, const int* l2i, const z64* q, const double* scale, z64* h, z64* g,
