@@ -95,3 +95,31 @@ def test_projector_row_groups(gpu, cell, nr, nv, m):
         assert gpu.profile_query("project")[1] == 1
     finally:
         gpu.profile(False)
+
+
+# either side of the rule that picks the CG's kernel: npw 1,536 (always), 4,193 (5
+# elements a thread: 8 columns beyond ten rows), 9,163 (9: 30 columns, 48 beyond 20 rows)
+@pytest.mark.parametrize("cell, nr, nv, m, kernel", [
+    (14.2, 45, 32, 1, True), (19.8, 54, 10, 1, True), (19.8, 54, 11, 7, False), (19.8, 54, 11, 8, True),
+    (25.7, 72, 10, 2, True), (25.7, 72, 20, 29, False), (25.7, 72, 20, 30, True), (25.7, 72, 21, 47, False),
+    (25.7, 72, 21, 48, True), (25.7, 72, 32, 3, False)])
+def test_solve_on_either_side_of_the_rule(gpu, cell, nr, nv, m, kernel):
+    from oracle.hamiltonian import apply_sternheimerop
+    gs = _state(cell, nr, nv, 0, 0, 3)
+    gpu.set_ground_state(gs)
+    rng = np.random.default_rng(m)
+    b = (rng.normal(size=(m, gs.npwx)) + 1j * rng.normal(size=(m, gs.npwx))) / (1.0 + gs.basis.g2kin)
+    b[:, 0] = b[:, 0].real
+    x = np.zeros_like(b)
+    e = -0.5 - rng.random(m)
+    gpu.profile(True)
+    try:
+        assert gpu.linsolve_sternheimer_m_wfcts(nv, m, b.copy(), x, e, np.full(m, 1.5), 1e-20) == 0
+        assert (gpu.profile_query("cg_project")[1] > 0) == kernel
+    finally:
+        gpu.profile(False)
+    # the first and the last column's residual r by the oracle's operator: <M^-1 r|r>
+    # < 1e-20 at the end, M <= 16/1.5, and roundings of sums of order ten
+    for i in {0, m - 1}:
+        r = apply_sternheimerop(gs, x[i:i + 1], e[i:i + 1], gs.alpha_pv) - b[i:i + 1]
+        assert 2.0 * np.sum(np.abs(r) ** 2) - np.abs(r[0, 0]) ** 2 <= 11e-20 + (1e-12) ** 2

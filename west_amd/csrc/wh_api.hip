@@ -334,7 +334,7 @@ int linsolve_dev(int m, z64* b, z64* x, const std::vector<double>& e_col, const 
   WH_TIMED("cg_prec", prec_rho(m, npw, c.gstart, d_l2i, g, ld, c.d_g2kin, d_eprec_col, d_rhob, s, true));
   const int nqp = c.l_kinetic_only ? c.nbndval : c.nbndval + c.nkb;
   // few projector rows: the operator's local part by band, then one kernel
-  const bool project = cg_project_fits(nqp, m, npw);
+  const bool project = cg_project_pays(nqp, m, npw);
   if (project) {
     // the first direction (beta = 0)
     WH_HIP(hipMemsetAsync(d_beta, 0, sizeof(double) * m, s));

@@ -77,9 +77,11 @@ void cg_select(int m, double tr2, int first, int group, const double* rhob, doub
 // again) for nq <= kCgProjRows projector rows, m <= 256 columns (one workgroup
 // a compute unit; with more, the matrix-core products share their reads of the
 // rows) and a band in the registers of 1,024 threads: projectors, update, rho
-// and the next direction in h.
+// and the next direction in h.  cg_project_pays: and a CG of m columns is faster
+// with it.
 constexpr int kCgProjRows = 32;
 bool cg_project_fits(int nq, int m, int npw);
+bool cg_project_pays(int nq, int m, int npw);
 // the projector part alone, t += Q s (Q^T x), same range; project_pays: and it is
 // the faster way there
 bool project_pays(int nq, int m, int npw);

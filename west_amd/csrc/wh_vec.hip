@@ -745,6 +745,24 @@ void cg_update(int nc, int npw, int gstart, const int* l2i, const z32* h, z32* g
 
 bool cg_project_fits(int nq, int m, int npw) { return nq <= kCgProjRows && m <= 256 && npw <= 9 * NTU; }
 
+// The CG with k_cg_project against the general iteration (a solve of some 20
+// iterations, ms).  Up to 4 elements a thread it wins throughout (npw = 3,761, 32
+// rows, 1 / 16 / 128 columns: 1.19 / 1.44 / 2.44 against 1.37 / 1.86 / 3.25).  With 9 the
+// one compute unit of a column goes through 2 x 9 x 16 kB of each row whatever npw
+// is, which many rows and few columns leave in the open (ours, general):
+//   npw, rows    1 column   8          16         32         64         128
+//   4,193, 28   1.40 1.36  1.58 1.60  1.65 1.82  1.71 1.93  2.08 2.43
+//   6,147, 16   1.18 1.15  1.37 1.38  1.50 1.57  1.74 1.86  2.04 2.31  2.73 3.21
+//   6,147, 32   1.62 1.38  1.86 1.83  2.00 2.00  2.24 2.30  2.55 2.80  3.27 3.99
+//   9,139, 10   1.21 1.21  1.50 1.48  1.61 1.64  1.95 2.04  2.39 2.59  3.62 4.25
+//   9,139, 16   1.43 1.28  1.72 1.62  1.85 1.80  2.18 2.23  2.63 2.83  3.85 4.78
+//   9,139, 32   2.15 1.54  2.47 2.12  2.65 2.38  2.96 2.84  3.35 3.54  4.57 5.89
+// so beyond ten rows it takes the more columns the more elements there are.
+bool cg_project_pays(int nq, int m, int npw) {
+  if (!cg_project_fits(nq, m, npw)) return false;
+  return npw <= 4 * NTU || nq <= 10 || m >= std::max(8, (ceil_div(npw, NTU) - 6) * (nq > 20 ? 16 : 10));
+}
+
 // k_project against the three products (a call, us; 1, 16, 256 columns): up to
 // 4 elements a thread it wins throughout (npw = 1,820: 8 rows 69 / 70 / 140 against
 // 92 / 92 / 175, 31 rows 86 / 88 / 161 against 102 / 104 / 213); with 9 the one
