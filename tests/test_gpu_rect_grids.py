@@ -61,3 +61,31 @@ def test_operator_and_response(nr, nbnd, nkb, m):
     got = wstat.dfpt(m, dv, -1.0)
     want = dfpt_ref(gs, dv, -1.0)
     assert np.abs(got - want)[:, :n].max() <= 1e-12 * np.abs(want).max()
+
+
+# n1 = n2 with another n3: every plane kernel that such a grid can take, the last
+# workgroup short of planes (n3 no multiple of 2, 3 or 4); the quad-lane kernels
+# at 60, 72 and 100, the LDS-pass kernel above 64, the density in two halves at 100
+# and 108 (its scratch by planes)
+@pytest.mark.parametrize("nr", [(54, 54, 25), (60, 60, 20), (60, 60, 25), (72, 72, 25), (80, 80, 18), (100, 100, 27),
+                                (108, 108, 20)])
+def test_square_planes(nr, monkeypatch):
+    from west_amd import wstat
+    gs = _ground_state(nr, 2, 1, seed=sum(nr))
+    n = gs.basis.npw
+    wstat.init(0)
+    rng = np.random.default_rng(6)
+    psi = np.zeros((3, gs.npwx), complex)
+    psi[:, :n] = rng.normal(size=(3, n)) + 1j * rng.normal(size=(3, n))
+    psi[:, 0] = psi[:, 0].real
+    e = rng.normal(size=3)
+    ref = apply_sternheimerop(gs, psi, e, gs.alpha_pv)
+    for variant in range(1, 10):   # LDS passes, register lines, quad lanes; beyond the last the last again
+        monkeypatch.setenv("WH_PLANE_OCC", str(variant))
+        wstat.set_ground_state(gs)
+        out = wstat.apply_sternheimerop_to_m_wfcs(2, psi, e, gs.alpha_pv)
+        assert np.abs(out - ref)[:, :n].max() <= 1e-12 * np.abs(ref).max(), variant
+    dv = psi / (1.0 + np.pad(gs.basis.g2kin, (0, gs.npwx - n)))
+    got = wstat.dfpt(3, dv, -1.0)
+    want = dfpt_ref(gs, dv, -1.0)
+    assert np.abs(got - want)[:, :n].max() <= 1e-12 * np.abs(want).max()
