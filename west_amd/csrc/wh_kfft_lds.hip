@@ -184,14 +184,16 @@ __global__ __launch_bounds__(KL_NT) void k_kvloc_lds(int n1, int n2, int n3, int
   }
 }
 
-// sum over the workgroup of nv values per thread (nv <= KL_NQ2); every
-// thread gets the sums in out[] (LDS)
 constexpr int KL_NQ2 = 32;   // projector rows (real view) the fused CG iteration takes
-__device__ __forceinline__ void kl_block_sums(double* v, int nv, double (*red)[KL_NT / 64], double* out) {
+
+// sums over the workgroup of nv <= MAXV values per thread; every thread gets
+// them in out[] (LDS)
+template <int NT, int MAXV>
+__device__ __forceinline__ void kl_sums(const double* v, int nv, double (*red)[NT / 64], double* out) {
   const int lane = threadIdx.x & 63;
   const int w = threadIdx.x >> 6;
 #pragma unroll
-  for (int i = 0; i < KL_NQ2; ++i) {
+  for (int i = 0; i < MAXV; ++i) {
     if (i < nv) {
       double x = v[i];
       for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
@@ -202,7 +204,7 @@ __device__ __forceinline__ void kl_block_sums(double* v, int nv, double (*red)[K
   if (threadIdx.x < nv) {
     double x = 0.0;
 #pragma unroll
-    for (int q = 0; q < KL_NT / 64; ++q) x += red[threadIdx.x][q];
+    for (int q = 0; q < NT / 64; ++q) x += red[threadIdx.x][q];
     out[threadIdx.x] = x;
   }
   __syncthreads();
@@ -290,28 +292,6 @@ __device__ __forceinline__ void kl_pass_rows(int n, z64* p, int rs, int imax, co
 #undef WH_KL_CASE
     default: break;
   }
-}
-
-template <int NT, int MAXV>
-__device__ __forceinline__ void kl_sums(const double* v, int nv, double (*red)[NT / 64], double* out) {
-  const int lane = threadIdx.x & 63;
-  const int w = threadIdx.x >> 6;
-#pragma unroll
-  for (int i = 0; i < MAXV; ++i) {
-    if (i < nv) {
-      double x = v[i];
-      for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
-      if (lane == 0) red[i][w] = x;
-    }
-  }
-  __syncthreads();
-  if (threadIdx.x < nv) {
-    double x = 0.0;
-#pragma unroll
-    for (int q = 0; q < NT / 64; ++q) x += red[threadIdx.x][q];
-    out[threadIdx.x] = x;
-  }
-  __syncthreads();
 }
 
 constexpr int KR_NT = 256;
@@ -515,7 +495,7 @@ __global__ __launch_bounds__(KL_NT) void k_pc_precond(int nb, int cols, long ld,
     for (int i = 0; i < KL_NQ2; ++i)
       if (i < nr) acc[i] += pk.q2[i * ldr + 2 * ig] * fv.x + pk.q2[i * ldr + 2 * ig + 1] * fv.y;
   }
-  kl_block_sums(acc, nr, red, sums);
+  kl_sums<KL_NT, KL_NQ2>(acc, nr, red, sums);
   for (int ig = tid; ig < ld; ig += KL_NT) {
     if (ig >= pk.npw) {
       xc[ig] = mk(0.0, 0.0);
