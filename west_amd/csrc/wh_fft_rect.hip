@@ -8,10 +8,12 @@
 // padding, V(r) and the row selection are folded into the passes, and the
 // inverse and forward a1 transforms meet in registers.
 //
-// What bounds it: LDS passes and their barriers, as for k_plane_vloc_t.
+// What bounds it: instruction issue between barriers.  On 40 x 54 x 96 the
+// vector ALUs are busy 58 % and the LDS 39 % of the cycles (27 % of those in bank
+// conflicts), with 14 of 16 waves a CU resident and 0.8 TB/s of HBM traffic.
 //  * Consecutive lanes take consecutive lines (not consecutive points): rows
-//    and lines have odd strides of 16-byte elements, so every LDS access of
-//    a pass is free of bank conflicts, and the twiddles of a butterfly are the
+//    and lines have odd strides of 16-byte elements, so neighbouring lanes of a
+//    pass fall on other banks, and the twiddles of a butterfly are the
 //    same for a whole line set (broadcast reads).  The potential must then be
 //    contiguous along a2: real-space arrays of these plans are [a3][a1][a2].
 //  * A pass is one butterfly per thread, staged in registers where it stores

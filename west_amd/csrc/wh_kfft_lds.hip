@@ -226,11 +226,12 @@ __device__ __forceinline__ void kl_sums(const double* v, int nv, double (*red)[N
 // a3 lines of the columns that hold points, the a2 lines of the rows, and
 // the a1 lines -- zero-padded from the rows in registers, V(r) between their
 // inverse and forward transforms -- are one line per thread each, so five
-// passes and as many barriers make the local term.  Bound by FP64 issue and
-// the passes' latency: 864 columns of that grid take 62 us an iteration (with
-// the whole grid in LDS, every line transformed, one workgroup a CU: 145; with
-// the columns' sticks in LDS and the planes in batches through two-radix
-// passes, 85 barriers: 138).  256 threads may use 256 registers each, which a
+// passes and as many barriers make the local term.  Bound by the passes' latency
+// with eight waves a CU (over a solve the vector ALUs are busy 20 % and the LDS
+// 16 % of the cycles, 1.4 TB/s of HBM traffic): 864 columns of that grid take 62 us
+// an iteration (with the whole grid in LDS, every line transformed, one
+// workgroup a CU: 145; with the columns' sticks in LDS and the planes in
+// batches through two-radix passes, 85 barriers: 138).  256 threads may use 256 registers each, which a
 // 24-point line with V(r) needs; 320 and 384 threads spill (chi0 of that case
 // 2.3 ms against 3.3 and 3.9).
 // FIRST: the CG's first step instead (127-205), every launched column in
@@ -244,7 +245,9 @@ struct KlRows {
 // widest |i| the a1 lines take: where the grid holds the products of two
 // functions the sphere spans at most (n + 1) / 4 either way, and the k point
 // less than one more.  WIDE: any sphere of the grid, every element may come
-// from a row.
+// from a row (dfpt at q, 8 k points, 4 bands, 32 perturbations, |i| <= 9 on 24 x 20
+// x 18 and 20 x 16 x 15: 2.00 and 1.38 ms; the operator in five launches an
+// iteration 4.72 and 4.14; the whole grid in LDS 2.36 and 1.99).
 constexpr int kl_row_bound(int n, bool wide) { return wide ? n / 2 : n / 4 + 1; }
 
 // a1 line from and to the rows: v(x) at p[(x or x - n1) rs], |x| <= imax

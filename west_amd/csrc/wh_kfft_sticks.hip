@@ -7,7 +7,8 @@
 // 25 Ry) has 2,300 points in 300 columns, so a band moves 0.17 MB of sticks
 // four times where full-grid transforms moved 0.75 MB fourteen times.
 //
-// Bound by memory (the sticks).  A workgroup takes CW columns: lane -> column,
+// Bound by memory (3.7 TB/s inverse, 4.4 forward, of the 4.4 that a large copy
+// reaches).  A workgroup takes CW columns: lane -> column,
 // so the sticks are read and written in runs of 16 CW bytes and the first
 // (zfwd) and last (zinv) pass touch global memory directly; LDS holds the
 // lines between the two passes and the sphere side.

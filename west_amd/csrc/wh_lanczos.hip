@@ -78,6 +78,7 @@ __global__ void k_lan_scale(int npw, const z64* r, const double* beta, z64* q, l
 // call on that case: one launch per vector with r in memory 27.2 ms (13.0 of
 // it in those), <18, 4> 14.4, <18, 8> 15.1 and <18, 18> 17.6 (registers spill),
 // each vector read twice instead of held 14.5, 1,024 threads 15.0 to 18.6.
+// Bound by those reads: 310 MB a launch on average at 4.0 TB/s.
 // Spheres beyond 18,432 points keep r in memory (k_lan_step_mem).
 constexpr int LNT = 512;
 

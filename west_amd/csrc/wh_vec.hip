@@ -238,11 +238,12 @@ __device__ __forceinline__ double uniform(double v) {
 // M^-1 g in registers.  <h|Q s Q^T h> is the sum of s_i (Q_i^T h)^2, so t is complete
 // only in the second pass and never stored.  (kCgProjRows rows: their two
 // passes come from the L2 and cost 2 npw rows 16 bytes a band.)
-// Bound: one compute unit's load path (64 bytes a cycle; the rows twice and
-// nine passes of the vectors) and three block-wide sums.  Before, the same work
-// was the products' three launches, the update and the direction: 35 bands, 7
-// rows, npw = 3,761: 12.2 + 4.3 + 4.5 + 8.9 + 4.1 -> 18 us; 192 bands, 6 rows,
-// npw = 6,147: 10.3 + 4.9 + 7.5 + 16.7 + 8.5 -> 31 us; and four gaps less.
+// Bound: what one compute unit loads (the rows twice and nine passes of the
+// vectors: 27 to 31 of its 64 bytes a cycle) around three block-wide sums; the
+// vector ALUs are busy 3 to 8 % of the cycles.  Before, the same work was the
+// products' three launches, the update and the direction: 35 bands, 7 rows,
+// npw = 3,761: 12.2 + 4.3 + 4.5 + 8.9 + 4.1 -> 18 us; 192 bands, 6 rows, npw =
+// 6,147: 10.3 + 4.9 + 7.5 + 16.7 + 8.5 -> 31 us; and four gaps less.
 // Rows in groups of RG; beyond nq the last one is repeated and not used.
 template <int E, int RG>
 __global__ __launch_bounds__(NTU) void k_cg_project(unsigned npw, int gstart, int nq, const int* l2i, const z64* q,
